@@ -16,7 +16,10 @@ Two entry points:
   kernels; the only device-to-host copy per round is (n_accepted, out_tokens).
 """
 
+import gc
+import threading
 from collections import OrderedDict
+from contextlib import contextmanager
 from typing import List, Optional, Sequence, Tuple
 
 import numpy as np
@@ -368,6 +371,30 @@ def _graph_key(model) -> tuple:
 
 _MAX_GRAPHS = 8
 
+_captures = {"lock": threading.Lock(), "open": 0, "collector": False}
+
+
+@contextmanager
+def _capturing(ctx):
+    """ctx (torch.cuda.graph) entered with Python's cyclic garbage collector off. A collection inside a
+    capture runs the destructors of whatever garbage it finds; a dead HIP graph among it (an engine or
+    batch caught in a reference cycle holds its pool's) waits for the device as it goes, which a
+    capturing stream refuses, and an error in a destructor ends the process. Captures may nest or run
+    on several threads: the collector comes back with the last of them, if it was on."""
+    with _captures["lock"]:
+        if _captures["open"] == 0:
+            _captures["collector"] = gc.isenabled()
+            gc.disable()
+        _captures["open"] += 1
+    try:
+        with ctx:
+            yield
+    finally:
+        with _captures["lock"]:
+            _captures["open"] -= 1
+            if _captures["open"] == 0 and _captures["collector"]:
+                gc.enable()
+
 
 def _round_state(target, draft, pool_t: PagedKVPool, pool_d: PagedKVPool, b: int, k: int, blocks_t, blocks_d,
                  sampling: bool, keyed: bool = False) -> "_RoundState":
@@ -438,7 +465,7 @@ def _launch_round(target, draft, pool_t, pool_d, st: "_RoundState", b: int, draw
         if st.graph is None:   # the whole round in one graph: no launch gap between its phases
             torch.cuda.current_stream().synchronize()
             g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g):
+            with _capturing(torch.cuda.graph(g)):
                 kernels()
             st.graph = g
         st.graph.replay()
@@ -454,7 +481,7 @@ def capture_phase_graphs(target, draft, pool_t, pool_d, st: "_RoundState") -> li
         gs = []
         for phase in range(st.k + 1):
             g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g):
+            with _capturing(torch.cuda.graph(g)):
                 _round_phase(target, draft, pool_t, pool_d, st, phase)
             gs.append(g)
         st.phase_graphs = gs

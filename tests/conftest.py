@@ -1,3 +1,4 @@
+import gc
 import os
 import sys
 
@@ -28,6 +29,14 @@ def pytest_collection_modifyitems(config, items):
 @pytest.fixture(autouse=True)
 def _seed():
     torch.manual_seed(0)
+
+
+@pytest.fixture(autouse=True, scope="module")
+def _no_garbage_between_modules():
+    """A module's cyclic garbage (engines that hold HIP graphs) goes before the next module's tests, which
+    capture graphs of their own: destroying a graph inside a capture ends the process."""
+    yield
+    gc.collect()
 
 
 def pytest_terminal_summary(terminalreporter):

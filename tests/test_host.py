@@ -68,3 +68,73 @@ def test_pool_key_layouts():
     with pytest.raises(ValueError):
         PagedKVPool(ModelConfig(vocab_size=32, d_model=48, n_layers=1, n_heads=4, n_kv_heads=2, max_seq_len=16), 4,
                     device="cpu", key_layout="groups")
+
+
+def test_captures_run_without_the_garbage_collector():
+    """Garbage in a reference cycle (as an engine whose method a caller replaced by a closure over it) is
+    not collected while a capture is open, whatever the capture's Python allocates; the collector is back
+    afterwards, also after nested captures, captures on several threads and an error, and stays off for
+    a caller that had it off."""
+    import contextlib
+    import gc
+    import threading
+
+    from forgeserve_amd.speculative import _capturing
+
+    died = []
+
+    class Holder:
+        def step(self):
+            pass
+
+        def __del__(self):
+            died.append(True)
+
+    def garbage():
+        h = Holder()
+        inner = h.step
+        h.step = lambda: inner()   # h -> closure -> bound method -> h
+
+    assert gc.isenabled()
+    gc.collect()
+    garbage()
+    with _capturing(contextlib.nullcontext()):
+        with _capturing(contextlib.nullcontext()):
+            keep = [[i] for i in range(200_000)]
+        keep += [[i] for i in range(200_000)]
+        assert not died and not gc.isenabled()
+    assert gc.isenabled()
+    gc.collect()
+    assert died and len(keep) == 400_000
+
+    try:
+        with _capturing(contextlib.nullcontext()):
+            raise KeyError
+    except KeyError:
+        pass
+    assert gc.isenabled()
+
+    first, second = threading.Event(), threading.Event()
+
+    def other():
+        with _capturing(contextlib.nullcontext()):
+            first.set()
+            second.wait(10)
+
+    t = threading.Thread(target=other)
+    t.start()
+    first.wait(10)
+    with _capturing(contextlib.nullcontext()):
+        pass
+    assert not gc.isenabled()   # the other thread's capture is still open
+    second.set()
+    t.join()
+    assert gc.isenabled()
+
+    gc.disable()
+    try:
+        with _capturing(contextlib.nullcontext()):
+            pass
+        assert not gc.isenabled()
+    finally:
+        gc.enable()
