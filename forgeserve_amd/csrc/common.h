@@ -146,6 +146,10 @@ namespace fs {
 void set_error(const char* fmt, ...);
 int arg_error(const char* fmt, ...);           // sets the message, returns FS_ERR_ARG
 int launch_status(const char* what);           // hipGetLastError after a launch -> 0 or >0
+// float32 projections on the matrix cores (gemm_f32.hip): whether the operands allow it, and the launch
+bool gemm_f32_ok(const void* A, int64_t lda, const void* B, int64_t ldb, int64_t K);
+void gemm_f32(const float* A, int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc, const float* R,
+              int64_t ldr, int64_t M, int64_t N, int64_t K, hipStream_t s);
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 }  // namespace fs
 

@@ -5,7 +5,8 @@
 // Every output element accumulates its K products in increasing k, 32 at a time, in one MFMA
 // accumulator, whatever the tile shape or M: a row's result does not depend on the batch it is in
 // (the draft step, the verify pass and prefill give identical rows for identical inputs).
-// f32 (and unaligned bf16) path: LDS-tiled VALU kernel, one fmaf chain per output in increasing k.
+// f32 path: matrix cores too (gemm_f32.hip). f16 and unaligned operands: LDS-tiled VALU kernel, one fmaf
+// chain per output in increasing k.
 #include "common.h"
 
 namespace {
@@ -471,7 +472,7 @@ __global__ void __launch_bounds__(256) gemm_splitk_reduce_kernel(const float* __
 }
 
 // ------------------------------------------------------------------------------------------------
-// VALU kernel (f32 / f16 / unaligned bf16): 64x64 tile, 16-deep k stages, 4x4 outputs per thread
+// VALU kernel (f16, and f32 / bf16 with unaligned rows): 64x64 tile, 16-deep k stages, 4x4 outputs per thread
 // ------------------------------------------------------------------------------------------------
 template <int DT>
 __global__ void __launch_bounds__(256) gemm_valu_kernel(const typename Elem<DT>::T* __restrict__ A, int64_t lda,
@@ -767,6 +768,10 @@ extern "C" int fs_gemm(const void* A, int64_t lda, const void* B, int64_t ldb, v
                                                                          (const uint16_t*)R, ldr, M, N, K, tn);
     }
     return fs::launch_status("gemm_bf16");
+  }
+  if (dtype == FS_F32 && fs::gemm_f32_ok(A, lda, B, ldb, K)) {
+    fs::gemm_f32((const float*)A, lda, (const float*)B, ldb, (float*)C, ldc, (const float*)R, ldr, M, N, K, s);
+    return fs::launch_status("gemm_f32");
   }
   const int tm = (int)((M + 63) / 64), tn = (int)((N + 63) / 64);
   dim3 grid((unsigned)(tm * tn));

@@ -61,6 +61,23 @@ def test_gemm_rows_do_not_depend_on_the_batch(dtype, n, k):
     assert torch.equal(ops.gemm(a[100:107], w), full[100:107])
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 1, 4), (1, 5, 12), (3, 17, 28), (15, 16, 32), (17, 33, 36), (33, 130, 260),
+                                   (65, 1376, 688), (640, 257, 688), (129, 4100, 100), (2100, 2052, 144)])
+def test_gemm_f32_tiles(m, n, k):
+    """float32 projections on the matrix cores at the edges of their tiles, K chunks and 16-k steps, with a
+    residual: against float64, and each row's bits the same alone, in a short batch and in the whole one
+    (the three tile shapes). Tolerance: k products and sums of at most one float32 rounding each."""
+    case("gemm f32", m, n, k)
+    g = torch.Generator().manual_seed(m + n + k)
+    a, w, r = torch.randn(m, k, generator=g), torch.randn(n, k, generator=g), torch.randn(m, n, generator=g)
+    ad, wd, rd = a.to(DEV), w.to(DEV), r.to(DEV)
+    got = ops.gemm(ad, wd, residual=rd)
+    bound = (k + 1) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T + r.double().abs())
+    assert ((got.cpu().double() - (a.double() @ w.double().T + r.double())).abs() <= bound).all()
+    for lo, hi in ((0, 1), (m - 1, m), (0, min(m, 40))):
+        assert torch.equal(ops.gemm(ad[lo:hi], wd, residual=rd[lo:hi]), got[lo:hi]), (lo, hi)
+
+
 @pytest.mark.parametrize("n,k", [(128, 256), (4096, 1024)])   # (4096, 1024) splits K
 def test_gemm_residual_epilogue(n, k):
     case("gemm residual", n, k)
