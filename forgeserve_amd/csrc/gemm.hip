@@ -175,6 +175,57 @@ struct RowStatsOut {
   int64_t nparts, ld;
 };
 
+// Four finished columns C[row][col0 .. col0 + 3] of a tile. SWIGLU: silu(gate) * up of the two (gate, up)
+// column pairs. part: the f32 partial of this k-range instead, for whatever adds the splits in order. Else
+// rounded, plus the residual, rounded again.
+template <bool SWIGLU>
+FS_DEVICE void store4(float4_t a, int64_t row, int64_t col0, uint16_t* C, int64_t ldc, const uint16_t* R, int64_t ldr,
+                      int64_t M, int64_t N, float* part, int split) {
+  typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2;
+  if (row >= M) return;
+  if (SWIGLU) {   // (no split, no residual on this path; N % 4 == 0)
+    if (col0 >= N) return;
+    float v[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = Elem<FS_BF16>::round(a[r]);
+    const uint32_t h0 = f32_to_bf16(silu_times<FS_BF16>(v[0], v[1]));
+    const uint32_t h1 = f32_to_bf16(silu_times<FS_BF16>(v[2], v[3]));
+    *reinterpret_cast<uint32_t*>(C + row * ldc + col0 / 2) = h0 | (h1 << 16);
+    return;
+  }
+  if (part) {   // (N % 4 == 0)
+    if (col0 < N) *reinterpret_cast<float4_t*>(part + ((int64_t)split * M + row) * N + col0) = a;
+    return;
+  }
+  uint16_t o[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    float v = Elem<FS_BF16>::round(a[r]);
+    if (R && col0 + r < N) v = v + bf16_to_f32(R[row * ldr + col0 + r]);
+    o[r] = f32_to_bf16(v);
+  }
+  if (col0 + 3 < N && ((ldc | col0) & 3) == 0) {
+    *reinterpret_cast<u32x2*>(C + row * ldc + col0) =
+        u32x2{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (col0 + r < N) C[row * ldc + col0 + r] = o[r];
+  }
+}
+
+// A wave's finished tile of 16x16 MFMAs: acc[i][j] holds, in lane (l16, g), C[row0 + 16i + l16][col0 + 16j + 4g + r].
+template <int TM, int TN, bool SWIGLU>
+FS_DEVICE void gemm_store(const float4_t (&acc)[TM][TN], int64_t wrow0, int64_t wcol0, uint16_t* C, int64_t ldc,
+                          const uint16_t* R, int64_t ldr, int64_t M, int64_t N, float* part, int split) {
+  const int l16 = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      store4<SWIGLU>(acc[i][j], wrow0 + 16 * i + l16, wcol0 + 16 * j + 4 * g, C, ldc, R, ldr, M, N, part, split);
+}
+
 // SWIGLU: W holds [gate; up] (N/2 rows each) and the tile's output columns are interleaved, column
 // 2j = gate row j and 2j + 1 = up row j, so that each lane's four consecutive columns are two (gate, up)
 // pairs; the epilogue stores silu(gate) * up to C[row][j] (model.py:93) instead of the products.
@@ -329,64 +380,8 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_bf16_lds_kernel(const uin
       for (int j = 0; j < TN; ++j) acc[i][j] = sum[i][j];
   }
 
-  // acc[i][j]: lane (l16, g) holds C[m = 16i + l16][n = 16j + 4g + r], r = 0..3 (wave-local)
-  if (SWIGLU) {   // (no split, no residual on this path; N % 4 == 0)
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int64_t row = m0 + wm * WM + 16 * i + l16;
-      if (row >= M) continue;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int64_t col0 = n0 + wn * WN + 16 * j + 4 * g;
-        if (col0 >= N) continue;
-        float v[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = Elem<FS_BF16>::round(acc[i][j][r]);
-        const uint32_t h0 = f32_to_bf16(silu_times<FS_BF16>(v[0], v[1]));
-        const uint32_t h1 = f32_to_bf16(silu_times<FS_BF16>(v[2], v[3]));
-        *reinterpret_cast<uint32_t*>(C + row * ldc + col0 / 2) = h0 | (h1 << 16);
-      }
-    }
-    return;
-  }
-  if (part) {   // split-K: f32 partial of this k-range, summed in split order by gemm_splitk_reduce_kernel
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int64_t row = m0 + wm * WM + 16 * i + l16;
-      if (row >= M) continue;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int64_t col0 = n0 + wn * WN + 16 * j + 4 * g;   // N % 4 == 0 on this path
-        if (col0 < N) *reinterpret_cast<float4_t*>(part + ((int64_t)split * M + row) * N + col0) = acc[i][j];
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int64_t row = m0 + wm * WM + 16 * i + l16;
-    if (row >= M) continue;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int64_t col0 = n0 + wn * WN + 16 * j + 4 * g;
-      uint16_t o[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float v = Elem<FS_BF16>::round(acc[i][j][r]);
-        if (R && col0 + r < N) v = v + bf16_to_f32(R[row * ldr + col0 + r]);
-        o[r] = f32_to_bf16(v);
-      }
-      if (col0 + 3 < N && ((ldc | col0) & 3) == 0) {
-        typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2;
-        *reinterpret_cast<u32x2*>(C + row * ldc + col0) =
-            u32x2{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (col0 + r < N) C[row * ldc + col0 + r] = o[r];
-      }
-    }
-  }
+  gemm_store<TM, TN, SWIGLU>(acc, m0 + wm * WM, n0 + wn * WN, C, ldc, R, ldr, M, N, part, split);
+  if (part) return;
   if (STATS) {   // (no residual on this path: the statistics are of the rounded products)
     constexpr float L2E = 1.4426950408889634f;
     const int64_t p = (n0 + wn * WN) / WN;
@@ -433,6 +428,293 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_bf16_lds_kernel(const uin
       se += __shfl_xor(se, 16, 64);   // (g0 + g1) + (g2 + g3) in every lane
       se += __shfl_xor(se, 32, 64);
       if (g == 0 && row < M && p < rs.nparts) rs.stats[row * rs.ld + p] = SoftmaxStat{ym, ym == -INFINITY ? 0.f : se, av, ai};
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// bf16 MFMA kernel for long batches: 256 x 256 tiles, 8 waves of 128 x 64 in two alternating groups
+//
+// Bound: the matrix cores. A CU's 64-deep stage of this tile is 2048 cycles of MFMA per SIMD against 192 KB
+// of operand reads (1536 cycles) and 64 KB of copies (512) on its LDS port, so the three have to overlap all
+// the time. Each stage is four phases of 16 MFMAs, one 64 x 32 quadrant of the wave's tile each, and the
+// quadrants go around so that each phase needs one new operand: X0 (rows 0-63) with the stage's first W
+// quarter, X0 with the second, X1 (rows 64-127) with the second, X1 with the first. The first quarter is W0
+// (columns 0-31) in even stages and W1 in odd ones, so the next stage's first quarter can be read while this
+// one's is still in use: 8, 4, 8 and 4 operand reads a phase. A phase reads its operand and issues two of the
+// wave's eight copies in its first half, and multiplies in its second. Waves w and w + 4 share a SIMD;
+// waves 4..7 run one barrier (half a phase) behind waves 0..3, so that on each SIMD one wave multiplies while
+// the other reads and copies. Two stages live in LDS; a quarter of a stage is overwritten once both groups
+// have read it, so copies are issued five phases before they are read, with eight per wave in flight.
+//
+//   phase of stage kt     reads                    copies                    waits for its copies of
+//   0                     X0                       W second of kt + 1        W second of kt
+//   1                     W second                 X1 of kt + 1              X1 of kt
+//   2                     X1                       W first of kt + 2         W first of kt + 1
+//   3                     W first of kt + 1        X0 of kt + 2              X0 of kt + 1
+// In halves from the stage's start (the second group one later): X0 is read in half 0 and used up by the end
+// of half 1 (1, 2), as is the W quarter read in half -2 (-1); second W read in 2 (3), done by 3 (4); X1 read
+// in 4 (5), done by 5 (6). Their next copies start in halves 6, 4, 8 and 10. A wave's wait comes before the
+// barrier that ends its phase's first half and leaves its eight youngest copies (fewer at the product's
+// end), so what the next phase reads has landed for every wave: the first group reads one half after the
+// second group's wait.
+// Same MFMA, operand roles and k order as the kernels above: the same bits.
+//
+// Measured on one box against the 8-wave ring kernel this replaces (one barrier per stage, every wave reading
+// then multiplying): gate|up at M = 8005 1.74 -> 1.43 ms (1.08 -> 1.32 PFLOP/s), at 32768 7.01 -> 5.68 ms, down
+// at 8005 1.00 -> 0.84 ms with its reduction. Without the copies the loop runs at 1.60 PFLOP/s, without the
+// operand reads at 1.62, with neither at 1.80: the LDS port is what is left. Not faster: 4 waves of 128 x 128
+// on v_mfma_f32_32x32x16 with a 5-slot ring of 32-deep stages (1.0 PFLOP/s; its 64-byte copies alone cost a
+// quarter, and one wave per SIMD issues at most 1.46), and this loop on 32x32x16 MFMAs (two independent
+// accumulators a quadrant: 1.26).
+// ------------------------------------------------------------------------------------------------
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+// dma16 from a wave-uniform base and a 32-bit byte offset per lane
+FS_DEVICE void dma16_at(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
+typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2;
+
+enum Mode { PLAIN, GATED, PARTIAL };   // what becomes of a tile: stored, its (gate, up) pairs gated, or kept in f32
+
+template <int MODE>
+__global__ void __launch_bounds__(512, 2) gemm_bf16_long_kernel(const uint16_t* __restrict__ X, int64_t ldx,
+                                                              const uint16_t* __restrict__ W, int64_t ldw,
+                                                              uint16_t* __restrict__ C, int64_t ldc,
+                                                              const uint16_t* __restrict__ R, int64_t ldr, int64_t M,
+                                                              int64_t N, int64_t K, int tiles_m, int ntiles,
+                                                              float* __restrict__ part) {
+  constexpr int BUF = 256 * 128;   // one operand's stage: 256 rows of 128 bytes (64 k)
+  constexpr int SMEM = 8 * 128 * 144;   // X stages 0, 1, then W stages 0, 1; at the end the rounded results
+  static_assert(SMEM >= 4 * BUF, "the ring fits");
+  __shared__ __attribute__((aligned(1024))) char smem[SMEM];
+
+  // tile order: as in gemm_bf16_lds_kernel
+  const int per_xcd = (ntiles + 7) / 8;
+  const int tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+  if (tile >= ntiles) return;
+  const int tiles_n = ntiles / tiles_m;
+  const int grp = tile / (8 * tiles_n), first = 8 * grp, gm = min(tiles_m - first, 8);
+  const int in_grp = tile - grp * 8 * tiles_n;
+  const int64_t m0 = (int64_t)(first + in_grp % gm) * 256;
+  const int64_t n0 = (int64_t)(in_grp / gm) * 256;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const int wm = wave >> 2, wn = wave & 3;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
+
+  // Copies: 8 rows of 128 bytes each; lane l takes row l >> 3, physical chunk l & 7 of it, which holds
+  // logical chunk (l & 7) ^ (row & 7). Quarter q of X: rows 64 q + 8 wave (+ 128); of W: rows
+  // 64 (wave >> 2) + 32 q + 8 (wave & 3) (+ 128).
+  const int cr = lane >> 3, cc = (lane & 7) ^ cr;
+  uint32_t xo[2][2], wo[2][2];
+  const int xrow = 8 * wave, wrow = 64 * (wave >> 2) + 8 * (wave & 3);
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int64_t xr = min(m0 + xrow + 64 * q + 128 * h + cr, M - 1) - m0;
+      xo[q][h] = (uint32_t)(2 * (xr * ldx + 8 * cc));
+      int64_t wr = min(n0 + wrow + 32 * q + 128 * h + cr, N - 1);
+      if (MODE == GATED) wr = (wr & 1) ? N / 2 + (wr >> 1) : (wr >> 1);   // interleaved column -> weight row
+      wo[q][h] = (uint32_t)(2 * ((MODE == GATED ? wr : wr - n0) * ldw + 8 * cc));
+    }
+  const int split = blockIdx.y;
+  const int nk = (int)(K / 64) / (int)gridDim.y;
+  const char* xb = reinterpret_cast<const char*>(X + m0 * ldx + (int64_t)split * nk * 64);
+  const char* wb = reinterpret_cast<const char*>(W + (MODE == GATED ? 0 : n0 * ldw) + (int64_t)split * nk * 64);
+  auto copy_x = [&](int q, int kt, int buf) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      dma16_at(xb + (int64_t)kt * 128, xo[q][h], lds0 + (uint32_t)(buf * BUF + (xrow + 64 * q + 128 * h) * 128));
+  };
+  auto copy_w = [&](int q, int kt, int buf) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      dma16_at(wb + (int64_t)kt * 128, wo[q][h], lds0 + (uint32_t)((2 + buf) * BUF + (wrow + 32 * q + 128 * h) * 128));
+  };
+
+  typedef __attribute__((address_space(3))) const bf16x8_t LdsFrag;
+  uint32_t xl[2], wl[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    const uint32_t c = 16 * ((4 * ks + g) ^ (l16 & 7));
+    xl[ks] = lds0 + (uint32_t)((wm * 128 + l16) * 128) + c;
+    wl[ks] = lds0 + 2 * BUF + (uint32_t)((wn * 64 + l16) * 128) + c;
+  }
+
+  float4_t acc[8][4];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+  bf16x8_t xf[4][2], w0[2][2], w1[2][2];
+
+  auto read_x = [&](int q, int buf) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) xf[i][ks] = *(LdsFrag*)(uintptr_t)(xl[ks] + (uint32_t)(buf * BUF + q * 64 * 128 + i * 16 * 128));
+  };
+  auto read_w = [&](bf16x8_t (&wf)[2][2], int q, int buf) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) wf[j][ks] = *(LdsFrag*)(uintptr_t)(wl[ks] + (uint32_t)(buf * BUF + q * 32 * 128 + j * 16 * 128));
+  };
+  auto barrier = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // one phase's second half: 16 MFMAs, each as its operands arrive
+  auto mul = [&](int qm, int qn, const bf16x8_t (&wf)[2][2]) {
+    barrier();
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[4 * qm + i][2 * qn + j] =
+              __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][ks], xf[i][ks], acc[4 * qm + i][2 * qn + j], 0, 0, 0);
+    __builtin_amdgcn_s_setprio(0);
+    barrier();
+  };
+  // buf = kt & 1, a constant at each call: the stage starts with W's quarter buf, and ends reading the next's
+  auto stage = [&](int kt, int buf) {
+    bf16x8_t (&wfirst)[2][2] = buf ? w1 : w0;
+    bf16x8_t (&wsecond)[2][2] = buf ? w0 : w1;
+    const bool next = kt + 1 < nk, next2 = kt + 2 < nk;
+    read_x(0, buf);
+    if (next) {
+      copy_w(buf, kt + 1, buf ^ 1);   // the next stage's second quarter is this stage's first
+      wait_vm<8>();
+    } else {
+      wait_vm<2>();
+    }
+    mul(0, buf, wfirst);
+    read_w(wsecond, buf ^ 1, buf);
+    if (next) {
+      copy_x(1, kt + 1, buf ^ 1);
+      wait_vm<8>();
+    } else {
+      wait_vm<0>();
+    }
+    mul(0, buf ^ 1, wsecond);
+    read_x(1, buf);
+    if (next2) {
+      copy_w(buf, kt + 2, buf);
+      wait_vm<8>();
+    } else if (next) {
+      wait_vm<6>();
+    }
+    mul(1, buf ^ 1, wsecond);
+    if (next) read_w(wsecond, buf ^ 1, buf ^ 1);
+    if (next2) {
+      copy_x(0, kt + 2, buf);
+      wait_vm<8>();
+    } else if (next) {
+      wait_vm<4>();
+    }
+    mul(1, buf, wfirst);
+  };
+
+  copy_w(0, 0, 0);
+  copy_x(0, 0, 0);
+  copy_w(1, 0, 0);
+  copy_x(1, 0, 0);
+  if (nk > 1) {
+    copy_w(1, 1, 1);
+    copy_x(0, 1, 1);
+    wait_vm<8>();
+  } else {
+    wait_vm<4>();
+  }
+  barrier();
+  if (wm) barrier();   // the second group runs one barrier behind
+  read_w(w0, 0, 0);
+  for (int kt = 0; kt < nk; kt += 2) {
+    stage(kt, 0);
+    if (kt + 1 < nk) stage(kt + 1, 1);
+  }
+  if (!wm) barrier();
+
+  // acc[i][j]: lane (l16, g) holds C[16i + l16][16j + 4g + r]
+  if (MODE == PARTIAL) {   // the f32 partial of this k-range (N % 4 == 0)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int64_t row = m0 + wm * 128 + 16 * i + l16;
+      float* prow = part + ((int64_t)split * M + row) * N;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int64_t col0 = n0 + wn * 64 + 16 * j + 4 * g;
+        if (row < M && col0 < N) *reinterpret_cast<float4_t*>(prow + col0) = acc[i][j];
+      }
+    }
+    return;
+  }
+  // The wave's rounded results (or gated pairs) to LDS, then out by whole rows, 16 bytes a lane (straight from
+  // the accumulators a store's lanes cover 16 rows of 32 bytes). Every copy has landed and, past this barrier,
+  // every wave has read its last operands: the ring's space is free.
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  constexpr int COLS = MODE == GATED ? 32 : 64, PITCH = COLS * 2 + 16, CH = COLS / 8;
+  static_assert(8 * 128 * PITCH <= SMEM, "the results fit");
+  char* out = smem + wave * 128 * PITCH;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      char* at = out + (16 * i + l16) * PITCH;
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = Elem<FS_BF16>::round(acc[i][j][r]);
+      if (MODE == GATED) {
+        const uint32_t h0 = f32_to_bf16(silu_times<FS_BF16>(v[0], v[1]));
+        const uint32_t h1 = f32_to_bf16(silu_times<FS_BF16>(v[2], v[3]));
+        *reinterpret_cast<uint32_t*>(at + 16 * j + 4 * g) = h0 | (h1 << 16);
+      } else {
+        u32x2 o;
+        o[0] = (__float_as_uint(v[0]) >> 16) | (__float_as_uint(v[1]) & 0xffff0000u);
+        o[1] = (__float_as_uint(v[2]) >> 16) | (__float_as_uint(v[3]) & 0xffff0000u);
+        *reinterpret_cast<u32x2*>(at + 2 * (16 * j + 4 * g)) = o;
+      }
+    }
+  const int64_t cols = MODE == GATED ? N / 2 : N;
+  const int64_t col = (MODE == GATED ? n0 / 2 : n0) + wn * COLS + 8 * (lane % CH);
+  const bool vec = col + 8 <= cols && ((ldc | ldr) & 7) == 0 &&
+                   ((reinterpret_cast<uintptr_t>(C) | reinterpret_cast<uintptr_t>(R)) & 15) == 0;
+#pragma unroll 4
+  for (int it = 0; it < 128 * CH / 64; ++it) {
+    const int lr = it * (64 / CH) + lane / CH;
+    const int64_t row = m0 + wm * 128 + lr;
+    u32x4 o = *reinterpret_cast<const u32x4*>(out + lr * PITCH + 16 * (lane % CH));
+    if (row >= M) continue;
+    if (vec) {
+      if (MODE == PLAIN && R) {
+        const u32x4 r = *reinterpret_cast<const u32x4*>(R + row * ldr + col);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          o[e] = (uint32_t)f32_to_bf16(bf16_to_f32((uint16_t)o[e]) + bf16_to_f32((uint16_t)r[e])) |
+                 ((uint32_t)f32_to_bf16(bf16_to_f32((uint16_t)(o[e] >> 16)) + bf16_to_f32((uint16_t)(r[e] >> 16))) << 16);
+      }
+      *reinterpret_cast<u32x4*>(C + row * ldc + col) = o;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if (col + e >= cols) break;
+        uint16_t x = (uint16_t)(o[e / 2] >> (16 * (e & 1)));
+        if (MODE == PLAIN && R) x = f32_to_bf16(bf16_to_f32(x) + bf16_to_f32(R[row * ldr + col + e]));
+        C[row * ldc + col + e] = x;
+      }
     }
   }
 }
@@ -541,18 +823,34 @@ int split_for(int64_t N, int64_t K) {
   return s;
 }
 
-// The LDS-kernel configuration a shape runs with. M <= 64 (a decode step) takes 64-row tiles. Larger
-// M takes 224-row tiles when they pad M less than 128- and 256-row tiles would (the verify pass,
-// M = 64 * 7 = 448, is exactly two), else 256- or 128-row tiles. Every configuration runs the same
-// MFMA over the same k order, so the tile shape never changes a result.
+// The tile a shape runs with. M <= 64 (a decode step) takes 64-row tiles, larger M the cheapest of
+// cheapest_tile's. Every configuration runs the same MFMA over the same k order, so the tile shape never
+// changes a result.
 struct LdsCfg {
   int bm, bn, wgm, wgn;
 };
 
-// Share of the CU slots a grid of `tiles` workgroups keeps busy (one tile per CU at a time, 256 CUs).
-double tile_fill(int64_t tiles) {
-  constexpr int64_t kCUs = 256;
-  return (double)tiles / (double)(kCUs * ((tiles + kCUs - 1) / kCUs));
+// The tile whose grid takes the fewest CU rounds (256 workgroups at a time), each weighed by what a round's
+// 64-deep stage takes in that tile (us, measured at M = 8005 and 448 on the 8B and 1B projections; `us`
+// receives the stage time of the whole grid). Against a fixed preference by how M pads: M = 256 down
+// (N 4096, K 14336) 68 -> 49 us and 1B gate|up 39.7 -> 27.6 us in 128 x 128 tiles instead of wider ones,
+// M = 7373 gate|up 1.62 -> 1.31 ms in 256 x 256 tiles instead of 224 x 224.
+LdsCfg cheapest_tile(int64_t M, int64_t N, int splits, double& us) {
+  struct Cand {
+    LdsCfg cf;
+    double us;
+  };
+  static const Cand cands[] = {{{256, 256, 4, 2}, 1.56}, {{224, 256, 2, 8}, 1.65}, {{224, 224, 7, 2}, 1.53},
+                               {{128, 256, 2, 4}, 1.153}, {{224, 128, 2, 4}, 1.07}, {{224, 96, 7, 2}, 0.864},
+                               {{128, 128, 2, 4}, 0.68}};
+  LdsCfg best = cands[0].cf;
+  us = 1e30;
+  for (const Cand& c : cands) {
+    const int64_t tiles = ((M + c.cf.bm - 1) / c.cf.bm) * ((N + c.cf.bn - 1) / c.cf.bn) * splits;
+    const double t = (double)((tiles + 255) / 256) * c.us;
+    if (t < us) us = t, best = c.cf;
+  }
+  return best;
 }
 
 LdsCfg lds_cfg(int64_t M, int64_t N, int splits, bool stats = false) {
@@ -562,34 +860,24 @@ LdsCfg lds_cfg(int64_t M, int64_t N, int splits, bool stats = false) {
   if (M <= 64)
     return N * splits >= 65536 ? (stats ? LdsCfg{64, 256, 2, 8} : LdsCfg{64, 128, 2, 4}) : LdsCfg{64, 64, 2, 2};
   auto pad = [&](int64_t bm) { return (M + bm - 1) / bm * bm - M; };
-  if (pad(224) < pad(128) && pad(224) < pad(256)) {
-    const int64_t tm = (M + 223) / 224;
-    if (stats) {   // 16 waves of 32-column blocks: the blocks a 64-row head's statistics use too
-      const int64_t t256 = tm * ((N + 255) / 256);
+  if (stats) {   // 16 waves of 32-column blocks where 224 rows pad least: the blocks a 64-row head uses too
+    if (pad(224) < pad(128) && pad(224) < pad(256)) {
+      const int64_t t256 = (M + 223) / 224 * ((N + 255) / 256);
       return t256 >= 192 ? LdsCfg{224, 256, 2, 8} : LdsCfg{224, 128, 2, 4};
     }
-    // the width whose tile count fills the CUs best, weighted by the throughput a tile of that
-    // width reaches (measured on the decoder's projections at M = 448: wider tiles re-read less)
-    struct Cand {
-      LdsCfg cf;
-      double eff;
-    };
-    const Cand cands[] = {{{224, 256, 2, 8}, 1.0}, {{224, 224, 7, 2}, 0.97}, {{224, 128, 2, 4}, 0.85},
-                          {{224, 96, 7, 2}, 0.8}};
-    LdsCfg best = cands[0].cf;
-    double best_score = -1.0;
-    for (const Cand& c : cands) {
-      const double score = tile_fill(tm * ((N + c.cf.bn - 1) / c.cf.bn) * splits) * c.eff;
-      if (score > best_score) best_score = score, best = c.cf;
-    }
-    return best;
+    const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256);
+    const int64_t t128 = ((M + 127) / 128) * ((N + 255) / 256);
+    if (t256 >= 192) return LdsCfg{256, 256, 4, 2};
+    if (t128 >= 128) return LdsCfg{128, 256, 2, 4};
+    return LdsCfg{128, 128, 2, 4};
   }
-  const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256) * splits;
-  const int64_t t128 = ((M + 127) / 128) * ((N + 255) / 256) * splits;
-  if (t256 >= 192) return LdsCfg{256, 256, 4, 2};
-  if (t128 >= 128) return LdsCfg{128, 256, 2, 4};
-  return LdsCfg{128, 128, 2, 4};
+  double us = 0;
+  return cheapest_tile(M, N, splits, us);
 }
+
+// gemm_bf16_long_kernel keeps a lane's source rows as 32-bit byte offsets: from the tile's first row, or, with
+// the gate and up rows interleaved, from the weight's.
+bool long_ok(int64_t lda, int64_t ldb, int64_t N) { return lda < (1 << 22) && ldb * (N > 256 ? N : 256) < (1LL << 31); }
 
 template <bool STATS, bool SWIGLU = false>
 void launch_lds(const uint16_t* a, int64_t lda, const uint16_t* b, int64_t ldb, uint16_t* c, int64_t ldc,
@@ -606,11 +894,17 @@ void launch_lds(const uint16_t* a, int64_t lda, const uint16_t* b, int64_t ldb, 
   if (cf.bm == 64 && cf.bn == 256) FS_LDS_LAUNCH(64, 256, 2, 2, 8, false);
   else if (cf.bm == 64 && cf.bn == 128) FS_LDS_LAUNCH(64, 128, 3, 2, 4, false);
   else if (cf.bm == 64) FS_LDS_LAUNCH(64, 64, 4, 2, 2, false);
-  else if (cf.bm == 224 && cf.bn == 256 && cf.wgn == 8) FS_LDS_LAUNCH(224, 256, 2, 2, 8, true);
-  else if (cf.bm == 224 && cf.bn == 256) FS_LDS_LAUNCH(224, 256, 2, 2, 4, false);
+  else if (cf.bm == 224 && cf.bn == 256) FS_LDS_LAUNCH(224, 256, 2, 2, 8, true);
   else if (cf.bm == 224 && cf.bn == 224) FS_LDS_LAUNCH(224, 224, 2, 7, 2, false);
   else if (cf.bm == 224 && cf.bn == 96) FS_LDS_LAUNCH(224, 96, 3, 7, 2, false);
   else if (cf.bm == 224) FS_LDS_LAUNCH(224, 128, 3, 2, 4, false);
+  else if (cf.bm == 256 && !STATS && long_ok(lda, ldb, N)) {
+    if (part)
+      gemm_bf16_long_kernel<PARTIAL><<<grid, 512, 0, s>>>(a, lda, b, ldb, c, ldc, r, ldr, M, N, K, tm, nt, part);
+    else
+      gemm_bf16_long_kernel<SWIGLU ? GATED : PLAIN><<<grid, 512, 0, s>>>(a, lda, b, ldb, c, ldc, r, ldr, M, N, K, tm, nt,
+                                                                         nullptr);
+  }
   else if (cf.bm == 256) FS_LDS_LAUNCH(256, 256, 2, 4, 2, false);
   else if (cf.bn == 256) FS_LDS_LAUNCH(128, 256, 3, 2, 4, false);
   else FS_LDS_LAUNCH(128, 128, 4, 2, 4, false);
@@ -624,11 +918,21 @@ bool lds_ok(const void* A, int64_t lda, const void* B, int64_t ldb, int64_t K) {
 // A split-K shape whose unsplit 256 x 128 tiles alone fill the GPU twice over (a long prefill) runs its
 // K splits one after the other inside each workgroup: the split-K arithmetic without the f32 partials.
 // Only for splits of at most 2048 k: there the partials' HBM traffic costs more than the narrower tile
-// the running sum forces (measured at M = 32768: the o projection 1.80 -> 1.38 ms, qkv even); with
-// 3584-k splits (the down projection) the 256 x 256 tiles and their partials are faster (3.9 vs 4.6 ms).
+// the running sum forces (measured at M = 8005: the 8B o projection 0.31 ms against 0.43, the 1B down
+// projection 0.28 against 0.41); with 3584-k splits (the 8B down projection) the 256 x 256 tiles and their
+// partials are faster (M = 32768: 3.4 ms against 4.6). Fewer tiles do so where the rounds of serial tiles
+// (1.12 us a stage and 6 us a round) cost less than the partials' tiles plus writing and reading
+// splits * M * N floats at 4.5 TB/s (M = 7373 1B down, 464 tiles: 0.29 ms against 0.38).
 constexpr int kSerialTiles = 512;
 bool serial_for(int64_t M, int64_t N, int64_t K, int splits) {
-  return splits > 1 && K / splits <= 2048 && ((M + 255) / 256) * ((N + 127) / 128) >= kSerialTiles;
+  if (splits <= 1 || K / splits > 2048 || M <= 64) return false;
+  const int64_t tiles = ((M + 255) / 256) * ((N + 127) / 128);
+  if (tiles >= kSerialTiles) return true;
+  const double stages = (double)(K / 64);
+  double us = 0;
+  cheapest_tile(M, N, splits, us);
+  return (double)((tiles + 255) / 256) * (stages * 1.12 + 6.0) <
+         us * stages / splits + (double)splits * (double)M * (double)N * 8.0 / 4.5e6;
 }
 
 void launch_serial(const uint16_t* a, int64_t lda, const uint16_t* b, int64_t ldb, uint16_t* c, int64_t ldc,

@@ -201,6 +201,30 @@ def test_long_batch_rows_equal_short_batch_rows(m, n, k, kind):
         assert torch.equal(fn(a[lo:hi], w), full[lo:hi])
 
 
+@pytest.mark.parametrize("m,n,k,kind", [(2303, 6100, 64, "plain"), (2290, 6001, 128, "plain"), (2303, 6104, 192, "plain"),
+                                        (2303, 6100, 8192, "plain"),   # K split in two, f32 partials
+                                        (2291, 6100, 320, "gated"), (2304, 6148, 64, "gated")])
+def test_gemm_long_batch_tiles(m, n, k, kind):
+    """The long batches' 256 x 256 tiles at the edges of M and N (rows of no whole 16 bytes among them), with
+    1, 2, 3, 5 and 64 stages of K, with a residual: every row as a short batch gives it, bit for bit."""
+    case("gemm long tiles", m, n, k, kind)
+    g = torch.Generator().manual_seed(m + n + k)
+    a = torch.randn(m, k, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(n, k, generator=g) * 0.05).bfloat16().to(DEV)
+    r = torch.randn(m, n, generator=g).bfloat16().to(DEV)
+    if kind == "gated":
+        run = lambda lo, hi: [ops.gemm_swiglu(a[lo:hi], w)]
+    else:
+        run = lambda lo, hi: [ops.gemm(a[lo:hi], w), ops.gemm(a[lo:hi], w, residual=r[lo:hi])]
+    full = run(0, m)
+    for lo in (0, 230, 1000, m - 60):
+        for x, y in zip(run(lo, min(lo + 60, m)), full):
+            assert torch.equal(x, y[lo: lo + 60]), lo
+    if kind == "plain":   # one rounding of the product (and of the sum with the residual)
+        ref = a[-64:].double() @ w.double().T.contiguous()
+        assert ((full[0][-64:].double() - ref).abs() <= ref.abs() * 2 ** -8 + 1e-3).all()
+
+
 # ---- row ops ------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_rmsnorm_and_residual(dtype):
