@@ -69,12 +69,17 @@ template <> struct Elem<FS_F16> {
 // ------------------------------------------------------------------------------------------------
 // wavefront (64-lane) reductions
 // ------------------------------------------------------------------------------------------------
-// silu(g) * u as a 16-bit SwiGLU computes it (model.py:93): silu rounded to the dtype, then the
-// product, which the caller rounds when it stores it; g and u are dtype values. Every kernel that
-// forms this product calls this one function, so their results agree bit for bit.
+// silu(g) * u as SwiGLU computes it (model.py:93): silu rounded to the dtype, then the product, which the
+// caller rounds when it stores it; g and u are dtype values. Every kernel that forms this product calls
+// this one function, so their results agree bit for bit. For the 16-bit types the exponential and the
+// reciprocal are the hardware's (float32, 5e-6 relative where e^-g is largest, against the dtype's 2^-9 or
+// 2^-12): expf and a correctly rounded division are ~45 instructions an element, 6% of a long gate|up
+// product (8005 x 28672 x 4096: 1.58 -> 1.49 ms).
 template <int DT>
 FS_DEVICE float silu_times(float g, float u) {
-  return Elem<DT>::round(g / (1.0f + expf(-g))) * u;
+  if (DT == FS_F32) return g / (1.0f + expf(-g)) * u;
+  const float e = __builtin_amdgcn_exp2f(g * -1.4426950408889634f);
+  return Elem<DT>::round(g * __builtin_amdgcn_rcpf(1.0f + e)) * u;
 }
 
 FS_DEVICE float wave_max(float v) {
