@@ -30,9 +30,7 @@ namespace {
 
 constexpr int QTILE = 32;            // query rows per MFMA wave
 constexpr int PLAN_THREADS = 256;
-constexpr int SPLIT_UNITS_MAX = 128;  // calls with at most this many units (half the CUs) split each in two,
-constexpr int SPLIT_MIN_KEYS = 3072;  // when their tables can hold this many keys (shorter units do not repay
-                                      // the exchange)
+constexpr int SPLIT_UNITS_MAX = 128;  // calls with at most this many units (half the CUs) may split each
 // workspace: item count (bytes 0..255), the split units' arrival counters (one unsigned each), then
 // the item list, the chunk partials and the split units' published partials
 constexpr int64_t WS_COUNTERS = 256;
@@ -67,7 +65,7 @@ struct AttnParams {
   // query tiles per plan item: 1 for the unit kernel, PF_WAVES for the prefill kernel (item.z is then
   // the index of a group of zgroup consecutive tiles, item.qmax the group's furthest query)
   int32_t zgroup;
-  // split units (attn_unit_half_kernel): one arrival counter per unit (zero between launches) and
+  // split units (attn_unit_part_kernel): one arrival counter per unit (zero between launches) and
   // SPLIT_SLOTS published partials per unit
   unsigned* split_cnt;
   float* split_ws;
@@ -154,8 +152,7 @@ FS_DEVICE int tile_chunks(const AttnParams& P, int qmax) {
 }
 
 constexpr int UNIT_WAVES = 8;                  // waves per unit workgroup
-constexpr int HALF_WAVES = UNIT_WAVES / 2;      // waves per workgroup of a split unit
-constexpr int SPLIT_SLOTS = 5;                  // published partials per split unit
+constexpr int SPLIT_SLOTS = 7;                  // published partials per split unit, at most (four parts)
 // floats of one published partial: m and l of the 32 rows, then acc as the LDS holds it (2 * D/16
 // (half, dim tile) pairs, 64 lanes, 4 values)
 constexpr int64_t split_slot_floats(int D) { return 2 * QTILE + (int64_t)QTILE * D; }
@@ -189,7 +186,7 @@ FS_DEVICE int block_scan(int x, int* sh, int& tot) {
 }
 
 __global__ void __launch_bounds__(PLAN_THREADS) attn_plan_kernel(AttnParams P) {
-  // the split units' arrival counters start at zero (each unit's second half leaves its counter zero,
+  // the split units' arrival counters start at zero (each unit's last part leaves its counter zero,
   // so calls that reuse this plan find them so too)
   for (int i = threadIdx.x; i < SPLIT_UNITS_MAX; i += PLAN_THREADS) st_ag(P.split_cnt + i, 0u);
   __shared__ int sh[PLAN_THREADS / 64];
@@ -335,13 +332,14 @@ constexpr float REF_SLACK = 8.f;   // log2 units a tile's maximum may exceed the
 // MFMA operands, and l <- l * alpha + (the lane's sum of p), alpha = 2^(m_old - m_new) for a row
 // that moved, else 1. Returns whether any row of the wave moved; alpha is for the caller's rescale
 // of acc. LAZY: when no row moved, l <- l + sum, which is l * 1 + sum bit for bit.
-template <bool FULL, bool LAZY>
+template <bool FULL, bool LAZY, bool TWO>
 FS_DEVICE bool tile_probs(const float4_t (&sc)[2], int j0, bool tile_valid, const int (&rpos)[2], float scale_log2,
                           float (&m_run)[2], float (&l_run)[2], float (&alpha)[2], short4_t (&pf)[2]) {
+  constexpr int NT = TWO ? 2 : 1;
   const int g = (threadIdx.x & 63) >> 4;
   float sv[2][4], x[2];
 #pragma unroll
-  for (int nt = 0; nt < 2; ++nt) {
+  for (int nt = 0; nt < NT; ++nt) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const float v = sc[nt][e] * scale_log2;
@@ -353,9 +351,9 @@ FS_DEVICE bool tile_probs(const float4_t (&sc)[2], int j0, bool tile_valid, cons
   // A row's tile maximum exceeds m + REF_SLACK exactly when one of its four lane groups' maxima does.
   // LAZY: when no lane's does, no row moves (m_new = m, alpha = 1), and the reduction across the lane
   // groups is skipped: the same values as the path below.
-  if (LAZY && !__any(x[0] > m_run[0] + REF_SLACK || x[1] > m_run[1] + REF_SLACK)) {
+  if (LAZY && !__any(x[0] > m_run[0] + REF_SLACK || (TWO && x[1] > m_run[1] + REF_SLACK))) {
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
+    for (int nt = 0; nt < NT; ++nt) {
       float pv[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e)
@@ -367,11 +365,11 @@ FS_DEVICE bool tile_probs(const float4_t (&sc)[2], int j0, bool tile_valid, cons
     return false;
   }
   float tmax[2];
-  max_across_groups2(x[0], x[1], tmax[0], tmax[1]);
+  max_across_groups2(x[0], x[TWO ? 1 : 0], tmax[0], tmax[1]);
   bool mv[2];
   float m_new[2], psum[2];
 #pragma unroll
-  for (int nt = 0; nt < 2; ++nt) {
+  for (int nt = 0; nt < NT; ++nt) {
     // (-inf > x is false: a row that sees nothing here keeps its reference)
     mv[nt] = tmax[nt] > m_run[nt] + REF_SLACK;
     m_new[nt] = mv[nt] ? tmax[nt] : m_run[nt];
@@ -382,33 +380,35 @@ FS_DEVICE bool tile_probs(const float4_t (&sc)[2], int j0, bool tile_valid, cons
     pf[nt] = bf16_rne4(pv);
     psum[nt] = (pv[0] + pv[1]) + (pv[2] + pv[3]);
   }
-  const bool moved = __any(mv[0] || mv[1]);
+  const bool moved = __any(mv[0] || (TWO && mv[1]));
   if (!LAZY || moved) {
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
+    for (int nt = 0; nt < NT; ++nt) {
       alpha[nt] = mv[nt] ? fast_exp2(m_run[nt] - m_new[nt]) : 1.f;
       l_run[nt] = l_run[nt] * alpha[nt] + psum[nt];
     }
   } else {
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
+    for (int nt = 0; nt < NT; ++nt) {
       alpha[nt] = 1.f;
       l_run[nt] = l_run[nt] + psum[nt];
     }
   }
 #pragma unroll
-  for (int nt = 0; nt < 2; ++nt) m_run[nt] = m_new[nt];
+  for (int nt = 0; nt < NT; ++nt) m_run[nt] = m_new[nt];
   return moved;
 }
 
-template <int D, bool LAZY, bool BOTH = false>
+// SEEN: every row sees every key of the tile (the caller knows; j0, tile_valid and qmax are not looked at).
+template <int D, bool LAZY, bool TWO, bool BOTH = false, bool SEEN = false>
 FS_DEVICE void attn_tile(const bf16x8_t (&kf)[D / 32], short4_t (&vf)[D / 16], int j0, bool tile_valid, int qmax,
                          const int (&rpos)[2], int rmin, bool two, const bf16x8_t (&qf)[2][D / 32],
                          float scale_log2, float4_t (&acc)[D / 16][2], float (&m_run)[2], float (&l_run)[2]) {
   constexpr int KS = D / 32;
   constexpr int MT = D / 16;
+  constexpr int NT = TWO ? 2 : 1;
   const int g = (threadIdx.x & 63) >> 4;
-  const bool full = tile_valid && j0 + 15 <= rmin;   // wave-uniform
+  const bool full = SEEN || (tile_valid && j0 + 15 <= rmin);   // wave-uniform
   if (!full && (!tile_valid || j0 + 15 > qmax)) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -431,7 +431,7 @@ FS_DEVICE void attn_tile(const bf16x8_t (&kf)[D / 32], short4_t (&vf)[D / 16], i
     }
   } else {
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
+    for (int nt = 0; nt < NT; ++nt) {
       sc[nt] = float4_t{0.f, 0.f, 0.f, 0.f};
       if (nt == 0 || two) {
 #pragma unroll
@@ -442,14 +442,14 @@ FS_DEVICE void attn_tile(const bf16x8_t (&kf)[D / 32], short4_t (&vf)[D / 16], i
   }
   short4_t pf[2];
   float alpha[2];
-  const bool moved = full ? tile_probs<true, LAZY>(sc, j0, tile_valid, rpos, scale_log2, m_run, l_run, alpha, pf)
-                          : tile_probs<false, LAZY>(sc, j0, tile_valid, rpos, scale_log2, m_run, l_run, alpha, pf);
+  const bool moved = full ? tile_probs<true, LAZY, TWO>(sc, j0, tile_valid, rpos, scale_log2, m_run, l_run, alpha, pf)
+                          : tile_probs<false, LAZY, TWO>(sc, j0, tile_valid, rpos, scale_log2, m_run, l_run, alpha, pf);
   // LAZY: only when a row moved (alpha = 1 for every row that did not, so skipping it is exact)
   if (!LAZY || moved) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < 2; ++nt) {
+      for (int nt = 0; nt < NT; ++nt) {
         acc[mt][nt][0] *= alpha[nt];
         acc[mt][nt][1] *= alpha[nt];
         acc[mt][nt][2] *= alpha[nt];
@@ -459,7 +459,7 @@ FS_DEVICE void attn_tile(const bf16x8_t (&kf)[D / 32], short4_t (&vf)[D / 16], i
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     acc[mt][0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vf[mt], pf[0], acc[mt][0], 0, 0, 0);
-    if (BOTH || two) acc[mt][1] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vf[mt], pf[1], acc[mt][1], 0, 0, 0);
+    if (TWO && (BOTH || two)) acc[mt][1] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vf[mt], pf[1], acc[mt][1], 0, 0, 0);
   }
 }
 
@@ -476,7 +476,15 @@ FS_DEVICE bool fold_weights(float M, float m, float& Mn, float& cM, float& cm) {
 }
 FS_DEVICE float fold_value(float x, float cM, float y, float cm) { return x * cM + y * cm; }
 
-template <int D, int BSZ>
+// Tile buffers of a wave. Two (one tile in flight) keep the unit kernel's 2,048 waves at what HBM delivers:
+// with three or four it is 1-10% slower (64 rows of 2048-8192 keys, T = 1: 205 / 209 / 211 us; of 1000-2000
+// slot-major keys: 71 / 76 / 82). Two waves on a CU (four parts) want a second tile in flight (one row of
+// 16000 keys: 59 -> 48 us; a third: 48), four (two parts) one at 128 dims and two at 64.
+constexpr int UNIT_BUFS = 2;
+constexpr int part_bufs(int D, int parts) { return parts == 4 || D == 64 ? 3 : 2; }
+
+// TWO: the tile has a second 16-row half. NB: tile buffers in registers.
+template <int D, int BSZ, bool TWO, int NB>
 __device__ __attribute__((always_inline)) inline void attn_wave_tiles(const AttnParams& P, int b, int kbeg, int kend,
                                                                       int qmax, int row0, int nrows,
                                                                       const int (&rpos)[2], int hkv, int w,
@@ -484,74 +492,51 @@ __device__ __attribute__((always_inline)) inline void attn_wave_tiles(const Attn
                                                                       float* red_l) {
   constexpr int KS = D / 32;   // k-steps of the QK^T product
   constexpr int MT = D / 16;   // 16-dim tiles of the PV product
+  constexpr int NT = TWO ? 2 : 1;
   const int lane = threadIdx.x & 63;
   const int l16 = lane & 15, g = lane >> 4;
   const int ntiles = (kend - kbeg + 15) >> 4;
   const int nt_w = ntiles > w ? (ntiles - w + UNIT_WAVES - 1) / UNIT_WAVES : 0;   // <= 128 tiles
-  const bool two = nrows > 16;
+  const bool two = TWO && nrows > 16;
   const int BS = BSZ ? BSZ : P.kv.block_size;
   const int64_t v_dim = BSZ ? BSZ : P.kv.v_dim;   // == block_size (dim-major values)
 
-  // lane i: raw table entries of the blocks holding this wave's tiles i and 64 + i (-1 past the table)
-  int my_phys[2] = {-1, -1};
+  // lane i: where the wave's tiles i and 64 + i start in the pool, in 16-byte units from the head's base (an
+  // unmapped block reads block 0 and is masked), and which of them are mapped
+  typedef uint16_t u16;
+  const u16* kpool = reinterpret_cast<const u16*>(P.kv.k) + (int64_t)hkv * P.kv.k_head;
+  const u16* vpool = reinterpret_cast<const u16*>(P.kv.v) + (int64_t)hkv * P.kv.v_head;
+  const int64_t k_slot = P.kv.k_slot;
+  uint32_t k_at[2] = {0, 0}, v_at[2] = {0, 0};
+  uint64_t mapped[2];
+  {
+    int phys[2] = {-1, -1}, slot0[2] = {0, 0};
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int i = 64 * h + lane;
-    if (i < nt_w) {
-      const int blk = (kbeg + 16 * (w + UNIT_WAVES * i)) / BS;
-      if (blk < P.max_blocks) my_phys[h] = P.table[(int64_t)b * P.table_stride + blk];
+    for (int h = 0; h < 2; ++h) {
+      const int i = 64 * h + lane;
+      if (i < nt_w) {
+        const int j0 = kbeg + 16 * (w + UNIT_WAVES * i), blk = j0 / BS;
+        slot0[h] = j0 - blk * BS;
+        if (blk < P.max_blocks) phys[h] = P.table[(int64_t)b * P.table_stride + blk];
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const bool ok = phys[h] >= 0 && phys[h] < P.kv.num_blocks;
+      mapped[h] = __ballot(ok);
+      const int64_t pb = ok ? phys[h] : 0;
+      k_at[h] = (uint32_t)((pb * P.kv.k_block + slot0[h] * k_slot) >> 3);
+      v_at[h] = (uint32_t)((pb * P.kv.v_block + slot0[h]) >> 3);
     }
   }
 
-  typedef uint16_t u16;
-  const u16* kpool = reinterpret_cast<const u16*>(P.kv.k);
-  const u16* vpool = reinterpret_cast<const u16*>(P.kv.v);
-  const int64_t k_head_off = (int64_t)hkv * P.kv.k_head;
-  const int64_t v_head_off = (int64_t)hkv * P.kv.v_head;
-  // key (slot, dims 8c .. 8c+7) at slot * k_slot + c * kgs: slot-major (k_slot = D, kgs = 8) or grouped
-  // (k_slot = 8, kgs = 8 * block_size: one load of a tile's 32 dims is a contiguous 1 KB)
-  const int64_t k_slot = P.kv.k_slot, kgs = key_group_stride(P.kv);
-
-  // Three tile buffers in registers: while tile i is consumed, tiles i+1 and i+2 are in flight.
-  // Every load is unconditional (a prefetch past the end re-reads the last tile, an unmapped block
-  // reads block 0 and is masked in consume) so that each wait before a consume counts exactly the
-  // loads issued after that tile, on every path through the loop.
-  bf16x8_t kb0[KS], kb1[KS], kb2[KS];
-  short4_t vb0[MT], vb1[MT], vb2[MT];
-
-  auto key0 = [&](int i) { return kbeg + 16 * (w + UNIT_WAVES * i); };
-  auto block_of = [&](int i) {   // physical block of the wave's i-th tile, -1 when unmapped (i uniform)
-    const int v = __builtin_amdgcn_readlane(i < 64 ? my_phys[0] : my_phys[1], i & 63);
-    return (v >= 0 && v < P.kv.num_blocks) ? v : -1;
-  };
-
-  // the lane's element offsets inside a tile, fixed for the launch; a tile adds its wave-uniform base
-  const int64_t k_lane = (int64_t)l16 * k_slot + g * kgs;
-  const int64_t v_lane = (int64_t)l16 * v_dim + 4 * g;
-  auto load_tile = [&](int i, bf16x8_t (&kd)[KS], short4_t (&vd)[MT]) {
-    const int ic = max(min(i, nt_w - 1), 0);   // a wave without tiles reads block 0 and consumes nothing
-    const int j0 = key0(ic);
-    const int phys = block_of(ic);
-    const int64_t pb = phys >= 0 ? phys : 0;
-    const int slot0 = j0 - (j0 / BS) * BS;
-    const u16* kt_ = kpool + (pb * P.kv.k_block + k_head_off + (int64_t)slot0 * k_slot) + k_lane;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)   // read once per launch: nontemporal
-      kd[ks] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(kt_ + 4 * ks * kgs));
-    const u16* vt_ = vpool + (pb * P.kv.v_block + v_head_off + slot0) + v_lane;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-      vd[mt] = __builtin_nontemporal_load(reinterpret_cast<const short4_t*>(vt_ + (int64_t)(16 * mt) * v_dim));
-  };
-
-  load_tile(0, kb0, vb0);
-  load_tile(1, kb1, vb1);
-
-  // Q fragments (B operand of S^T): Q[row][32*ks + 8*g .. +8]
+  // Q fragments (B operand of S^T): Q[row][32*ks + 8*g .. +8]. Loaded before the first tiles: vmcnt counts in
+  // order, so a wait for queries loaded after them would wait for every tile in flight, at each turn of
+  // the loop (the compiler merges the first turn's state into all).
   const u16* qbase = reinterpret_cast<const u16*>(P.q);
   bf16x8_t qf[2][KS];
 #pragma unroll
-  for (int nt = 0; nt < 2; ++nt) {
+  for (int nt = 0; nt < NT; ++nt) {
     const int r = row0 + 16 * nt + l16;
     const bool in_tile = (16 * nt + l16) < nrows;
     const bool ok = in_tile && token_exists(P, b, r / P.G);
@@ -567,6 +552,46 @@ __device__ __attribute__((always_inline)) inline void attn_wave_tiles(const Attn
     }
   }
 
+  // NB tile buffers in registers: while tile i is consumed, tiles i+1 .. i+NB-1 are in flight. Every load is
+  // unconditional (a prefetch past the end re-reads the last tile) and the loops have one back edge each,
+  // so that each wait before a product counts exactly the loads issued after its operand.
+  static_assert((NB - 1) * (KS + MT) < 64, "vmcnt counts every load in flight");
+  bf16x8_t kb[NB][KS];
+  short4_t vb[NB][MT];
+  auto key0 = [&](int i) { return kbeg + 16 * (w + UNIT_WAVES * i); };
+  // a lane's byte offsets inside a tile; a tile adds its wave-uniform base. Key (slot, dims 8c .. 8c+7) is at
+  // slot * k_slot + c * kgs: slot-major (k_slot = D, kgs = 8) or grouped (k_slot = 8, kgs = 8 * block_size:
+  // one load of a tile's 32 dims is a contiguous 1 KB)
+  const int64_t kgs = key_group_stride(P.kv);
+  uint32_t k_lane[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) k_lane[ks] = (uint32_t)(2 * (l16 * k_slot + (g + 4 * ks) * kgs));
+  const uint32_t v_lane = (uint32_t)(2 * (l16 * v_dim + 4 * g));
+  auto load_tile = [&](int i, bf16x8_t (&kd)[KS], short4_t (&vd)[MT]) {
+    const int ic = max(min(i, nt_w - 1), 0);   // (a wave without tiles reads block 0 and consumes nothing)
+    const int k0 = __builtin_amdgcn_readlane((int)k_at[0], ic & 63), k1 = __builtin_amdgcn_readlane((int)k_at[1], ic & 63);
+    const int v0 = __builtin_amdgcn_readlane((int)v_at[0], ic & 63), v1 = __builtin_amdgcn_readlane((int)v_at[1], ic & 63);
+    uint64_t kt_ = reinterpret_cast<uint64_t>(kpool) + ((uint64_t)(uint32_t)(ic < 64 ? k0 : k1) << 4);
+    uint64_t vt_ = reinterpret_cast<uint64_t>(vpool) + ((uint64_t)(uint32_t)(ic < 64 ? v0 : v1) << 4);
+    asm("" : "+s"(kt_), "+s"(vt_));   // a scalar base and 32-bit lane offsets: no 64-bit vector adds per load
+    typedef __attribute__((address_space(1))) const char GChar;
+    typedef __attribute__((address_space(1))) const bf16x8_t GKey;
+    typedef __attribute__((address_space(1))) const short4_t GVal;
+    GChar* kt = (GChar*)kt_;
+    GChar* vt = (GChar*)vt_;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)   // read once per launch: nontemporal
+      kd[ks] = __builtin_nontemporal_load((GKey*)(kt + k_lane[ks]));
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+      vd[mt] = __builtin_nontemporal_load((GVal*)(vt + (v_lane + (uint32_t)(32 * mt * v_dim))));
+  };
+#pragma unroll
+  for (int j = 0; j < NB - 1; ++j) {
+    load_tile(j, kb[j], vb[j]);
+    __builtin_amdgcn_sched_barrier(0);   // in tile order, as the loops' waits count them
+  }
+
   float4_t acc[MT][2];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
@@ -576,25 +601,37 @@ __device__ __attribute__((always_inline)) inline void attn_wave_tiles(const Attn
   float m_run[2] = {-INFINITY, -INFINITY};
   float l_run[2] = {0.f, 0.f};
 
+  // The wave's first n_full tiles have every key mapped and seen by every row: they take a loop without
+  // masks or lookups. The rest (the tiles around the rows' own positions, or all of them where a row is
+  // padding or a block unmapped) are consumed one by one.
   const int rmin = rows_min_pos(rpos, nrows);
-  auto consume = [&](int i, const bf16x8_t (&kf)[KS], short4_t (&vf)[MT]) {
-    attn_tile<D, true>(kf, vf, key0(i), block_of(i) >= 0, qmax, rpos, rmin, two, qf, P.scale_log2, acc, m_run,
-                        l_run);
-  };
-
-  for (int i = 0; i < nt_w; i += 3) {
-    load_tile(i + 2, kb2, vb2);
-    consume(i, kb0, vb0);
-    if (i + 1 >= nt_w) break;
-    load_tile(i + 3, kb0, vb0);
-    consume(i + 1, kb1, vb1);
-    if (i + 2 >= nt_w) break;
-    load_tile(i + 4, kb1, vb1);
-    consume(i + 2, kb2, vb2);
+  const int n_seen = rmin + 1 > kbeg ? min((rmin + 1 - kbeg) >> 4, ntiles) : 0;   // tiles all rows see
+  const uint64_t want0 = nt_w >= 64 ? ~0ull : (1ull << nt_w) - 1;
+  const uint64_t want1 = nt_w >= 128 ? ~0ull : nt_w > 64 ? (1ull << (nt_w - 64)) - 1 : 0;
+  const bool all_mapped = (mapped[0] & want0) == want0 && (mapped[1] & want1) == want1;
+  const int n_full = all_mapped && n_seen > w ? (n_seen - w + UNIT_WAVES - 1) / UNIT_WAVES : 0;
+  int i = 0;
+  for (; i + NB <= n_full; i += NB) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      load_tile(i + j + NB - 1, kb[(j + NB - 1) % NB], vb[(j + NB - 1) % NB]);
+      attn_tile<D, true, TWO, false, true>(kb[j], vb[j], 0, true, 0, rpos, rmin, two, qf, P.scale_log2, acc, m_run, l_run);
+    }
+  }
+  for (; i < nt_w; i += NB) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      load_tile(i + j + NB - 1, kb[(j + NB - 1) % NB], vb[(j + NB - 1) % NB]);
+      if (i + j < nt_w) {
+        const int t = i + j;
+        const bool valid = (((t < 64 ? mapped[0] : mapped[1]) >> (t & 63)) & 1) != 0;
+        attn_tile<D, true, TWO>(kb[j], vb[j], key0(t), valid, qmax, rpos, rmin, two, qf, P.scale_log2, acc, m_run, l_run);
+      }
+    }
   }
   // this wave's partial to LDS: acc by (query half, dim tile, lane), m and l by query row
 #pragma unroll
-  for (int nt = 0; nt < 2; ++nt) {
+  for (int nt = 0; nt < NT; ++nt) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) red_acc[nt * MT + mt][lane] = acc[mt][nt];
     const float lsum = sum_across_groups(l_run[nt]);
@@ -633,11 +670,11 @@ FS_DEVICE void attn_emit(const AttnParams& P, int b, int s, int kbeg, int hkv, i
   }
 }
 
-template <int D, int BSZ>
+template <int D, int BSZ, bool TWO>
 __global__ void __launch_bounds__(64 * UNIT_WAVES) __attribute__((amdgpu_waves_per_eu(2)))
 attn_unit_kernel(AttnParams P) {
-  constexpr int MT = D / 16;
-  __shared__ float4_t red_acc[UNIT_WAVES][2 * MT][64];
+  constexpr int MT = D / 16, NG = (TWO ? 2 : 1) * MT;
+  __shared__ float4_t red_acc[UNIT_WAVES][NG][64];
   __shared__ float red_m[UNIT_WAVES][QTILE], red_l[UNIT_WAVES][QTILE];
   const int nkv = P.kv.n_kv_heads;
   const int64_t e_idx = blockIdx.x / nkv;
@@ -660,12 +697,12 @@ attn_unit_kernel(AttnParams P) {
   const int kbeg = s * P.split;
   const int kend = min(kbeg + P.split, qmax + 1);
 
-  attn_wave_tiles<D, BSZ>(P, b, kbeg, kend, qmax, row0, nrows, rpos, hkv, w, red_acc[w], red_m[w], red_l[w]);
+  attn_wave_tiles<D, BSZ, TWO, UNIT_BUFS>(P, b, kbeg, kend, qmax, row0, nrows, rpos, hkv, w, red_acc[w], red_m[w], red_l[w]);
   __syncthreads();
 
   // fold the waves' partials in wave order; wave w takes the (query half, 16-dim tile) pairs w,
   // w + UNIT_WAVES, ...
-  for (int gi = w; gi < 2 * MT; gi += UNIT_WAVES) {
+  for (int gi = w; gi < NG; gi += UNIT_WAVES) {
     const int nt = gi / MT, mt = gi - nt * MT;
     const int r = 16 * nt + l16;
     if (r >= nrows) continue;
@@ -688,7 +725,7 @@ attn_unit_kernel(AttnParams P) {
 // Device-coherent accesses to a split unit's published partials: buffer loads and stores with the sc1
 // cache policy (coherent at device scope, the encoding agent-scope atomics get), four floats at a time
 // where the data allows. Being plain accesses, the compiler issues a wave's loads together; the
-// barrier and the arrival count order them against the other half's stores.
+// barrier and the arrival count order them against the other parts' stores.
 constexpr int CPOL_SC1 = 16;
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 FS_DEVICE __amdgpu_buffer_rsrc_t slot_rsrc(float* base, int bytes) {
@@ -707,27 +744,30 @@ FS_DEVICE float ld1_dev(__amdgpu_buffer_rsrc_t r, int off) {
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, CPOL_SC1));
 }
 
-// A unit split in two: workgroup 2u + h (HALF_WAVES waves) builds classes HALF_WAVES*h + w of unit u,
-// each with the unit kernel's attn_wave_tiles, so that a call with few units keeps twice as many CUs
-// streaming. A row's result is the unit kernel's fold over classes 0..7 in increasing order: half 0
-// folds classes 0..3 and publishes that prefix (M, L, O), half 1 publishes its four class partials,
-// and the half that arrives second continues the fold through classes 4..7 and emits the rows. The
-// arrival is counted (an agent-scope atomic), never awaited; the published values cross XCDs through
-// device-coherent accesses.
-template <int D, int BSZ>
-__global__ void __launch_bounds__(64 * HALF_WAVES) __attribute__((amdgpu_waves_per_eu(2)))
-attn_unit_half_kernel(AttnParams P) {
-  constexpr int MT = D / 16, NG = 2 * MT / HALF_WAVES;
+// A unit split over PARTS workgroups: workgroup PARTS * u + part (UNIT_WAVES / PARTS waves) builds classes
+// WPP * part + w of unit u, each with the unit kernel's attn_wave_tiles, so that a call with few units keeps
+// more CUs streaming (a CU has about 40 KB of misses outstanding, 45 GB/s from HBM, however deep its waves
+// prefetch). A row's result is the unit kernel's fold over classes 0..7 in increasing order: part 0 publishes
+// its classes folded, (M, L, O), every other part its class partials one by one, and the part that arrives
+// last folds them in order and emits the rows. The arrival is counted (an agent-scope atomic), never awaited;
+// the published values cross XCDs through device-coherent accesses.
+template <int D, int BSZ, bool TWO, int PARTS>
+__global__ void __launch_bounds__(64 * UNIT_WAVES / PARTS) __attribute__((amdgpu_waves_per_eu(2)))
+attn_unit_part_kernel(AttnParams P) {
+  constexpr int WPP = UNIT_WAVES / PARTS;
+  constexpr int MT = D / 16, GI = (TWO ? 2 : 1) * MT;
+  constexpr int NSLOT = 1 + UNIT_WAVES - WPP;   // part 0's prefix, then classes WPP .. 7
   constexpr int64_t SLOT = split_slot_floats(D);
-  __shared__ float4_t red_acc[HALF_WAVES][2 * MT][64];
-  __shared__ float red_m[HALF_WAVES][QTILE], red_l[HALF_WAVES][QTILE];
+  static_assert(NSLOT <= SPLIT_SLOTS, "the workspace holds the published partials");
+  __shared__ float4_t red_acc[WPP][GI][64];
+  __shared__ float red_m[WPP][QTILE], red_l[WPP][QTILE];
   __shared__ int sh_last;
   const int nkv = P.kv.n_kv_heads;
-  const int64_t unit = blockIdx.x >> 1;
-  const int h = blockIdx.x & 1;
+  const int64_t unit = blockIdx.x / PARTS;
+  const int part = blockIdx.x % PARTS;
   const int64_t e_idx = unit / nkv;
   const int hkv = (int)(unit - e_idx * nkv);
-  if (e_idx >= P.n_items[0]) return;   // uniform over the workgroup (and over both halves)
+  if (e_idx >= P.n_items[0]) return;   // uniform over the workgroup (and over a unit's parts)
   typedef __attribute__((address_space(4))) const AttnItem ConstItem;
   ConstItem* ep = (ConstItem*)(uintptr_t)(P.items + e_idx);
   const int b = ep->b, z = ep->z, s = ep->s, qmax = ep->qmax;
@@ -745,27 +785,23 @@ attn_unit_half_kernel(AttnParams P) {
   const int kbeg = s * P.split;
   const int kend = min(kbeg + P.split, qmax + 1);
 
-  attn_wave_tiles<D, BSZ>(P, b, kbeg, kend, qmax, row0, nrows, rpos, hkv, HALF_WAVES * h + w, red_acc[w], red_m[w],
-                          red_l[w]);
+  attn_wave_tiles<D, BSZ, TWO, part_bufs(D, PARTS)>(P, b, kbeg, kend, qmax, row0, nrows, rpos, hkv, WPP * part + w,
+                                                         red_acc[w], red_m[w], red_l[w]);
   __syncthreads();
 
-  // this unit's published partials, SLOT floats each: slot 0 half 0's prefix, slots 1..4 classes 4..7
+  // this unit's published partials, SLOT floats each
   const __amdgpu_buffer_rsrc_t scr =
       slot_rsrc(P.split_ws + unit * SPLIT_SLOTS * SLOT, (int)(SPLIT_SLOTS * SLOT * sizeof(float)));
   auto m_at = [&](int slot, int r) { return (int)((slot * SLOT + r) * sizeof(float)); };
   auto l_at = [&](int slot, int r) { return (int)((slot * SLOT + QTILE + r) * sizeof(float)); };
   auto acc_at = [&](int slot, int gi) { return (int)((slot * SLOT + 2 * QTILE + (gi * 64 + lane) * 4) * sizeof(float)); };
-  float Mp[NG], Lp[NG];
-  float4_t op[NG];
-  if (h == 0) {   // classes 0..3 folded as the unit kernel folds them, then published
-#pragma unroll
-    for (int j = 0; j < NG; ++j) {
-      const int gi = w + HALF_WAVES * j, nt = gi / MT, mt = gi - nt * MT;
-      const int r = 16 * nt + l16;
+  if (part == 0) {
+    for (int gi = w; gi < GI; gi += WPP) {
+      const int nt = gi / MT, mt = gi - nt * MT, r = 16 * nt + l16;
       float M = -INFINITY, L = 0.f;
       float4_t o = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int v = 0; v < HALF_WAVES; ++v) {
+      for (int v = 0; v < WPP; ++v) {
         float Mn, cM, cm;
         if (!fold_weights(M, red_m[v][r], Mn, cM, cm)) continue;
         L = fold_value(L, cM, red_l[v][r], cm);
@@ -774,9 +810,6 @@ attn_unit_half_kernel(AttnParams P) {
         for (int c = 0; c < 4; ++c) o[c] = fold_value(o[c], cM, a[c], cm);
         M = Mn;
       }
-      Mp[j] = M;
-      Lp[j] = L;
-      op[j] = o;
       st4_dev(scr, acc_at(0, gi), o);
       if (mt == 0 && g == 0) {
         st1_dev(scr, m_at(0, r), M);
@@ -784,76 +817,44 @@ attn_unit_half_kernel(AttnParams P) {
       }
     }
   } else {   // this wave's class partial, as the unit kernel's LDS holds it
+    const int slot = 1 + WPP * (part - 1) + w;
 #pragma unroll
-    for (int gi = 0; gi < 2 * MT; ++gi) st4_dev(scr, acc_at(1 + w, gi), red_acc[w][gi][lane]);
-    if (lane < QTILE) {
-      st1_dev(scr, m_at(1 + w, lane), red_m[w][lane]);
-      st1_dev(scr, l_at(1 + w, lane), red_l[w][lane]);
+    for (int gi = 0; gi < GI; ++gi) st4_dev(scr, acc_at(slot, gi), red_acc[w][gi][lane]);
+    if (lane < (TWO ? QTILE : 16)) {
+      st1_dev(scr, m_at(slot, lane), red_m[w][lane]);
+      st1_dev(scr, l_at(slot, lane), red_l[w][lane]);
     }
   }
   stores_done();
   __syncthreads();   // every wave's published values have completed
-  if (threadIdx.x == 0) sh_last = count_in(P.split_cnt + unit, 2u);
+  if (threadIdx.x == 0) sh_last = count_in(P.split_cnt + unit, (unsigned)PARTS);
   __syncthreads();
   if (!sh_last) return;
 
-  // the unit's second arrival: the fold continues through classes 4..7, then the rows are emitted
-  if (h == 0) {
-    float4_t a[NG][HALF_WAVES];   // every published value this wave needs, loaded at once
-    float m[NG][HALF_WAVES], l[NG][HALF_WAVES];
+  // the unit's last arrival: the prefix, then the remaining classes in order, then the rows. Every value a
+  // (half, dim tile) pair needs is loaded at once.
+  for (int gi = w; gi < GI; gi += WPP) {
+    const int nt = gi / MT, mt = gi - nt * MT, r = 16 * nt + l16;
+    float4_t a[NSLOT];
+    float m[NSLOT], l[NSLOT];
 #pragma unroll
-    for (int j = 0; j < NG; ++j) {
-      const int gi = w + HALF_WAVES * j, r = 16 * (gi / MT) + l16;
-#pragma unroll
-      for (int v = 0; v < HALF_WAVES; ++v) {
-        a[j][v] = ld4_dev(scr, acc_at(1 + v, gi));
-        m[j][v] = ld1_dev(scr, m_at(1 + v, r));
-        l[j][v] = ld1_dev(scr, l_at(1 + v, r));
-      }
+    for (int v = 0; v < NSLOT; ++v) {
+      a[v] = ld4_dev(scr, acc_at(v, gi));
+      m[v] = ld1_dev(scr, m_at(v, r));
+      l[v] = ld1_dev(scr, l_at(v, r));
     }
+    float M = m[0], L = l[0];
+    float4_t o = a[0];
 #pragma unroll
-    for (int j = 0; j < NG; ++j) {
-      const int gi = w + HALF_WAVES * j, nt = gi / MT, mt = gi - nt * MT;
-      const int r = 16 * nt + l16;
-      float M = Mp[j], L = Lp[j];
-      float4_t o = op[j];
+    for (int v = 1; v < NSLOT; ++v) {
+      float Mn, cM, cm;
+      if (!fold_weights(M, m[v], Mn, cM, cm)) continue;
+      L = fold_value(L, cM, l[v], cm);
 #pragma unroll
-      for (int v = 0; v < HALF_WAVES; ++v) {
-        float Mn, cM, cm;
-        if (!fold_weights(M, m[j][v], Mn, cM, cm)) continue;
-        L = fold_value(L, cM, l[j][v], cm);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) o[c] = fold_value(o[c], cM, a[j][v][c], cm);
-        M = Mn;
-      }
-      if (r < nrows) attn_emit<D>(P, b, s, kbeg, hkv, row0 + r, rpos[nt], mt, M, L, o);
+      for (int c = 0; c < 4; ++c) o[c] = fold_value(o[c], cM, a[v][c], cm);
+      M = Mn;
     }
-  } else {
-#pragma unroll
-    for (int j = 0; j < NG; ++j) {
-      const int gi = w + HALF_WAVES * j, r = 16 * (gi / MT) + l16;
-      Mp[j] = ld1_dev(scr, m_at(0, r));
-      Lp[j] = ld1_dev(scr, l_at(0, r));
-      op[j] = ld4_dev(scr, acc_at(0, gi));
-    }
-#pragma unroll
-    for (int j = 0; j < NG; ++j) {
-      const int gi = w + HALF_WAVES * j, nt = gi / MT, mt = gi - nt * MT;
-      const int r = 16 * nt + l16;
-      float M = Mp[j], L = Lp[j];
-      float4_t o = op[j];
-#pragma unroll
-      for (int v = 0; v < HALF_WAVES; ++v) {
-        float Mn, cM, cm;
-        if (!fold_weights(M, red_m[v][r], Mn, cM, cm)) continue;
-        L = fold_value(L, cM, red_l[v][r], cm);
-        const float4_t av = red_acc[v][gi][lane];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) o[c] = fold_value(o[c], cM, av[c], cm);
-        M = Mn;
-      }
-      if (r < nrows) attn_emit<D>(P, b, s, kbeg, hkv, row0 + r, rpos[nt], mt, M, L, o);
-    }
+    if (r < nrows) attn_emit<D>(P, b, s, kbeg, hkv, row0 + r, nt ? rpos[1] : rpos[0], mt, M, L, o);
   }
 }
 
@@ -1125,7 +1126,7 @@ attn_prefill_kernel(AttnParams P) {
       for (int mt = 0; mt < MT; ++mt) vf[mt] = *(LdsV*)(uintptr_t)(vad + (uint32_t)(u * TB + mt * 16 * 32));
       const int key0 = kbeg + 16 * t;
       const bool tv = all_mapped || tbl[key0 / BS - blk0] >= 0;
-      attn_tile<D, true, true>(kf, vf, key0, tv, qmax, rpos, rmin, two, qf, P.scale_log2, acc, m_run, l_run);
+      attn_tile<D, true, true, true>(kf, vf, key0, tv, qmax, rpos, rmin, two, qf, P.scale_log2, acc, m_run, l_run);
     }
   }
   if (nrows <= 0) return;
@@ -1342,6 +1343,18 @@ int64_t split_bytes(int64_t units, int32_t head_dim) {
          (int64_t)sizeof(float);
 }
 
+// Workgroups per unit of a call of at most `units` units whose tables hold `keys` keys; two: its tiles have a
+// second half of query rows (twice the partials to exchange). Measured (us: one, two and four workgroups a
+// unit; 32/8 heads, 128 dims unless said): 24 units of 8000-30000 keys, T = 1: 159 / 95 / 63; 8 of 1000: 14.6 /
+// 12.0 / 13.9; 32 of 500-2000: 23.3 / 17.4 / 16.3; 64 of 512-4096: 61 / 38 / 29; 128 of them: 46.7 / 39.8 / 41.6;
+// 128 of 128-1280 keys, 64 dims: 15.2 / 12.6 / 13.4. With two halves (T = 5): 64 of 512-4096: 64 / 43 / 38; 128 of
+// them: 49.6 / 44.9 / 50.8; 16 of 2000-6000: 58 / 39 / 40; 128 of 1000-3000 keys, 64 dims: 21.2 / 22.1 / 24.5; 8 of
+// 500, 64 dims: 10.3 / 11.1 / 13.7. 256 units of 512-4096 keys in two: 61 -> 69.
+int split_parts(int64_t units, int64_t keys, bool two) {
+  if (units > SPLIT_UNITS_MAX || keys < (two ? 3072 : 768)) return 1;
+  return units <= SPLIT_UNITS_MAX / 2 && keys >= (two ? 4096 : 2048) ? 4 : 2;
+}
+
 }  // namespace
 
 extern "C" int32_t fs_paged_attention_split(void) { return attn_split(); }
@@ -1470,25 +1483,28 @@ int paged_attention(const void* q, int64_t q_sb, int64_t q_st, int64_t q_sh, con
         if (bs16) attn_prefill_kernel<64, 16><<<grid, threads, 0, st>>>(P);
         else attn_prefill_kernel<64, 0><<<grid, threads, 0, st>>>(P);
       }
-    } else if (units <= SPLIT_UNITS_MAX && (int64_t)max_blocks * kv->block_size >= SPLIT_MIN_KEYS) {
-      // few, possibly long units: two workgroups each, to keep more CUs reading
-      const unsigned threads = 64 * HALF_WAVES;
-      if (kv->head_dim == 128) {
-        if (bs16) attn_unit_half_kernel<128, 16><<<2 * grid, threads, 0, st>>>(P);
-        else attn_unit_half_kernel<128, 0><<<2 * grid, threads, 0, st>>>(P);
-      } else {
-        if (bs16) attn_unit_half_kernel<64, 16><<<2 * grid, threads, 0, st>>>(P);
-        else attn_unit_half_kernel<64, 0><<<2 * grid, threads, 0, st>>>(P);
-      }
     } else {
-      const unsigned threads = 64 * UNIT_WAVES;
-      if (kv->head_dim == 128) {
-        if (bs16) attn_unit_kernel<128, 16><<<grid, threads, 0, st>>>(P);
-        else attn_unit_kernel<128, 0><<<grid, threads, 0, st>>>(P);
-      } else {
-        if (bs16) attn_unit_kernel<64, 16><<<grid, threads, 0, st>>>(P);
-        else attn_unit_kernel<64, 0><<<grid, threads, 0, st>>>(P);
-      }
+      // few, possibly long units: several workgroups each, to keep more CUs reading
+      const bool two = (int64_t)T * P.G > 16;   // else no tile has a second half of query rows
+      const int parts = split_parts(units, (int64_t)max_blocks * kv->block_size, two);
+      const unsigned pgrid = grid * (unsigned)parts, pthreads = 64 * UNIT_WAVES / (unsigned)parts;
+#define FS_ATTN_LAUNCH(D_, BS_, TWO_)                                                     \
+  do {                                                                                    \
+    if (parts == 4) attn_unit_part_kernel<D_, BS_, TWO_, 4><<<pgrid, pthreads, 0, st>>>(P); \
+    else if (parts == 2) attn_unit_part_kernel<D_, BS_, TWO_, 2><<<pgrid, pthreads, 0, st>>>(P); \
+    else attn_unit_kernel<D_, BS_, TWO_><<<grid, 64 * UNIT_WAVES, 0, st>>>(P);                   \
+  } while (0)
+#define FS_ATTN_LAUNCH_D(D_)                                                              \
+  do {                                                                                    \
+    if (bs16 && two) FS_ATTN_LAUNCH(D_, 16, true);                                        \
+    else if (bs16) FS_ATTN_LAUNCH(D_, 16, false);                                         \
+    else if (two) FS_ATTN_LAUNCH(D_, 0, true);                                            \
+    else FS_ATTN_LAUNCH(D_, 0, false);                                                    \
+  } while (0)
+      if (kv->head_dim == 128) FS_ATTN_LAUNCH_D(128);
+      else FS_ATTN_LAUNCH_D(64);
+#undef FS_ATTN_LAUNCH_D
+#undef FS_ATTN_LAUNCH
     }
   } else {
     last_plan = PlanKey{};   // no plan on this path

@@ -575,6 +575,39 @@ def test_attention_split_units_equal_unit_kernel_bitwise(d, g, bs, t, b, lo_ctx,
     assert rel_err(full[2:8].float(), ref) < 2e-2
 
 
+@pytest.mark.parametrize("d,g,bs,t,hi_ctx", [(128, 4, 16, 1, 4100), (128, 4, 16, 4, 900), (64, 8, 32, 2, 2100),
+                                             (128, 2, 48, 9, 4200), (64, 4, 16, 7, 5000), (128, 1, 16, 1, 17000)])
+def test_attention_unit_parts_equal_unit_kernel_bitwise(d, g, bs, t, hi_ctx):
+    """A unit's keys run in one workgroup, in two or in four, by the number of units and the table's width,
+    with one half of query rows (t * g <= 16) or two: the rows of one call of 140, recomputed in calls that
+    take each way, give identical bits, contexts of 1 key, of whole tiles and of a few tiles among them,
+    padding queries and an unmapped block too."""
+    case("attention unit parts", d, g, bs, t, hi_ctx)
+    hkv, b = 2, 140
+    gen = torch.Generator().manual_seed(d + g + t + hi_ctx)
+    ctx = torch.randint(t, hi_ctx + 1, (b,), generator=gen)
+    ctx[:8] = torch.tensor([hi_ctx, t, 16, 17, 128, 129, 500, hi_ctx - 1]).clamp(min=t, max=hi_ctx)
+    maxb = -(-hi_ctx // bs)
+    nblocks = maxb + 5
+    tables = torch.randint(0, nblocks, (b, maxb), generator=gen)
+    k = torch.randn(nblocks, hkv, bs, d, generator=gen).bfloat16()
+    v = torch.randn(nblocks, hkv, bs, d, generator=gen).bfloat16()
+    q = torch.randn(b, t, hkv * g, d, generator=gen).bfloat16()
+    pos = ctx[:, None] - t + torch.arange(t)[None, :]
+    pos[3, 0] = -1   # a padding query
+    _, pool = _run_attention(q[:1], k, v, tables[:1], pos[:1], torch.bfloat16, bs)
+    tables[6, 2] = -1   # an unmapped block: its keys are masked
+    qd, lay, tab, pd = q.to(DEV), pool.layout(0), tables.int().to(DEV), pos.int().to(DEV)
+    run = lambda lo, hi: ops.paged_attention(qd[lo:hi], lay, tab[lo:hi].contiguous(), pd[lo:hi].contiguous(), d ** -0.5)
+    full = run(0, b)
+    units = (-(-t * g // 32)) * (-(-maxb * bs // _lib.load().fs_paged_attention_split())) * hkv   # of one row
+    for rows in (1, 8, max(1, 64 // units), max(1, 128 // units)):
+        for lo in (0, 5, b - rows):
+            assert torch.equal(run(lo, lo + rows), full[lo: lo + rows]), (rows, lo)
+    ref = _oracle_attention(q[:3], k, v, tables[:3], pos[:3], g)
+    assert rel_err(full[:3].float().cpu(), ref) < 2e-2
+
+
 def test_attention_split_units_replayed_from_a_graph():
     """The split-unit kernel captured in a HIP graph: each replay, with new queries copied in and other
     attention calls run eagerly between replays, gives the eager call's bits (the arrival counters
