@@ -4,8 +4,8 @@
 // Reference: paged.py:80-81 (gather every table block) + model.py:70-76 (repeat_interleave GQA,
 // key_pos <= query_pos mask, scaled_dot_product_attention with scale 1/sqrt(D)).
 //
-// Work split (both kernels): the keys of a row are cut into fixed chunks of `split` absolute positions
-// (512 for the generic kernel, FS_ATTN_SPLIT (default 16384) for the MFMA kernels; fixed for the life
+// Work split (all kernels): the keys of a row are cut into fixed chunks of `split` absolute positions
+// (512 for the float32 and generic kernels, FS_ATTN_SPLIT (default 16384) for the MFMA kernels; fixed for the life
 // of the process); chunk s covers keys
 // [s*split, (s+1)*split). Each workgroup produces the softmax partial
 // (running max m, sum l, unnormalised output acc) of its chunk, and attn_combine merges the chunks of
@@ -21,6 +21,8 @@
 //   O^T[dim, row] += V^T . P^T v_mfma_f32_16x16x16_bf16, A = 16 dims x 4 keys of the dim-major tile
 // With the transposed products every lane owns whole query rows (row = lane % 16), so the softmax
 // statistics, the P operand and the O rescale stay in the lane's own registers.
+// float32 in such a layout takes the same products on v_mfma_f32_16x16x4_f32; any other type or layout the
+// scalar kernel.
 #include <math.h>
 #include <stdlib.h>
 
@@ -1222,6 +1224,190 @@ __global__ void __launch_bounds__(64) attn_generic_kernel(AttnParams P) {
 }
 
 // ------------------------------------------------------------------------------------------------
+// float32 kernel: one wave per (batch row, KV head, 16 query rows, chunk of GENERIC_SPLIT keys)
+// ------------------------------------------------------------------------------------------------
+// The bf16 kernels' transposed products on v_mfma_f32_16x16x4_f32, nothing rounded below float32: 16-key
+// tiles, lane group g holding dims 16s + 4g .. +3 of a key (one 16-byte load), so four instructions add 16 dims;
+// S^T leaves lane (l16, g) with row l16's scores of keys 4g .. 4g+3, which are the keys it reads 16 bytes of
+// per dim of the dim-major values. Dims past head_dim are zeros. A tile's keys and values are loaded while
+// the one before is multiplied. A query's result depends on its own position only: a row's tiles run in
+// order, a tile above its position leaves its state as it is, chunks are merged by attn_combine.
+//
+// Latency-bound at the sizes float32 models have (a few waves of a few tiles each). The scalar kernel below
+// walked 64 keys per step with a lane per key and then a lane per dim. One row of a token at position 100 (8/4
+// heads of 32 dims): 30 -> 12 us; four rows of 160 tokens: 83 -> 18 us.
+constexpr int F32_ROWS = 16;
+
+template <int S>   // 16-dim groups: head_dim <= 16 S
+__global__ void __launch_bounds__(64) attn_f32_kernel(AttnParams P) {
+  const int lane = threadIdx.x, l16 = lane & 15, g = lane >> 4;
+  const int nkv = P.kv.n_kv_heads, D = P.kv.head_dim, BS = P.kv.block_size;
+  const int qtiles = (P.T * P.G + F32_ROWS - 1) / F32_ROWS;
+  const int hkv = (int)(blockIdx.x % nkv);
+  const int bz = (int)(blockIdx.x / nkv);
+  const int b = bz / qtiles, row0 = (bz - b * qtiles) * F32_ROWS;
+  const int s = blockIdx.y;
+  const int kbeg = s * P.split;
+  const int qmax = rows_qmax(P, b, row0, F32_ROWS);
+  if (qmax < kbeg && s > 0) return;
+  const int kend = min(kbeg + P.split, qmax + 1);
+  const int r = row0 + l16;
+  const bool in = r < P.T * P.G;
+  const int t = in ? r / P.G : 0, h = hkv * P.G + (in ? r - t * P.G : 0);
+  const bool exists = in && token_exists(P, b, t);
+  const int pos = in ? P.pos[(int64_t)b * P.T + t] : -1;
+
+  int rmin = in ? pos : 0x7fffffff;   // the smallest position of the 16 rows
+#pragma unroll
+  for (int o = 1; o < 16; o <<= 1) rmin = min(rmin, __shfl_xor(rmin, o, 64));
+
+  const float4_t zero = float4_t{0.f, 0.f, 0.f, 0.f};
+  const float* qr = reinterpret_cast<const float*>(P.q) + (exists ? q_offset(P, b, t) + (int64_t)h * P.q_sh : 0);
+  float4_t qf[S];
+#pragma unroll
+  for (int i = 0; i < S; ++i) qf[i] = exists && 16 * i + 4 * g < D ? *reinterpret_cast<const float4_t*>(qr + 16 * i + 4 * g) : zero;
+
+  const float* kp = reinterpret_cast<const float*>(P.kv.k) + (int64_t)hkv * P.kv.k_head;
+  const float* vp = reinterpret_cast<const float*>(P.kv.v) + (int64_t)hkv * P.kv.v_head;
+  const int32_t* trow = P.table + (int64_t)b * P.table_stride;
+  const int shift = (BS & (BS - 1)) == 0 ? 31 - __clz(BS) : -1;
+  auto block_index = [&](int j) { return shift >= 0 ? j >> shift : j / BS; };
+  // block of key j, -1 when past the chunk's keys or unmapped
+  auto block_of = [&](int j) {
+    const int bi = block_index(j);
+    const int v = j < kend && bi < P.max_blocks ? trow[bi] : -1;
+    return v >= 0 && v < P.kv.num_blocks ? v : -1;
+  };
+  // A tile: lane (l16, g) holds dims 16i + 4g .. of key j0 + l16, and keys j0 + 4g .. of dim 16i + l16 (block_size
+  // % 4 == 0: the four share a block); `ok` has a bit per key of its four that may be used
+  struct Tile {
+    float4_t k[S], v[S];
+    int ok;
+  };
+  auto load = [&](Tile& x, int j0) {
+    const int jk = j0 + l16, bk = block_of(jk), jv = j0 + 4 * g, bv = block_of(jv);
+    const float* kr = kp + (bk < 0 ? 0 : bk * P.kv.k_block + (int64_t)(jk - block_index(jk) * BS) * P.kv.k_slot);
+    const float* vr = vp + (bv < 0 ? 0 : bv * P.kv.v_block + (int64_t)(jv - block_index(jv) * BS));
+    x.ok = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (bv >= 0 && jv + e < kend) x.ok |= 1 << e;
+#pragma unroll
+    for (int i = 0; i < S; ++i) {
+      x.k[i] = bk >= 0 && 16 * i + 4 * g < D ? *reinterpret_cast<const float4_t*>(kr + key_dim_off(P.kv, 16 * i + 4 * g)) : zero;
+      x.v[i] = bv >= 0 && 16 * i + l16 < D ? *reinterpret_cast<const float4_t*>(vr + (16 * i + l16) * P.kv.v_dim) : zero;
+    }
+  };
+
+  float4_t acc[S];
+#pragma unroll
+  for (int i = 0; i < S; ++i) acc[i] = zero;
+  float m_run = -INFINITY, l_run = 0.f;
+  auto consume = [&](const Tile& x, int j0) {
+    float4_t sc = zero;
+#pragma unroll
+    for (int i = 0; i < S; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sc = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[i][e], qf[i][e], sc, 0, 0, 0);
+    float sv[4], tmax = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      sv[e] = (x.ok >> e & 1) && j0 + 4 * g + e <= pos ? sc[e] * P.scale_log2 : -INFINITY;
+      tmax = fmaxf(tmax, sv[e]);
+    }
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    const float m_new = fmaxf(m_run, tmax);
+    const float alpha = m_new == -INFINITY ? 1.f : exp2f(m_run - m_new);
+    float p[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) p[e] = sv[e] == -INFINITY ? 0.f : exp2f(sv[e] - m_new);
+    l_run = l_run * alpha + ((p[0] + p[1]) + (p[2] + p[3]));   // this lane group's keys
+    m_run = m_new;
+#pragma unroll
+    for (int i = 0; i < S; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[i][e] *= alpha;
+    // A key that a row may not see has weight 0 there, which an infinite or NaN value would turn into NaN:
+    // in a tile that some row sees only in part, such values take the products key by key.
+    float4_t v[S];
+    float bad = 0.f;
+#pragma unroll
+    for (int i = 0; i < S; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {   // (a value never written may be anything)
+        v[i][e] = x.ok >> e & 1 ? x.v[i][e] : 0.f;
+        bad = fmaf(v[i][e], 0.f, bad);
+      }
+    if (j0 + 15 > rmin && __any(bad != 0.f)) {
+      for (int j = 0; j < 16; ++j) {
+        const int src = (j >> 2) * 16;   // the lane group that holds key j's weights and values
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (e != (j & 3)) continue;
+          const float pj = __shfl(p[e], src + l16, 64);
+#pragma unroll
+          for (int i = 0; i < S; ++i)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+              const float vj = __shfl(v[i][e], src + 4 * g + c, 64);   // dim 16i + 4g + c
+              if (pj != 0.f) acc[i][c] = fmaf(pj, vj, acc[i][c]);
+            }
+        }
+      }
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < S; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i][e], p[e], acc[i], 0, 0, 0);
+  };
+
+  Tile a, c;
+  if (kbeg < kend) load(a, kbeg);
+  for (int j0 = kbeg; j0 < kend; j0 += 32) {
+    if (j0 + 16 < kend) load(c, j0 + 16);
+    consume(a, j0);
+    if (j0 + 32 < kend) load(a, j0 + 32);
+    if (j0 + 16 < kend) consume(c, j0 + 16);
+  }
+  // (g0 + g1) + (g2 + g3) in every lane
+  float l = l_run + __shfl_xor(l_run, 16, 64);
+  l = l + __shfl_xor(l, 32, 64);
+
+  // acc[i]: lane (l16, g) has row l16's dims 16i + 4g .. +3
+  if (!in) return;
+  if (P.nsplit == 1) {   // one chunk: the same division as attn_combine's (a padding query, pos < 0, gives zeros)
+    if (!exists) return;
+    float* orow = reinterpret_cast<float*>(P.out) + o_offset(P, b, t, P.o_sb, P.o_st) + (int64_t)h * P.o_sh;
+#pragma unroll
+    for (int i = 0; i < S; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (16 * i + 4 * g + e < D) orow[16 * i + 4 * g + e] = l > 0.f ? acc[i][e] / l : 0.f;
+    return;
+  }
+  if (pos < kbeg) return;   // attn_combine reads the chunks that hold keys a query sees
+  const int64_t R = row_index(P, b, t, h);
+#pragma unroll
+  for (int i = 0; i < S; ++i)
+    if (16 * i + 4 * g < D) *reinterpret_cast<float4_t*>(P.ws_acc + (R * P.nsplit + s) * D + 16 * i + 4 * g) = acc[i];
+  if (g == 0) {
+    float* pm = P.ws_ml + (R * P.nsplit + s) * 2;
+    pm[0] = m_run;
+    pm[1] = l;
+  }
+}
+
+// Whole 16-byte pieces of queries, keys and values, head_dim <= 128, four consecutive keys in one block.
+bool f32_eligible(const fs_kv_layout& kv, const void* q, int64_t q_sb, int64_t q_st, int64_t q_sh) {
+  if (kv.dtype != FS_F32 || kv.head_dim % 4 || kv.head_dim > 128 || kv.block_size % 4) return false;
+  if (kv.k_dim != 1 || kv.v_slot != 1) return false;
+  if ((kv.k_block | kv.k_head | kv.k_slot | kv.k_group | kv.v_block | kv.v_head | kv.v_dim | q_sb | q_st | q_sh) & 3) return false;
+  return ((reinterpret_cast<uintptr_t>(kv.k) | reinterpret_cast<uintptr_t>(kv.v) | reinterpret_cast<uintptr_t>(q)) & 15) == 0;
+}
+
+// ------------------------------------------------------------------------------------------------
 // combine: out[b,t,h,:] = sum_s 2^(m_s - M) acc_s / sum_s 2^(m_s - M) l_s, chunks in increasing order
 // ------------------------------------------------------------------------------------------------
 constexpr int COMBINE_ROWS = 4;   // rows (waves) per combine workgroup
@@ -1509,7 +1695,17 @@ int paged_attention(const void* q, int64_t q_sb, int64_t q_st, int64_t q_sh, con
   } else {
     last_plan = PlanKey{};   // no plan on this path
     dim3 grid((unsigned)rows, (unsigned)P.nsplit);
-    switch (kv->dtype) {
+    if (f32_eligible(*kv, q, q_sb, q_st, q_sh)) {
+      const int64_t tiles = (int64_t)B * (((int64_t)T * P.G + F32_ROWS - 1) / F32_ROWS) * kv->n_kv_heads;
+      FS_CHECK_ARG(tiles < 0x7fffffff, "paged_attention: %lld work units", (long long)tiles);
+      const dim3 fgrid((unsigned)tiles, (unsigned)P.nsplit);
+      if (kv->head_dim <= 16) attn_f32_kernel<1><<<fgrid, 64, 0, st>>>(P);
+      else if (kv->head_dim <= 32) attn_f32_kernel<2><<<fgrid, 64, 0, st>>>(P);
+      else if (kv->head_dim <= 64) attn_f32_kernel<4><<<fgrid, 64, 0, st>>>(P);
+      else attn_f32_kernel<8><<<fgrid, 64, 0, st>>>(P);
+      if (int e = fs::launch_status("paged_attention")) return e;
+      if (P.nsplit == 1) return 0;   // every output is written
+    } else switch (kv->dtype) {
       case FS_F32: attn_generic_kernel<FS_F32><<<grid, 64, 0, st>>>(P); break;
       case FS_BF16: attn_generic_kernel<FS_BF16><<<grid, 64, 0, st>>>(P); break;
       default: attn_generic_kernel<FS_F16><<<grid, 64, 0, st>>>(P); break;

@@ -437,6 +437,40 @@ def test_attention_generic_f32(d, bs, t):
     torch.testing.assert_close(out.cpu(), ref, atol=1e-5, rtol=1e-5)
 
 
+@pytest.mark.parametrize("d,bs,t,g,layout", [(4, 4, 1, 1, "slots"), (8, 8, 5, 2, "groups"), (20, 16, 3, 4, "slots"),
+                                             (32, 16, 9, 2, "groups"), (36, 12, 17, 1, "slots"), (64, 48, 5, 8, "groups"),
+                                             (100, 16, 2, 3, "slots"), (128, 16, 4, 4, "groups")])
+def test_attention_f32_tiles(d, bs, t, g, layout):
+    """The float32 attention at the edges of its 16-dim groups, 16-key tiles, 16-row tiles and 512-key chunks, both
+    key layouts, with padding queries and an unmapped block: against the oracle, and each query's bits the same
+    alone as in its window. An infinite value at a later position leaves the earlier queries as they are."""
+    case("attention f32 tiles", d, bs, t, g, layout)
+    ctx = [t, 16, 17, 33, 500, 512, 513, 1100]
+    ctx = [max(c, t) for c in ctx]
+    b, hkv = len(ctx), 2
+    q, k, v, tables, pos = _paged_case(b, t, hkv * g, hkv, d, bs, ctx, sum(-(-c // bs) for c in ctx) + 3, torch.float32, d + bs)
+    out, pool = _run_attention(q, k, v, tables, pos, torch.float32, bs, layout)
+    torch.testing.assert_close(out.cpu(), _oracle_attention(q, k, v, tables, pos, g), atol=2e-6, rtol=2e-5)
+    lay, tab, qd, pd = pool.layout(0), tables.int().to(DEV), q.to(DEV), pos.int().to(DEV)
+    run = lambda q_, tab_, pos_: ops.paged_attention(q_, lay, tab_, pos_, 1.0 / math.sqrt(d))
+    for i in range(t):
+        assert torch.equal(run(qd[:, i: i + 1].contiguous(), tab, pd[:, i: i + 1].contiguous())[:, 0], out[:, i]), i
+    narrow = tab[:4, : -(-max(ctx[:4]) // bs)].contiguous()   # a table of one chunk: written without the merge
+    assert torch.equal(run(qd[:4], narrow, pd[:4].contiguous()), out[:4])
+    hole = tab.clone()
+    hole[7, 1] = -1
+    hp = pd.clone()
+    hp[2, 0] = -1   # a padding query: zeros
+    got = run(qd, hole, hp)
+    assert torch.count_nonzero(got[2, 0]) == 0 and torch.equal(got[:2], out[:2]) and not torch.equal(got[7], out[7])
+    if t > 1:
+        last = int(pos[4, -1])
+        pool.v[0][int(tables[4, last // bs]), :, last % bs] = float("inf")
+        got = run(qd, tab, pd)
+        assert torch.isfinite(got[4, :-1]).all() and not torch.isfinite(got[4, -1]).any()
+        torch.testing.assert_close(got[4, :-1], out[4, :-1], atol=2e-6, rtol=2e-5)
+
+
 @pytest.mark.parametrize("d,t,g", [(128, 5, 4), (128, 7, 4), (64, 5, 4), (128, 1, 4), (128, 9, 4), (64, 3, 8)])
 def test_attention_mfma_bf16(d, t, g):
     case("attention bf16 mfma", d, t, g)
