@@ -18,7 +18,7 @@
 // dim-major values): one wavefront per (chunk, batch row, kv head, 32-row query tile). The query
 // tile is the (token, group-head) pairs of one KV head: rows = T * (n_heads / n_kv_heads).
 //   S^T[key, row] = K . Q^T    v_mfma_f32_16x16x32_bf16, A = 16 keys x 32 dims straight from HBM
-//   O^T[dim, row] += V^T . P^T v_mfma_f32_16x16x16_bf16, A = 16 dims x 4 keys of the dim-major tile
+//   O^T[dim, row] += V^T . P^T v_mfma_f32_16x16x32_bf16, A = 16 dims x 4 keys of each tile of a pair
 // With the transposed products every lane owns whole query rows (row = lane % 16), so the softmax
 // statistics, the P operand and the O rescale stay in the lane's own registers.
 // float32 in such a layout takes the same products on v_mfma_f32_16x16x4_f32; any other type or layout the
@@ -38,6 +38,7 @@ constexpr int SPLIT_UNITS_MAX = 128;  // calls with at most this many units (hal
 constexpr int64_t WS_COUNTERS = 256;
 constexpr int64_t WS_HEADER = WS_COUNTERS + 4 * SPLIT_UNITS_MAX;
 constexpr float LOG2E = 1.4426950408889634f;
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 struct AttnParams {
   const void* q;
@@ -158,8 +159,8 @@ constexpr int SPLIT_SLOTS = 7;                  // published partials per split 
 // floats of one published partial: m and l of the 32 rows, then acc as the LDS holds it (2 * D/16
 // (half, dim tile) pairs, 64 lanes, 4 values)
 constexpr int64_t split_slot_floats(int D) { return 2 * QTILE + (int64_t)QTILE * D; }
-constexpr int MAX_SPLIT = 2 * 64 * 16 * UNIT_WAVES;   // keys per chunk, at most: a wave's tiles fit two
-                                                       // table entries per lane
+constexpr int MAX_SPLIT = 2 * 64 * 16 * UNIT_WAVES;   // keys per chunk, at most: a wave's pairs fit one
+                                                       // lane each
 
 // One workgroup lists every item: first the chunks that lie wholly below their tile's furthest
 // query (the full chunks), tile by tile, then the last chunk of each tile, longest first. Workgroups
@@ -293,28 +294,12 @@ __global__ void __launch_bounds__(PLAN_THREADS) attn_plan_kernel(AttnParams P) {
 // ------------------------------------------------------------------------------------------------
 // unit kernel: one workgroup of UNIT_WAVES waves per (plan item, KV head)
 // ------------------------------------------------------------------------------------------------
-// The item's keys [kbeg, kend) are cut into 16-key tiles; wave w takes tiles w, w + UNIT_WAVES, ...
+// The item's keys [kbeg, kend) are cut into pairs of 16-key tiles; wave w takes pairs w, w + UNIT_WAVES, ...
 // in increasing order and keeps its own softmax partial, and the waves' partials are merged through
-// LDS in wave order. Which tiles a wave sees, and in what order, depends only on absolute key
-// positions, and a tile wholly above a query's position leaves that query's partial exactly as it
+// LDS in wave order. Which pairs a wave sees, and in what order, depends only on absolute key
+// positions, and a pair wholly above a query's position leaves that query's partial exactly as it
 // was; a query's result therefore does not depend on the other queries of its tile.
 
-// One 16-key tile into a wave's online-softmax partial of up to 32 query rows (two 16-row halves; the
-// second only when `two`). kf holds the tile's keys as A operands of S^T = K.Q^T, vf its values as A
-// operands of O^T += V^T.P^T (zeroed in place where a key must not reach the product: an unmapped
-// block, or a key past qmax, the furthest query of the 32 rows, which may never have been written).
-// j0 is the tile's first key, rpos the positions of the lane's two rows (-1: no query), rmin the
-// smallest position over all 32 rows (-1 if any row is missing). A key above a row's position gets
-// score -inf.
-//
-// The partial is (m, l, acc) with p = 2^(s - m): m is a reference maximum that moves only when a
-// tile's maximum exceeds it by more than 8 (then to that maximum, and acc and l are rescaled), so
-// p <= 2^8 and the rescale is rare once a row has seen a few tiles. A tile wholly above a row leaves
-// that row's partial exactly as it was (m unchanged, alpha = 1, p = 0). A tile whose keys every row
-// sees takes a path without the per-key masks; its arithmetic is the same. LAZY skips the rescale
-// when no row of the wave moved (multiplying by alpha = 1 is exact, so the bits do not change). Every
-// kernel that builds a partial calls this function, so a row's partial does not depend on which
-// kernel ran it.
 // Smallest position over the rows r < nrows of a wave's 32-row tile (-1 if nrows <= 0); the rows of
 // lane l16 are l16 and 16 + l16, whose positions are rpos[0] and rpos[1].
 FS_DEVICE int rows_min_pos(const int (&rpos)[2], int nrows) {
@@ -326,146 +311,176 @@ FS_DEVICE int rows_min_pos(const int (&rpos)[2], int nrows) {
   return __builtin_amdgcn_readfirstlane(v);
 }
 
-constexpr float REF_SLACK = 8.f;   // log2 units a tile's maximum may exceed the reference by
+constexpr float REF_SLACK = 8.f;   // log2 units a pair's maximum may exceed the reference by
 
-// The softmax step of one tile for the lane's two rows: scores in log2 units (a key the row may not
-// see gets -inf; FULL: every row sees every key), the tile's row maxima, the references (a row's m
-// moves to the tile's maximum when that exceeds m by more than REF_SLACK), p = 2^(s - m) as bf16
-// MFMA operands, and l <- l * alpha + (the lane's sum of p), alpha = 2^(m_old - m_new) for a row
-// that moved, else 1. Returns whether any row of the wave moved; alpha is for the caller's rescale
-// of acc. LAZY: when no row moved, l <- l + sum, which is l * 1 + sum bit for bit.
-template <bool FULL, bool LAZY, bool TWO>
-FS_DEVICE bool tile_probs(const float4_t (&sc)[2], int j0, bool tile_valid, const int (&rpos)[2], float scale_log2,
-                          float (&m_run)[2], float (&l_run)[2], float (&alpha)[2], short4_t (&pf)[2]) {
+// A pair of 16-key tiles (32 keys from j0 on) into a wave's online-softmax partial of up to 32 query rows (two
+// 16-row halves; TWO: the second too, whatever rows of it exist), in two steps: the scores S^T = K.Q^T, tile
+// by tile, and pair_step. The pair is one k = 32 product O^T += V^T.P^T: in the operands lane group g's eight k
+// slots are keys 4g .. 4g+3 of the first tile, then of the second, so its probabilities (the S^T accumulators)
+// and its values (8 bytes per dim and tile) lie in the lane as the product wants them. One product of 32 keys
+// costs what one of 16 does, and the softmax's reductions and branches are paid once per 32 keys.
+//
+// ok: whether each tile is there (a mapped block, a tile the chunk has); fresh: acc is all zeros; rpos: the
+// positions of the lane's two rows (-1: no query), rmin the smallest position over all 32 rows (-1 if any row
+// is missing), qmax the furthest. A key above a row's position gets score -inf; values that must not reach the
+// product (an absent tile, or a key past qmax, which may never have been written) are zeroed.
+//
+// The partial is (m, l, acc) with p = 2^(s - m): m is a reference maximum that moves only when a pair's
+// maximum exceeds it by more than 8 (then to that maximum, and acc and l are rescaled), so p <= 2^8 and the
+// rescale is rare once a row has seen a few pairs. A pair wholly above a row leaves that row's partial
+// exactly as it was (m unchanged, alpha = 1, p = 0), and the part of a pair above it counts as exact zeros.
+// A pair whose keys every row sees takes a path without the per-key masks; its arithmetic is the same. Every
+// kernel that builds a partial calls these functions, so a row's partial does not depend on which kernel
+// ran it.
+template <int D, bool TWO>
+FS_DEVICE void tile_scores(const bf16x8_t (&kf)[D / 32], const bf16x8_t (&qf)[2][D / 32], float4_t (&sc)[2]) {
+  constexpr int KS = D / 32;
+  sc[0] = float4_t{0.f, 0.f, 0.f, 0.f};
+  sc[1] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    sc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks], qf[0][ks], sc[0], 0, 0, 0);
+    if (TWO) sc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks], qf[1][ks], sc[1], 0, 0, 0);
+  }
+}
+
+// Queries whose scale is negative are negated as they are loaded, and zeroed where it is 0 (both exact), so
+// scores are scaled by a positive number: a maximum commutes with it, and a masked score stays -inf.
+FS_DEVICE bf16x8_t signed_query(bf16x8_t q, float scale_log2) {
+  const unsigned flip = scale_log2 < 0.f ? 0x80008000u : 0u, keep = scale_log2 == 0.f ? 0u : ~0u;
+  return __builtin_bit_cast(bf16x8_t, (__builtin_bit_cast(u32x4, q) ^ flip) & keep);
+}
+FS_DEVICE float positive_scale(float scale_log2) { return scale_log2 == 0.f ? 1.f : fabsf(scale_log2); }
+
+// The softmax step of one pair for the lane's two rows: the references, p = 2^(s - m) as bf16 operands, and
+// l <- l * alpha + (the lane's sum of p), alpha = 2^(m_old - m_new) for a row that moved, else 1. Returns
+// whether any row of the wave moved; alpha is for the caller's rescale of acc.
+template <bool TWO>
+FS_DEVICE bool pair_probs(const float (&sc)[2][2][4], float scale, float (&m_run)[2], float (&l_run)[2], float (&alpha)[2],
+                          bf16x8_t (&pf)[2]) {
   constexpr int NT = TWO ? 2 : 1;
-  const int g = (threadIdx.x & 63) >> 4;
-  float sv[2][4], x[2];
+  float x[2];   // the lane's largest score of each row, unscaled
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
+    float a[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float v = sc[nt][e] * scale_log2;
-      sv[nt][e] = (FULL || (tile_valid && j0 + 4 * g + e <= rpos[nt])) ? v : -INFINITY;
-    }
-    x[nt] = __builtin_elementwise_maximum(__builtin_elementwise_maximum(sv[nt][0], sv[nt][1]),
-                                          __builtin_elementwise_maximum(sv[nt][2], sv[nt][3]));
+    for (int e = 0; e < 4; ++e) a[e] = __builtin_elementwise_maximum(sc[0][nt][e], sc[1][nt][e]);
+    x[nt] = __builtin_elementwise_maximum(__builtin_elementwise_maximum(a[0], a[1]), __builtin_elementwise_maximum(a[2], a[3]));
   }
-  // A row's tile maximum exceeds m + REF_SLACK exactly when one of its four lane groups' maxima does.
-  // LAZY: when no lane's does, no row moves (m_new = m, alpha = 1), and the reduction across the lane
-  // groups is skipped: the same values as the path below.
-  if (LAZY && !__any(x[0] > m_run[0] + REF_SLACK || (TWO && x[1] > m_run[1] + REF_SLACK))) {
+  auto probs = [&](int nt, float m) {   // the lane's p of a row, into pf; returns their sum
+    const float ref = m == -INFINITY ? 0.f : m;   // (a row that has seen nothing yet: every p is 0)
+    float pv[2][4];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pv[u][e] = fast_exp2(fmaf(sc[u][nt][e], scale, -ref));
+    struct Halves { short4_t a, b; } h = {bf16_rne4(pv[0]), bf16_rne4(pv[1])};
+    pf[nt] = __builtin_bit_cast(bf16x8_t, h);
+    return ((pv[0][0] + pv[0][1]) + (pv[0][2] + pv[0][3])) + ((pv[1][0] + pv[1][1]) + (pv[1][2] + pv[1][3]));
+  };
+  // A row's maximum exceeds m + REF_SLACK exactly when one of its four lane groups' maxima does. When no
+  // lane's does, no row moves (m_new = m, alpha = 1), and the reduction across the lane groups is skipped.
+    const bool moved = __any(x[0] * scale > m_run[0] + REF_SLACK || (TWO && x[1] * scale > m_run[1] + REF_SLACK));
+  if (moved) {
+    float tmax[2];
+    max_across_groups2(x[0], x[TWO ? 1 : 0], tmax[0], tmax[1]);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-      float pv[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        pv[e] = (FULL || sv[nt][e] != -INFINITY) ? fast_exp2(sv[nt][e] - m_run[nt]) : 0.f;
-      pf[nt] = bf16_rne4(pv);
-      alpha[nt] = 1.f;
-      l_run[nt] = l_run[nt] + ((pv[0] + pv[1]) + (pv[2] + pv[3]));
-    }
-    return false;
-  }
-  float tmax[2];
-  max_across_groups2(x[0], x[TWO ? 1 : 0], tmax[0], tmax[1]);
-  bool mv[2];
-  float m_new[2], psum[2];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    // (-inf > x is false: a row that sees nothing here keeps its reference)
-    mv[nt] = tmax[nt] > m_run[nt] + REF_SLACK;
-    m_new[nt] = mv[nt] ? tmax[nt] : m_run[nt];
-    float pv[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      pv[e] = (FULL || sv[nt][e] != -INFINITY) ? fast_exp2(sv[nt][e] - m_new[nt]) : 0.f;
-    pf[nt] = bf16_rne4(pv);
-    psum[nt] = (pv[0] + pv[1]) + (pv[2] + pv[3]);
-  }
-  const bool moved = __any(mv[0] || (TWO && mv[1]));
-  if (!LAZY || moved) {
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      alpha[nt] = mv[nt] ? fast_exp2(m_run[nt] - m_new[nt]) : 1.f;
-      l_run[nt] = l_run[nt] * alpha[nt] + psum[nt];
-    }
-  } else {
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      alpha[nt] = 1.f;
-      l_run[nt] = l_run[nt] + psum[nt];
+      const float t = tmax[nt] * scale;
+      const bool mv = t > m_run[nt] + REF_SLACK;   // (false for a row that sees nothing here)
+      const float m_new = mv ? t : m_run[nt];
+      alpha[nt] = mv ? fast_exp2(m_run[nt] - m_new) : 1.f;
+      l_run[nt] *= alpha[nt];
+      m_run[nt] = m_new;
     }
   }
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) m_run[nt] = m_new[nt];
+  for (int nt = 0; nt < NT; ++nt) l_run[nt] += probs(nt, m_run[nt]);
   return moved;
 }
 
-// SEEN: every row sees every key of the tile (the caller knows; j0, tile_valid and qmax are not looked at).
-template <int D, bool LAZY, bool TWO, bool BOTH = false, bool SEEN = false>
-FS_DEVICE void attn_tile(const bf16x8_t (&kf)[D / 32], short4_t (&vf)[D / 16], int j0, bool tile_valid, int qmax,
-                         const int (&rpos)[2], int rmin, bool two, const bf16x8_t (&qf)[2][D / 32],
-                         float scale_log2, float4_t (&acc)[D / 16][2], float (&m_run)[2], float (&l_run)[2]) {
-  constexpr int KS = D / 32;
+// SEEN: every row sees every key of the pair (the caller knows; j0, ok and qmax are not looked at).
+// value(mt): the pair's values of dims 16 mt .. as the product's operand.
+template <int D, bool TWO, bool SEEN = false, class Value>
+FS_DEVICE void pair_step(const float4_t (&sc)[2][2], Value value, int j0, const bool (&ok)[2], bool fresh, int qmax,
+                         const int (&rpos)[2], int rmin, float scale, float4_t (&acc)[D / 16][2], float (&m_run)[2],
+                         float (&l_run)[2]) {
   constexpr int MT = D / 16;
   constexpr int NT = TWO ? 2 : 1;
   const int g = (threadIdx.x & 63) >> 4;
-  const bool full = SEEN || (tile_valid && j0 + 15 <= rmin);   // wave-uniform
-  if (!full && (!tile_valid || j0 + 15 > qmax)) {
+  const bool full = SEEN || (ok[0] && ok[1] && j0 + 31 <= rmin);   // wave-uniform
+  float s[2][2][4];   // (one by one: masked in place)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (!tile_valid || j0 + 4 * g + e > qmax) {
+  for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) vf[mt][e] = 0;
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[u][nt][e] = sc[u][nt][e];
+  if (!full) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        const int last = (ok[u] ? rpos[nt] : -1) - j0 - 16 * u - 4 * g;   // the row sees the lane's keys e <= last
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[u][nt][e] = e <= last ? s[u][nt][e] : -INFINITY;
       }
-    }
   }
-  // BOTH: the second half's products are formed whatever `two` says (rows past the tile's end hold
-  // values that are never written out), so the two halves' MFMA chains interleave without a branch
-  float4_t sc[2];
-  if (BOTH) {
-    sc[0] = float4_t{0.f, 0.f, 0.f, 0.f};
-    sc[1] = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      sc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks], qf[0][ks], sc[0], 0, 0, 0);
-      sc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks], qf[1][ks], sc[1], 0, 0, 0);
-    }
-  } else {
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      sc[nt] = float4_t{0.f, 0.f, 0.f, 0.f};
-      if (nt == 0 || two) {
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
-          sc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks], qf[nt][ks], sc[nt], 0, 0, 0);
-      }
-    }
-  }
-  short4_t pf[2];
+  bf16x8_t pf[2];
   float alpha[2];
-  const bool moved = full ? tile_probs<true, LAZY, TWO>(sc, j0, tile_valid, rpos, scale_log2, m_run, l_run, alpha, pf)
-                          : tile_probs<false, LAZY, TWO>(sc, j0, tile_valid, rpos, scale_log2, m_run, l_run, alpha, pf);
-  // LAZY: only when a row moved (alpha = 1 for every row that did not, so skipping it is exact)
-  if (!LAZY || moved) {
+  const bool moved = pair_probs<TWO>(s, scale, m_run, l_run, alpha, pf);
+  if (moved && !fresh) {   // (alpha = 1 for every row that did not: skipping the rescale is exact)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        acc[mt][nt][0] *= alpha[nt];
-        acc[mt][nt][1] *= alpha[nt];
-        acc[mt][nt][2] *= alpha[nt];
-        acc[mt][nt][3] *= alpha[nt];
-      }
-  }
+      for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    acc[mt][0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vf[mt], pf[0], acc[mt][0], 0, 0, 0);
-    if (TWO && (BOTH || two)) acc[mt][1] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vf[mt], pf[1], acc[mt][1], 0, 0, 0);
+        for (int e = 0; e < 4; ++e) acc[mt][nt][e] *= alpha[nt];
+  }
+  // zero bits for the values that must not reach the product (ands behind a branch that every group of dims
+  // takes or skips: a second copy of the products took 50 registers more)
+  const bool masked = !full && !(ok[0] && ok[1] && j0 + 31 <= qmax);
+  u32x4 keep = {~0u, ~0u, ~0u, ~0u};
+  if (masked) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int last = (ok[c >> 1] ? qmax : -1) - j0 - 16 * (c >> 1) - 4 * g, e = 2 * (c & 1);   // keys e, e + 1
+      keep[c] = (e <= last ? 0xffffu : 0u) | (e < last ? 0xffff0000u : 0u);
+    }
+  }
+  // two groups of dims at a time with the next two's values on their way (read sooner, they would need
+  // registers of their own)
+  __builtin_amdgcn_sched_barrier(0);
+  bf16x8_t v[2][2];
+  v[0][0] = value(0);
+  v[0][1] = value(1);
+#pragma unroll
+  for (int mt = 0; mt < MT; mt += 2) {
+    bf16x8_t(&now)[2] = v[mt / 2 & 1], (&next)[2] = v[(mt / 2 & 1) ^ 1];
+    if (mt + 2 < MT) {
+      next[0] = value(mt + 2);
+      next[1] = value(mt + 3);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (masked) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) now[i] = __builtin_bit_cast(bf16x8_t, __builtin_bit_cast(u32x4, now[i]) & keep);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      acc[mt + i][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(now[i], pf[0], acc[mt + i][0], 0, 0, 0);
+      if (TWO) acc[mt + i][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(now[i], pf[1], acc[mt + i][1], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-// A chunk's result for one query row is its 8 partials (tiles t with t % 8 == v, v = 0..7) folded in
+// The operand of a pair's values: the first tile's four keys of the lane, then the second's.
+FS_DEVICE bf16x8_t pair_value(short4_t a, short4_t b) {
+  return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+// A chunk's result for one query row is its 8 partials (class v: pairs p with p % 8 == v) folded in
 // increasing v: (M, L, O) <- (max(M, m), L*2^(M-M') + l*2^(m-M'), O*2^(M-M') + a*2^(m-M')). An empty
 // partial (m = -inf: no visible key) leaves the state as it is; the first non-empty one gets weight 1
 // and the empty state weight 2^-inf = 0. fold_weights returns false for an empty partial.
@@ -476,17 +491,19 @@ FS_DEVICE bool fold_weights(float M, float m, float& Mn, float& cM, float& cm) {
   cm = fast_exp2(m - Mn);
   return true;
 }
-FS_DEVICE float fold_value(float x, float cM, float y, float cm) { return x * cM + y * cm; }
+FS_DEVICE float fold_value(float x, float cM, float y, float cm) { return fmaf(x, cM, y * cm); }
 
-// Tile buffers of a wave. Two (one tile in flight) keep the unit kernel's 2,048 waves at what HBM delivers:
-// with three or four it is 1-10% slower (64 rows of 2048-8192 keys, T = 1: 205 / 209 / 211 us; of 1000-2000
-// slot-major keys: 71 / 76 / 82). Two waves on a CU (four parts) want a second tile in flight (one row of
-// 16000 keys: 59 -> 48 us; a third: 48), four (two parts) one at 128 dims and two at 64.
-constexpr int UNIT_BUFS = 2;
-constexpr int part_bufs(int D, int parts) { return parts == 4 || D == 64 ? 3 : 2; }
+// Pairs of tiles a wave holds in registers. One (a key buffer is refilled as soon as its scores are formed, a
+// value buffer after its product, so about two tiles are in flight) keeps the unit kernel's 2,048 waves at what
+// HBM delivers: with two, where the registers allow them, 64 rows of 1000-2000 keys take 75 us instead of 68.
+// Two waves on a CU (four parts) want two (3 rows of 8000-30000 keys: 68 -> 64 us); four want one (16 rows of
+// 128-1280 keys, 64 dims: 12.3 against 13.4). The last pair is consumed with nothing left to load: prefetching
+// past the end cost 64 rows of 1000-2000 keys 7 us.
+constexpr int UNIT_PAIRS = 1;
+constexpr int part_pairs(int parts) { return parts == 4 ? 2 : 1; }
 
-// TWO: the tile has a second 16-row half. NB: tile buffers in registers.
-template <int D, int BSZ, bool TWO, int NB>
+// TWO: the tile has a second 16-row half. NP: pair buffers in registers.
+template <int D, int BSZ, bool TWO, int NP>
 __device__ __attribute__((always_inline)) inline void attn_wave_tiles(const AttnParams& P, int b, int kbeg, int kend,
                                                                       int qmax, int row0, int nrows,
                                                                       const int (&rpos)[2], int hkv, int w,
@@ -498,37 +515,46 @@ __device__ __attribute__((always_inline)) inline void attn_wave_tiles(const Attn
   const int lane = threadIdx.x & 63;
   const int l16 = lane & 15, g = lane >> 4;
   const int ntiles = (kend - kbeg + 15) >> 4;
-  const int nt_w = ntiles > w ? (ntiles - w + UNIT_WAVES - 1) / UNIT_WAVES : 0;   // <= 128 tiles
-  const bool two = TWO && nrows > 16;
+  const int npairs = (ntiles + 1) >> 1;
+  const int np_w = npairs > w ? (npairs - w + UNIT_WAVES - 1) / UNIT_WAVES : 0;   // <= 64 pairs
+  auto pair_key = [&](int i) { return kbeg + 32 * (w + UNIT_WAVES * i); };   // the first key of the wave's pair i
   const int BS = BSZ ? BSZ : P.kv.block_size;
   const int64_t v_dim = BSZ ? BSZ : P.kv.v_dim;   // == block_size (dim-major values)
 
-  // lane i: where the wave's tiles i and 64 + i start in the pool, in 16-byte units from the head's base (an
-  // unmapped block reads block 0 and is masked), and which of them are mapped
+  // lane i: where the tiles of the wave's pair i start in the pool, in 16-byte units from the head's base (an
+  // unmapped block reads block 0 and is masked, a second tile that the chunk lacks reads the first), and
+  // which of them are there
   typedef uint16_t u16;
   const u16* kpool = reinterpret_cast<const u16*>(P.kv.k) + (int64_t)hkv * P.kv.k_head;
   const u16* vpool = reinterpret_cast<const u16*>(P.kv.v) + (int64_t)hkv * P.kv.v_head;
   const int64_t k_slot = P.kv.k_slot;
-  uint32_t k_at[2] = {0, 0}, v_at[2] = {0, 0};
+  uint32_t k_at[2], v_at[2];
   uint64_t mapped[2];
+  bool all_mapped = true;
   {
     int phys[2] = {-1, -1}, slot0[2] = {0, 0};
+    bool exists[2];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int i = 64 * h + lane;
-      if (i < nt_w) {
-        const int j0 = kbeg + 16 * (w + UNIT_WAVES * i), blk = j0 / BS;
-        slot0[h] = j0 - blk * BS;
-        if (blk < P.max_blocks) phys[h] = P.table[(int64_t)b * P.table_stride + blk];
+    for (int u = 0; u < 2; ++u) {
+      const int j0 = pair_key(lane) + 16 * u, blk = j0 / BS;
+      exists[u] = lane < np_w && j0 < kend;
+      if (exists[u]) {
+        slot0[u] = j0 - blk * BS;
+        if (blk < P.max_blocks) phys[u] = P.table[(int64_t)b * P.table_stride + blk];
       }
     }
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const bool ok = phys[h] >= 0 && phys[h] < P.kv.num_blocks;
-      mapped[h] = __ballot(ok);
-      const int64_t pb = ok ? phys[h] : 0;
-      k_at[h] = (uint32_t)((pb * P.kv.k_block + slot0[h] * k_slot) >> 3);
-      v_at[h] = (uint32_t)((pb * P.kv.v_block + slot0[h]) >> 3);
+    for (int u = 0; u < 2; ++u) {
+      const bool ok = phys[u] >= 0 && phys[u] < P.kv.num_blocks;
+      mapped[u] = __ballot(ok);
+      all_mapped &= mapped[u] == __ballot(exists[u]);
+      const int64_t pb = ok ? phys[u] : 0;
+      k_at[u] = (uint32_t)((pb * P.kv.k_block + slot0[u] * k_slot) >> 3);
+      v_at[u] = (uint32_t)((pb * P.kv.v_block + slot0[u]) >> 3);
+    }
+    if (!exists[1]) {
+      k_at[1] = k_at[0];
+      v_at[1] = v_at[0];
     }
   }
 
@@ -548,19 +574,18 @@ __device__ __attribute__((always_inline)) inline void attn_wave_tiles(const Attn
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       if (ok)
-        qf[nt][ks] = *reinterpret_cast<const bf16x8_t*>(qr + 32 * ks + 8 * g);
+        qf[nt][ks] = signed_query(*reinterpret_cast<const bf16x8_t*>(qr + 32 * ks + 8 * g), P.scale_log2);
       else
         qf[nt][ks] = bf16x8_t{};
     }
   }
 
-  // NB tile buffers in registers: while tile i is consumed, tiles i+1 .. i+NB-1 are in flight. Every load is
-  // unconditional (a prefetch past the end re-reads the last tile) and the loops have one back edge each,
-  // so that each wait before a product counts exactly the loads issued after its operand.
-  static_assert((NB - 1) * (KS + MT) < 64, "vmcnt counts every load in flight");
-  bf16x8_t kb[NB][KS];
-  short4_t vb[NB][MT];
-  auto key0 = [&](int i) { return kbeg + 16 * (w + UNIT_WAVES * i); };
+  // NP pair buffers: a pair's keys are loaded once the scores that read the buffer are formed, its values once
+  // the product is. Every load of a loop is unconditional and the loops have one back edge each, so that each wait before a product counts exactly the loads issued
+  // after its operand.
+  static_assert(NP * 2 * (KS + MT) < 64, "vmcnt counts every load in flight");
+  bf16x8_t kb[NP][2][KS];
+  short4_t vb[NP][2][MT];
   // a lane's byte offsets inside a tile; a tile adds its wave-uniform base. Key (slot, dims 8c .. 8c+7) is at
   // slot * k_slot + c * kgs: slot-major (k_slot = D, kgs = 8) or grouped (k_slot = 8, kgs = 8 * block_size:
   // one load of a tile's 32 dims is a contiguous 1 KB)
@@ -569,29 +594,39 @@ __device__ __attribute__((always_inline)) inline void attn_wave_tiles(const Attn
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) k_lane[ks] = (uint32_t)(2 * (l16 * k_slot + (g + 4 * ks) * kgs));
   const uint32_t v_lane = (uint32_t)(2 * (l16 * v_dim + 4 * g));
-  auto load_tile = [&](int i, bf16x8_t (&kd)[KS], short4_t (&vd)[MT]) {
-    const int ic = max(min(i, nt_w - 1), 0);   // (a wave without tiles reads block 0 and consumes nothing)
-    const int k0 = __builtin_amdgcn_readlane((int)k_at[0], ic & 63), k1 = __builtin_amdgcn_readlane((int)k_at[1], ic & 63);
-    const int v0 = __builtin_amdgcn_readlane((int)v_at[0], ic & 63), v1 = __builtin_amdgcn_readlane((int)v_at[1], ic & 63);
-    uint64_t kt_ = reinterpret_cast<uint64_t>(kpool) + ((uint64_t)(uint32_t)(ic < 64 ? k0 : k1) << 4);
-    uint64_t vt_ = reinterpret_cast<uint64_t>(vpool) + ((uint64_t)(uint32_t)(ic < 64 ? v0 : v1) << 4);
-    asm("" : "+s"(kt_), "+s"(vt_));   // a scalar base and 32-bit lane offsets: no 64-bit vector adds per load
-    typedef __attribute__((address_space(1))) const char GChar;
-    typedef __attribute__((address_space(1))) const bf16x8_t GKey;
-    typedef __attribute__((address_space(1))) const short4_t GVal;
-    GChar* kt = (GChar*)kt_;
-    GChar* vt = (GChar*)vt_;
+  // where a tile of the wave's pair i starts (a wave without pairs reads block 0 and consumes nothing)
+  auto tile_at = [&](const u16* pool, uint32_t at, int i) {
+    const int a = __builtin_amdgcn_readlane((int)at, max(min(i, np_w - 1), 0));
+    uint64_t t = reinterpret_cast<uint64_t>(pool) + ((uint64_t)(uint32_t)a << 4);
+    asm("" : "+s"(t));   // a scalar base and 32-bit lane offsets: no 64-bit vector adds per load
+    return (__attribute__((address_space(1))) const char*)t;
+  };
+  typedef __attribute__((address_space(1))) const bf16x8_t GKey;
+  typedef __attribute__((address_space(1))) const short4_t GVal;
+  auto load_keys = [&](int pair, bf16x8_t (&kd)[2][KS]) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)   // read once per launch: nontemporal
-      kd[ks] = __builtin_nontemporal_load((GKey*)(kt + k_lane[ks]));
+    for (int u = 0; u < 2; ++u) {
+      auto kt = tile_at(kpool, k_at[u], pair);
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-      vd[mt] = __builtin_nontemporal_load((GVal*)(vt + (v_lane + (uint32_t)(32 * mt * v_dim))));
+      for (int ks = 0; ks < KS; ++ks)   // read once per launch: nontemporal
+        kd[u][ks] = __builtin_nontemporal_load((GKey*)(kt + k_lane[ks]));
+    }
+  };
+  auto load_values = [&](int pair, short4_t (&vd)[2][MT]) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      auto vt = tile_at(vpool, v_at[u], pair);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+        vd[u][mt] = __builtin_nontemporal_load((GVal*)(vt + (v_lane + (uint32_t)(32 * mt * v_dim))));
+    }
   };
 #pragma unroll
-  for (int j = 0; j < NB - 1; ++j) {
-    load_tile(j, kb[j], vb[j]);
-    __builtin_amdgcn_sched_barrier(0);   // in tile order, as the loops' waits count them
+  for (int j = 0; j < NP; ++j) {   // in the order that the loops' waits count
+    load_keys(j, kb[j]);
+    __builtin_amdgcn_sched_barrier(0);
+    load_values(j, vb[j]);
+    __builtin_amdgcn_sched_barrier(0);
   }
 
   float4_t acc[MT][2];
@@ -603,34 +638,52 @@ __device__ __attribute__((always_inline)) inline void attn_wave_tiles(const Attn
   float m_run[2] = {-INFINITY, -INFINITY};
   float l_run[2] = {0.f, 0.f};
 
-  // The wave's first n_full tiles have every key mapped and seen by every row: they take a loop without
-  // masks or lookups. The rest (the tiles around the rows' own positions, or all of them where a row is
-  // padding or a block unmapped) are consumed one by one.
+  // The wave's first n_full pairs have every key mapped and seen by every row: they take a loop without masks
+  // or lookups. The rest (the pairs around the rows' own positions, or all of them where a row is padding or
+  // a block unmapped) follow; a pair past the wave's last is two absent tiles.
   const int rmin = rows_min_pos(rpos, nrows);
-  const int n_seen = rmin + 1 > kbeg ? min((rmin + 1 - kbeg) >> 4, ntiles) : 0;   // tiles all rows see
-  const uint64_t want0 = nt_w >= 64 ? ~0ull : (1ull << nt_w) - 1;
-  const uint64_t want1 = nt_w >= 128 ? ~0ull : nt_w > 64 ? (1ull << (nt_w - 64)) - 1 : 0;
-  const bool all_mapped = (mapped[0] & want0) == want0 && (mapped[1] & want1) == want1;
+  const int n_seen = rmin + 1 > kbeg ? min((rmin + 1 - kbeg) >> 5, ntiles >> 1) : 0;   // pairs all rows see
   const int n_full = all_mapped && n_seen > w ? (n_seen - w + UNIT_WAVES - 1) / UNIT_WAVES : 0;
+  const float scale = positive_scale(P.scale_log2);
+  auto there = [&](int i, int u) { return i < np_w && ((mapped[u] >> (i & 63)) & 1) != 0; };
   int i = 0;
-  for (; i + NB <= n_full; i += NB) {
+  auto refill_keys = [&](int j) {   // (moved up, they would need registers of their own)
+    __builtin_amdgcn_sched_barrier(0);
+    load_keys(i + j + NP, kb[j]);
+  };
+  auto refill_values = [&](int j) {
+    __builtin_amdgcn_sched_barrier(0);
+    load_values(i + j + NP, vb[j]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto value = [&](int j) { return [&, j](int mt) { return pair_value(vb[j][0][mt], vb[j][1][mt]); }; };
+  for (; i + NP <= n_full && i + NP < np_w; i += NP) {
 #pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      load_tile(i + j + NB - 1, kb[(j + NB - 1) % NB], vb[(j + NB - 1) % NB]);
-      attn_tile<D, true, TWO, false, true>(kb[j], vb[j], 0, true, 0, rpos, rmin, two, qf, P.scale_log2, acc, m_run, l_run);
+    for (int j = 0; j < NP; ++j) {
+      float4_t sc[2][2];
+      tile_scores<D, TWO>(kb[j][0], qf, sc[0]);
+      tile_scores<D, TWO>(kb[j][1], qf, sc[1]);
+      refill_keys(j);
+      pair_step<D, TWO, true>(sc, value(j), 0, {true, true}, i + j == 0, 0, rpos, rmin, scale, acc, m_run, l_run);
+      refill_values(j);
     }
   }
-  for (; i < nt_w; i += NB) {
+  auto masked_pair = [&](int j, bool refill) {
+    const int p = i + j;
+    float4_t sc[2][2];
+    tile_scores<D, TWO>(kb[j][0], qf, sc[0]);
+    tile_scores<D, TWO>(kb[j][1], qf, sc[1]);
+    if (refill) refill_keys(j);
+    pair_step<D, TWO>(sc, value(j), pair_key(p), {there(p, 0), there(p, 1)}, p == 0, qmax, rpos, rmin, scale, acc, m_run,
+                      l_run);
+    if (refill) refill_values(j);
+  };
+  for (; i + NP < np_w; i += NP) {
 #pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      load_tile(i + j + NB - 1, kb[(j + NB - 1) % NB], vb[(j + NB - 1) % NB]);
-      if (i + j < nt_w) {
-        const int t = i + j;
-        const bool valid = (((t < 64 ? mapped[0] : mapped[1]) >> (t & 63)) & 1) != 0;
-        attn_tile<D, true, TWO>(kb[j], vb[j], key0(t), valid, qmax, rpos, rmin, two, qf, P.scale_log2, acc, m_run, l_run);
-      }
-    }
+    for (int j = 0; j < NP; ++j) masked_pair(j, true);
   }
+#pragma unroll
+  for (int j = 0; j < NP; ++j) masked_pair(j, false);   // the last pairs, or absent ones: nothing is left to load
   // this wave's partial to LDS: acc by (query half, dim tile, lane), m and l by query row
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
@@ -657,8 +710,8 @@ FS_DEVICE void attn_emit(const AttnParams& P, int b, int s, int kbeg, int hkv, i
   const int t = rr / P.G, h = hkv * P.G + (rr - t * P.G);
   if (direct) {   // the same normalisation as attn_combine's
     if (!token_exists(P, b, t)) return;
-    const float f[4] = {L > 0.f ? o[0] / L : 0.f, L > 0.f ? o[1] / L : 0.f, L > 0.f ? o[2] / L : 0.f,
-                        L > 0.f ? o[3] / L : 0.f};
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    const float f[4] = {o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv};
     uint16_t* orow = reinterpret_cast<uint16_t*>(P.out) + o_offset(P, b, t, P.o_sb, P.o_st) + (int64_t)h * P.o_sh;
     *reinterpret_cast<short4_t*>(orow + 16 * mt + 4 * g) = bf16_rne4(f);
     return;
@@ -699,7 +752,7 @@ attn_unit_kernel(AttnParams P) {
   const int kbeg = s * P.split;
   const int kend = min(kbeg + P.split, qmax + 1);
 
-  attn_wave_tiles<D, BSZ, TWO, UNIT_BUFS>(P, b, kbeg, kend, qmax, row0, nrows, rpos, hkv, w, red_acc[w], red_m[w], red_l[w]);
+  attn_wave_tiles<D, BSZ, TWO, UNIT_PAIRS>(P, b, kbeg, kend, qmax, row0, nrows, rpos, hkv, w, red_acc[w], red_m[w], red_l[w]);
   __syncthreads();
 
   // fold the waves' partials in wave order; wave w takes the (query half, 16-dim tile) pairs w,
@@ -729,7 +782,6 @@ attn_unit_kernel(AttnParams P) {
 // where the data allows. Being plain accesses, the compiler issues a wave's loads together; the
 // barrier and the arrival count order them against the other parts' stores.
 constexpr int CPOL_SC1 = 16;
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 FS_DEVICE __amdgpu_buffer_rsrc_t slot_rsrc(float* base, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(base, (short)0, bytes, 0x00020000);
 }
@@ -754,7 +806,7 @@ FS_DEVICE float ld1_dev(__amdgpu_buffer_rsrc_t r, int off) {
 // last folds them in order and emits the rows. The arrival is counted (an agent-scope atomic), never awaited;
 // the published values cross XCDs through device-coherent accesses.
 template <int D, int BSZ, bool TWO, int PARTS>
-__global__ void __launch_bounds__(64 * UNIT_WAVES / PARTS) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(64 * UNIT_WAVES / PARTS) __attribute__((amdgpu_waves_per_eu(1)))
 attn_unit_part_kernel(AttnParams P) {
   constexpr int WPP = UNIT_WAVES / PARTS;
   constexpr int MT = D / 16, GI = (TWO ? 2 : 1) * MT;
@@ -787,7 +839,7 @@ attn_unit_part_kernel(AttnParams P) {
   const int kbeg = s * P.split;
   const int kend = min(kbeg + P.split, qmax + 1);
 
-  attn_wave_tiles<D, BSZ, TWO, part_bufs(D, PARTS)>(P, b, kbeg, kend, qmax, row0, nrows, rpos, hkv, WPP * part + w,
+  attn_wave_tiles<D, BSZ, TWO, part_pairs(PARTS)>(P, b, kbeg, kend, qmax, row0, nrows, rpos, hkv, WPP * part + w,
                                                          red_acc[w], red_m[w], red_l[w]);
   __syncthreads();
 
@@ -867,10 +919,16 @@ attn_unit_part_kernel(AttnParams P) {
 // wave w owns tile PF_WAVES * item.z + w) share every key and value tile through an LDS ring that
 // direct global->LDS copies fill, so a key tile is read from memory once per 256 query rows instead of
 // once per 32. Each wave computes, for its own rows, exactly what the unit kernel computes for them:
-// the partial of tiles v, v + 8, v + 16, ... (v = 0..7, increasing), with attn_tile, folded in
-// increasing v with fold_weights/fold_value. The ring therefore carries the chunk's tiles in that
-// order (all tiles t % 8 == 0, then t % 8 == 1, ...), and a wave skips the tiles wholly above its
+// the partial of the pairs p = v, v + 8, v + 16, ... (v = 0..7, increasing), with pair_step, folded in
+// increasing v with fold_weights/fold_value. The ring therefore carries the chunk's pairs in that
+// order (all pairs p % 8 == 0, then p % 8 == 1, ...), and a wave skips the pairs wholly above its
 // furthest query (no-ops for every row of the wave). Output bits equal the unit kernel's.
+//
+// Bound by vector instructions and the waits between the steps of a pair (2 waves per SIMD, 244 registers at 128
+// dims: no room to form one pair's scores under another's softmax): per pair and wave 32 products (512 cycles)
+// against about 240 vector instructions, a quarter of them the folds of the 8 classes. Tile by tile instead of
+// pair by pair it issued 360. Prompts of 4096, 1228, 1817, 1837 and 817 tokens (32/8 heads, 128 dims):
+// 494 -> 437 us; raising the waves' priority around the products changes it by 1%.
 constexpr int PF_WAVES = 8;      // query tiles (waves) per workgroup
 constexpr int PF_TILES = 4;      // 16-key tiles per ring stage
 constexpr int PF_NS = 4;         // ring stages (two in flight behind the one awaited)
@@ -891,22 +949,22 @@ FS_DEVICE void pf_wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// The chunk's tiles in the ring's order: class v = t % 8 in increasing v, increasing t inside a class.
-// The tile after t (of a chunk of n tiles) is t + 8, or the next class's first tile (t % 8) + 1.
-FS_DEVICE int pf_next_tile(int t, int n) {
-  t += 8;
-  return t < n ? t : (t & 7) + 1;
+// The chunk's pairs of tiles (2p, 2p + 1) in the ring's order: class v = p % 8 in increasing v, increasing p inside
+// a class. The pair after p (of n) is p + 8, or the next class's first pair (p % 8) + 1.
+FS_DEVICE int pf_next_pair(int p, int n) {
+  p += 8;
+  return p < n ? p : (p & 7) + 1;
 }
-// The tile at ring position j (0 <= j < n): class v holds the n_v = ceil((n - v) / 8) tiles v, v + 8, ...
-FS_DEVICE int pf_ring_tile(int j, int n) {
-  int first = 0, t = 0;
+// The pair at place j (0 <= j < n): class v holds the n_v = ceil((n - v) / 8) pairs v, v + 8, ...
+FS_DEVICE int pf_pair(int j, int n) {
+  int first = 0, p = 0;
 #pragma unroll
   for (int v = 0; v < 8; ++v) {
     const int nv = n > v ? ((n - 1 - v) >> 3) + 1 : 0;
-    if (j >= first && j < first + nv) t = v + 8 * (j - first);
+    if (j >= first && j < first + nv) p = v + 8 * (j - first);
     first += nv;
   }
-  return t;
+  return p;
 }
 
 template <int D, int BSZ>
@@ -938,13 +996,13 @@ attn_prefill_kernel(AttnParams P) {
   const int kbeg = s * P.split;
   const int kend = min(kbeg + P.split, qmax_item + 1);
   const int ntiles = max((kend - kbeg + 15) >> 4, 0);
-  const int nst = (ntiles + PF_TILES - 1) / PF_TILES;
+  const int npairs = (ntiles + 1) >> 1;
+  const int nst = (2 * npairs + PF_TILES - 1) / PF_TILES;
 
   // this wave's query tile: the unit kernel's tile z, with its rows, positions and furthest query
   const int z = zb * PF_WAVES + w;
   const int row0 = z * QTILE;
   const int nrows = min(QTILE, P.T * P.G - row0);   // <= 0: a wave past the last tile (copies only)
-  const bool two = nrows > 16;
   const int* posb = P.pos + (int64_t)b * P.T;
   int rpos[2];
 #pragma unroll
@@ -968,7 +1026,8 @@ attn_prefill_kernel(AttnParams P) {
     const int h = hkv * P.G + (ok ? r - (r / P.G) * P.G : 0);
     const u16* qr = qbase + q_offset(P, b, t) + (int64_t)h * P.q_sh;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[nt][ks] = ok ? *reinterpret_cast<const bf16x8_t*>(qr + 32 * ks + 8 * g) : bf16x8_t{};
+    for (int ks = 0; ks < KS; ++ks)
+      qf[nt][ks] = ok ? signed_query(*reinterpret_cast<const bf16x8_t*>(qr + 32 * ks + 8 * g), P.scale_log2) : bf16x8_t{};
   }
 
   // the chunk's table entries
@@ -1022,23 +1081,23 @@ attn_prefill_kernel(AttnParams P) {
   const uint32_t ring0 = (uint32_t)(uintptr_t)ring;
   // this lane's operand reads inside a tile (bytes)
   const int fk = CPR == 16 ? (l16 & 15) : ((l16 >> 1) & 7);
-  int koff[KS];
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) koff[ks] = (kgrp ? (4 * ks + g) * 16 + l16 : l16 * CPR + ((4 * ks + g) ^ fk)) * 16;
+  // (chunk 4ks + g of a row's keys lies at koff ^ (ks * kx): one register for the KS addresses)
+  const int koff = (kgrp ? g * 16 + l16 : l16 * CPR + (g ^ fk)) * 16, kx = kgrp ? 1024 : 64;
   const int voff = TK + (2 * l16 + ((g >> 1) ^ ((l16 >> 3) & 1))) * 16 + 8 * (g & 1);
 
-  // Copies walk the ring positions PF_TILES at a time; a position past the last tile copies the last
+  // Copies walk the ring positions PF_TILES at a time; a position without a tile copies the last
   // tile again. Lane j holds the byte offset of the tile at ring position 64 * win + j (relative to
   // pool_h), refreshed when a stage enters the next 64 positions, so a copy reads its tile's offset
   // with two lane reads instead of walking the order and the table per copy.
   static_assert(64 % PF_TILES == 0, "a stage's positions lie in one 64-position window");
   uint32_t woff_lo = 0, woff_hi = 0;
   auto refresh = [&](int win) {
-    const int t = pf_ring_tile(min(64 * win + lane, ntiles - 1), ntiles);
+    const int j = min(64 * win + lane, 2 * npairs - 1);
+    const int t = min(2 * pf_pair(j >> 1, npairs) + (j & 1), ntiles - 1);
     const int key0 = kbeg + 16 * t;
     const int bi = key0 / BS;
     const int ph = tbl[bi - blk0];
-    const int64_t pb = ph >= 0 ? ph : 0;         // unmapped: block 0, masked in attn_tile
+    const int64_t pb = ph >= 0 ? ph : 0;         // unmapped: block 0, masked in pair_step
     const uint64_t o = (uint64_t)(2 * (pb * blk_stride + (int64_t)(key0 - bi * BS) * slot_mul));
     woff_lo = (uint32_t)o;
     woff_hi = (uint32_t)(o >> 32);
@@ -1095,40 +1154,51 @@ attn_prefill_kernel(AttnParams P) {
 #pragma unroll
   for (int k = 0; k < PF_NS - 1; ++k)
     if (k < nst) issue(k);
-  int rt = 0;   // the tile consumed next
+  int next = 0;   // the pair consumed next
+  bool fresh = true;   // acc is all zeros
   int cur_v = 0;
+  const float scale = positive_scale(P.scale_log2);
+  auto mapped = [&](int key0) { return all_mapped || tbl[key0 / BS - blk0] >= 0; };
   for (int k = 0; k < nst; ++k) {
     wait_stages(min(PF_NS - 2, nst - 1 - k));
     __syncthreads();   // stage k has landed for every wave; stage k-1 is no longer being read
     if (k + PF_NS - 1 < nst) issue(k + PF_NS - 1);
     // the stage's operand addresses, once per stage: each tile's reads add only its constant offset
     const uint32_t st_lds = ring0 + (uint32_t)((k % PF_NS) * STAGE);
-    uint32_t kad[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) kad[ks] = st_lds + (uint32_t)koff[ks];
     const uint32_t vad = st_lds + (uint32_t)voff;
 #pragma unroll
-    for (int u = 0; u < PF_TILES; ++u) {
-      if (k * PF_TILES + u >= ntiles) break;
-      const int t = rt;
-      rt = pf_next_tile(rt, ntiles);
+    for (int u = 0; u < PF_TILES; u += 2) {
+      if (k * (PF_TILES / 2) + u / 2 >= npairs) break;
+      const int pair = next;
+      next = pf_next_pair(next, npairs);
       if (nrows <= 0) continue;
-      if ((t & 7) != cur_v) {   // a new class: fold the last one into the row state
+      if ((pair & 7) != cur_v) {   // a new class: fold the last one into the row state
         fold();
-        cur_v = t & 7;
+        fresh = true;
+        cur_v = pair & 7;
       }
-      if (t >= ntiles_w) continue;   // wholly above every query of the wave
+      if (2 * pair >= ntiles_w) continue;   // wholly above every query of the wave
       typedef __attribute__((address_space(3))) const bf16x8_t LdsK;
       typedef __attribute__((address_space(3))) const short4_t LdsV;
-      bf16x8_t kf[KS];
-      short4_t vf[MT];
+      auto value = [&](int mt) {
+        // (an address that the compiler cannot split pairs the two tiles' reads, into the operand's registers)
+        uint32_t at = vad + (uint32_t)(u * TB + mt * 16 * 32);
+        asm("" : "+v"(at));
+        return pair_value(*(LdsV*)(uintptr_t)at, *(LdsV*)(uintptr_t)(at + TB));
+      };
+      float4_t sc[2][2];
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) kf[ks] = *(LdsK*)(uintptr_t)(kad[ks] + (uint32_t)(u * TB));
+      for (int h = 0; h < 2; ++h) {
+        bf16x8_t kf[KS];
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) vf[mt] = *(LdsV*)(uintptr_t)(vad + (uint32_t)(u * TB + mt * 16 * 32));
-      const int key0 = kbeg + 16 * t;
-      const bool tv = all_mapped || tbl[key0 / BS - blk0] >= 0;
-      attn_tile<D, true, true, true>(kf, vf, key0, tv, qmax, rpos, rmin, two, qf, P.scale_log2, acc, m_run, l_run);
+        for (int ks = 0; ks < KS; ++ks) kf[ks] = *(LdsK*)(uintptr_t)(st_lds + (uint32_t)(koff ^ (ks * kx)) + (uint32_t)((u + h) * TB));
+        tile_scores<D, true>(kf, qf, sc[h]);
+        __builtin_amdgcn_sched_barrier(0);   // (one tile's keys in registers)
+      }
+      const int key0 = kbeg + 32 * pair;
+      const bool ok[2] = {mapped(key0), 2 * pair + 1 < ntiles && mapped(key0 + 16)};
+      pair_step<D, true>(sc, value, key0, ok, fresh, qmax, rpos, rmin, scale, acc, m_run, l_run);
+      fresh = false;
     }
   }
   if (nrows <= 0) return;
@@ -1473,7 +1543,8 @@ __global__ void __launch_bounds__(64 * COMBINE_ROWS) attn_combine_kernel(AttnPar
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     const int d = lane + 64 * c;
-    if (d < D) E::store(orow, d, L > 0.f ? acc[c] / L : 0.f);
+    // (16-bit outputs: one division per row, as attn_emit has it)
+    if (d < D) E::store(orow, d, DT == FS_F32 ? (L > 0.f ? acc[c] / L : 0.f) : acc[c] * (L > 0.f ? 1.f / L : 0.f));
   }
 }
 

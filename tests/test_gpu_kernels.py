@@ -642,6 +642,33 @@ def test_attention_unit_parts_equal_unit_kernel_bitwise(d, g, bs, t, hi_ctx):
     assert rel_err(full[:3].float().cpu(), ref) < 2e-2
 
 
+@pytest.mark.parametrize("d,t,g,bs,layout", [(64, 1, 4, 16, "slots"), (128, 5, 4, 16, "groups"), (128, 9, 4, 48, "slots"),
+                                            (64, 40, 4, 16, "groups"), (128, 50, 4, 16, "groups")])
+def test_attention_tile_pairs(d, t, g, bs, layout):
+    """Pairs of 16-key tiles: contexts that end in a pair's first or second tile or fill it, a block unmapped in
+    the first or the second tile of a pair, for the unit kernel (one and two halves of rows) and the prefill
+    kernel: against float64 on the bf16 inputs. A negative scale is the positive one with the queries negated
+    and a scale of 0 the queries zeroed, bit for bit."""
+    case("attention tile pairs", d, t, g, bs, layout)
+    ctx = [max(c, t) for c in (1, 15, 16, 17, 32, 33, 48, 255, 256, 257, 273, 300, 300)]
+    b, hkv = len(ctx), 2
+    q, k, v, tables, pos = _paged_case(b, t, hkv * g, hkv, d, bs, ctx, sum(-(-c // bs) for c in ctx) + 3, torch.bfloat16, d + t)
+    tables[11, 2], tables[12, 5] = -1, -1
+    out, pool = _run_attention(q, k, v, tables, pos, torch.bfloat16, bs, layout)
+    blocks = tables.clamp_min(0)
+    kk, vv = ((x.double()[blocks].permute(0, 2, 1, 3, 4).reshape(b, hkv, -1, d).repeat_interleave(g, 1)) for x in (k, v))
+    s = q.double().transpose(1, 2) @ kk.transpose(2, 3) / math.sqrt(d)
+    keys = torch.arange(kk.shape[2])
+    seen = (keys <= pos[:, None, :, None]) & (tables.repeat_interleave(bs, 1) >= 0)[:, None, None, :]
+    ref = (s.masked_fill(~seen, -math.inf).softmax(-1) @ vv).transpose(1, 2)
+    # probabilities and outputs are rounded to bf16 (2^-9 each, relative to a weighted sum of |v| <= 5)
+    torch.testing.assert_close(out.cpu().double(), ref, atol=2 * 5 * 2 ** -9, rtol=2 ** -8)
+    lay, tab, pd, qd = pool.layout(0), tables.int().to(DEV), pos.int().to(DEV), q.to(DEV)
+    run = lambda q_, scale: ops.paged_attention(q_, lay, tab, pd, scale)
+    assert torch.equal(run(qd, -1.0 / math.sqrt(d)), run(-qd, 1.0 / math.sqrt(d)))
+    assert torch.equal(run(qd, 0.0), run(torch.zeros_like(qd), 1.0 / math.sqrt(d)))
+
+
 def test_attention_split_units_replayed_from_a_graph():
     """The split-unit kernel captured in a HIP graph: each replay, with new queries copied in and other
     attention calls run eagerly between replays, gives the eager call's bits (the arrival counters
