@@ -669,6 +669,25 @@ def test_attention_tile_pairs(d, t, g, bs, layout):
     assert torch.equal(run(qd, 0.0), run(torch.zeros_like(qd), 1.0 / math.sqrt(d)))
 
 
+def test_attention_prefill_plan_of_many_groups():
+    """A prefill plan of more groups of query rows than it has threads (33 rows x 32 groups), most of them
+    padding, positions not in order inside a row: each row's bits the same as alone, padding zeros."""
+    case("attention prefill plan of many groups")
+    b, t, g, d, bs = 33, 1024, 8, 64, 16
+    lens = [1 + (37 * i) % 90 for i in range(b)]
+    lens[5], lens[20] = 1024, 700
+    q, k, v, tables, pos = _paged_case(b, t, g, 1, d, bs, [1024] * b, b * 64, torch.bfloat16, 3)
+    pos[:] = -1
+    for i, n in enumerate(lens):
+        pos[i, :n] = torch.arange(n).flip(0) if i % 2 else torch.arange(n)
+    out, pool = _run_attention(q, k, v, tables, pos, torch.bfloat16, bs)
+    lay, tab, pd, qd = pool.layout(0), tables.int().to(DEV), pos.int().to(DEV), q.to(DEV)
+    for i, n in enumerate(lens):
+        one = ops.paged_attention(qd[i: i + 1, :n].contiguous(), lay, tab[i: i + 1], pd[i: i + 1, :n].contiguous(), 1.0 / math.sqrt(d))
+        assert torch.equal(out[i, :n], one[0]), i
+        assert torch.count_nonzero(out[i, n:]) == 0, i
+
+
 def test_attention_split_units_replayed_from_a_graph():
     """The split-unit kernel captured in a HIP graph: each replay, with new queries copied in and other
     attention calls run eagerly between replays, gives the eager call's bits (the arrival counters
