@@ -59,32 +59,9 @@ FS_DEVICE const typename Elem<DT>::T* row_ptr(const RowSet& rs, int b, int i) {
   return reinterpret_cast<const T_*>(rs.base1) + b * rs.sb1 + (i - rs.n0) * rs.si1;
 }
 
-// Load 8 consecutive columns starting at v (a multiple of 8) as f32; columns >= V read as `fill`.
-template <int DT>
-FS_DEVICE void load8(const typename Elem<DT>::T* row, int64_t v, int64_t V, bool vec_ok, float fill, float (&x)[8]) {
-  if (vec_ok && v + 8 <= V) {
-    if (DT == FS_F32) {
-      const float4_t a = *reinterpret_cast<const float4_t*>(reinterpret_cast<const float*>(row) + v);
-      const float4_t c = *reinterpret_cast<const float4_t*>(reinterpret_cast<const float*>(row) + v + 4);
-      x[0] = a[0]; x[1] = a[1]; x[2] = a[2]; x[3] = a[3];
-      x[4] = c[0]; x[5] = c[1]; x[6] = c[2]; x[7] = c[3];
-    } else {
-      typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
-      const u32x4 w = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(row) + v);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        x[2 * j] = Elem<DT>::to_f32((uint16_t)(w[j] & 0xffffu));
-        x[2 * j + 1] = Elem<DT>::to_f32((uint16_t)(w[j] >> 16));
-      }
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = (v + j < V) ? Elem<DT>::load(row, v + j) : fill;
-  }
-}
-
-// Raw registers of 8 consecutive columns (two 16-byte loads for f32, one for bf16/f16), loaded
-// without bounds checks, then converted to f32 apart from the load. A block of loads is issued
+// Raw registers of 8 consecutive columns (two 16-byte loads for f32, one for bf16/f16, at the type's own
+// alignment: a row of an odd vocabulary starts anywhere, and global loads need no more), loaded without
+// bounds checks, then converted to f32 apart from the load. A block of loads is issued
 // first and converted after a scheduling barrier: a conversion between two loads makes the second
 // wait for the first (the compiler places the wait before the conversion).
 template <int DT>
@@ -92,9 +69,7 @@ struct Raw8 {
   typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
   u32x4 w[DT == FS_F32 ? 2 : 1];
   FS_DEVICE void load(const typename Elem<DT>::T* row, int64_t v) {
-    const u32x4* q = reinterpret_cast<const u32x4*>(row + v);
-    w[0] = q[0];
-    if (DT == FS_F32) w[DT == FS_F32 ? 1 : 0] = q[1];
+    __builtin_memcpy(w, row + v, sizeof(w));
   }
   FS_DEVICE void to_f32(float (&x)[8]) const {
 #pragma unroll
@@ -110,20 +85,33 @@ struct Raw8 {
   }
 };
 
-// Every group u (columns v0 + u * THREADS * VEC .. + 7) of a U-group block is in range and 16-byte
-// loadable: false only in a row's last chunk (or for unaligned rows).
+// Load 8 consecutive columns starting at v (a multiple of 8) as f32; columns >= V read as `fill`.
+template <int DT>
+FS_DEVICE void load8(const typename Elem<DT>::T* row, int64_t v, int64_t V, float fill, float (&x)[8]) {
+  if (v + 8 <= V) {
+    Raw8<DT> r;
+    r.load(row, v);
+    r.to_f32(x);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = (v + j < V) ? Elem<DT>::load(row, v + j) : fill;
+  }
+}
+
+// Every group u (columns v0 + u * THREADS * VEC .. + 7) of a U-group block is in range: false only in a
+// row's last chunk.
 template <int U>
-FS_DEVICE bool block_in_range(int64_t v0, int64_t V, bool vec_ok) {
-  return vec_ok && v0 + (int64_t)(U - 1) * THREADS * VEC + VEC <= V;
+FS_DEVICE bool block_in_range(int64_t v0, int64_t V) {
+  return v0 + (int64_t)(U - 1) * THREADS * VEC + VEC <= V;
 }
 
 // U groups of 8 consecutive columns per thread, group u at column v0 + u * THREADS * VEC, as f32;
 // columns >= V read as `fill`. In range, the U loads are issued back to back before any conversion.
 template <int DT, int U>
-FS_DEVICE void load_block(const typename Elem<DT>::T* row, int64_t v0, int64_t V, bool vec_ok, float fill,
+FS_DEVICE void load_block(const typename Elem<DT>::T* row, int64_t v0, int64_t V, float fill,
                           float (&x)[U][8]) {
   constexpr int64_t STRIDE = (int64_t)THREADS * VEC;
-  if (block_in_range<U>(v0, V, vec_ok)) {
+  if (block_in_range<U>(v0, V)) {
     Raw8<DT> r[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) r[u].load(row, v0 + u * STRIDE);
@@ -132,7 +120,7 @@ FS_DEVICE void load_block(const typename Elem<DT>::T* row, int64_t v0, int64_t V
     for (int u = 0; u < U; ++u) r[u].to_f32(x[u]);
   } else {
 #pragma unroll
-    for (int u = 0; u < U; ++u) load8<DT>(row, v0 + u * STRIDE, V, vec_ok, fill, x[u]);
+    for (int u = 0; u < U; ++u) load8<DT>(row, v0 + u * STRIDE, V, fill, x[u]);
   }
 }
 
@@ -187,6 +175,57 @@ FS_DEVICE Stat merge_row(const Stat* st, int nch) {
   return r;
 }
 
+// The chunk statistics of R rows (one wave, lane c holding chunk c of each) merged as merge_row does:
+// the max over the chunks, Σ s_c 2^(m_c - M) added in chunk order, the first argmax. The rows'
+// reductions are interleaved step by step, so their cross-lane latencies overlap.
+template <int R>
+FS_DEVICE void merge_rows_wave(const Stat (&st)[R], bool in, int nch, Stat (&out)[R]) {
+  float M[R], S[R], term[R], av[R];
+  int ai[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    M[i] = in ? st[i].m : -INFINITY;
+    av[i] = in ? st[i].av : -INFINITY;
+    ai[i] = in ? st[i].ai : 0x7fffffff;
+    S[i] = 0.f;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    float oa[R], om[R];
+    int oi[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      om[i] = __shfl_xor(M[i], o, 64);
+      oa[i] = __shfl_xor(av[i], o, 64);
+      oi[i] = __shfl_xor(ai[i], o, 64);
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      M[i] = fmaxf(M[i], om[i]);
+      argmax_merge(av[i], ai[i], oa[i], oi[i]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+    term[i] = (!in || st[i].m == -INFINITY) ? 0.f : st[i].s * __builtin_amdgcn_exp2f((st[i].m - M[i]) * LOG2E_F);
+  for (int c = 0; c < nch; ++c)
+#pragma unroll
+    for (int i = 0; i < R; ++i) S[i] += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(term[i]), c));
+#pragma unroll
+  for (int i = 0; i < R; ++i) out[i] = Stat{M[i], S[i], av[i], ai[i]};
+}
+
+// The same for one row whose chunk statistics the calling wave reads itself. (One thread walking the chunks,
+// a load at a time, took as long as the 8192 columns it was for.)
+FS_DEVICE Stat merge_row_wave(const Stat* st, int nch) {
+  if (nch > 64) return merge_row(st, nch);
+  const int lane = threadIdx.x & 63;
+  Stat in[1] = {Stat{-INFINITY, 0.f, -INFINITY, 0x7fffffff}}, out[1];
+  if (lane < nch) in[0] = st[lane];
+  merge_rows_wave<1>(in, lane < nch, nch, out);
+  return out[0];
+}
+
 // The probability of logit x in a row with merged statistics (M, S) at temperature T > 0
 // (sampling.py:13): y = x / T (a true division; exact and skipped at T == 1), then exp(y - M) times the
 // correctly rounded 1/S, the order torch's softmax uses. Every kernel that needs a probability on the
@@ -203,13 +242,37 @@ struct ProbFn {
 
 // y = x / T in place for a block of registers, under a branch uniform over the workgroup (T is the
 // row's or the sequence's), so T == 1 costs nothing; padding (-inf or 0) stays what it was.
+//
+// The divisor is the same for the whole row, so the correctly rounded quotient comes from its reciprocal
+// (Markstein): q = x r is within 2 ulps; one step q + r (x - q T) leaves a faithful quotient and a second one
+// the correctly rounded one, the remainders being exact. That takes 5 instructions for a division's 13 (the
+// statistics of 832 rows of 128256, a third at T = 0.7: 50 -> 46 us with the argmax of the T = 0 rows). Quotients of 2^120 or more, infinities among them, and
+// temperatures of odd sizes take the division. (A remainder of |x| < 2^-100 may underflow; a y that small
+// only ever enters as y - M.)
 template <int U>
 FS_DEVICE void divide_by_t(float (&x)[U][8], float T) {
-  if (T != 1.f) {
+  if (T == 1.f) return;
+  const float r = 1.f / T;
+  float big = 0.f;
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) big = fmaxf(big, fabsf(x[u][j]));   // (a NaN stays one either way)
+  const bool slow = !(T >= 0x1p-60f && T <= 0x1p60f) || __any(!(big * r < 0x1p120f));
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (slow) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[u][j] = x[u][j] / T;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        float q = x[u][j] * r;
+        q = fmaf(fmaf(-q, T, x[u][j]), r, q);
+        x[u][j] = fmaf(fmaf(-q, T, x[u][j]), r, q);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);   // (all groups at once would take half the occupancy)
   }
 }
 
@@ -219,32 +282,32 @@ FS_DEVICE void divide_by_t(float (&x)[U][8], float T) {
 // pass (the sum's exp is the bare exp2; S differs from torch's sum by rounding either way).
 template <int DT>
 FS_DEVICE Stat chunk_stat(const typename Elem<DT>::T* row, int c, int64_t V, float T, float* shf, int* shi) {
-  const bool vec_ok = (V % VEC) == 0 && ((reinterpret_cast<uintptr_t>(row) & 15) == 0);
   float x[UNROLL][8];
-  load_block<DT, UNROLL>(row, (int64_t)c * CH + (int64_t)threadIdx.x * VEC, V, vec_ok, -INFINITY, x);
+  load_block<DT, UNROLL>(row, (int64_t)c * CH + (int64_t)threadIdx.x * VEC, V, -INFINITY, x);
   Stat st;
   if (T <= 0.f) {
     float amv = -INFINITY;
     int ami = 0x7fffffff;
+    // the maximum, then the first column that equals it (a thread's columns are in increasing order; padding
+    // reads -inf past the row's end)
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      const int64_t v0 = (int64_t)c * CH + (int64_t)(threadIdx.x + THREADS * u) * VEC;
+    for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (v0 + j < V) argmax_merge(amv, ami, x[u][j], (int)(v0 + j));
-    }
+      for (int j = 0; j < 8; ++j) amv = fmaxf(amv, x[u][j]);
+    const int64_t v0 = (int64_t)c * CH + (int64_t)threadIdx.x * VEC;
+#pragma unroll
+    for (int u = UNROLL - 1; u >= 0; --u)
+#pragma unroll
+      for (int j = 7; j >= 0; --j)
+        if (x[u][j] == amv) ami = THREADS * VEC * u + j;
+    ami = v0 + ami < V ? (int)(v0 + ami) : 0x7fffffff;
     block_argmax(amv, ami, shf, shi);
     st.m = st.av = amv;
     st.ai = ami;
     st.s = 0.f;
     return st;
   }
-  if (T != 1.f) {
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) x[u][j] = x[u][j] / T;  // padding stays -inf
-  }
+  divide_by_t(x, T);   // padding stays -inf
   float m = -INFINITY;
 #pragma unroll
   for (int u = 0; u < UNROLL; ++u)
@@ -298,19 +361,16 @@ __global__ void __launch_bounds__(THREADS) sample_argmax_kernel(RowSet rs, int64
                                                                 float* __restrict__ pv, int* __restrict__ pi) {
   __shared__ float shf[THREADS / 64];
   __shared__ int shi[THREADS / 64];
-  __shared__ Stat shs;
   const int c = blockIdx.x, r = blockIdx.y;
   const float T = temps ? temps[r] : t_all;
   if (T <= 0.f) return;
   const auto* row = row_ptr<DT>(rs, r, 0);
   const float* er = E + (int64_t)r * ldE;
-  const bool vec_ok = (V % VEC) == 0 && ((reinterpret_cast<uintptr_t>(row) & 15) == 0) &&
-                      ((reinterpret_cast<uintptr_t>(er) & 15) == 0);
   float bv = -INFINITY;
   int bi = 0x7fffffff;
   float x[UNROLL][8], e[UNROLL][8];   // the chunk's loads go out before the row's statistics are merged
   const int64_t vb = (int64_t)c * CH + (int64_t)threadIdx.x * VEC;
-  if (block_in_range<UNROLL>(vb, V, vec_ok)) {
+  if (block_in_range<UNROLL>(vb, V)) {
     Raw8<DT> rx[UNROLL];
     Raw8<FS_F32> re[UNROLL];
 #pragma unroll
@@ -325,19 +385,35 @@ __global__ void __launch_bounds__(THREADS) sample_argmax_kernel(RowSet rs, int64
       re[u].to_f32(e[u]);
     }
   } else {
-    load_block<DT, UNROLL>(row, vb, V, vec_ok, -INFINITY, x);
-    load_block<FS_F32, UNROLL>(er, vb, V, vec_ok, 1.f, e);
+    load_block<DT, UNROLL>(row, vb, V, -INFINITY, x);
+    load_block<FS_F32, UNROLL>(er, vb, V, 1.f, e);
   }
-  if (threadIdx.x == 0) shs = merge_row(stats + (int64_t)r * nch, nch);
-  __syncthreads();
-  const ProbFn fs(T, shs);
+  const ProbFn fs(T, merge_row_wave(stats + (int64_t)r * nch, nch));
   divide_by_t(x, T);
+  // The columns are ranked by cheap keys 2^((y - M) log2 e) * rcp(E), which differ from the exact ones (times S)
+  // by the exponent's rounding, under 2^-16 while p is a normal number, and a few ulps; a column below
+  // max * (1 - 2^-12) cannot win. Only the others, a wave's one or two, are scored exactly. The bound holds
+  // for reciprocals up to 2^30 and a maximum of at least 2^-60 (a p below 2^-90 then loses whatever its E, so
+  // no product of a winner underflows); otherwise every column is scored. 64 bf16 rows of 128256: 18 us with every column scored
+  // (and the row's statistics merged by one thread) -> 11.
+  float key[UNROLL][8], km = 0.f, rm = 0.f;
+#pragma unroll
+  for (int u = 0; u < UNROLL; ++u)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float rc = __builtin_amdgcn_rcpf(e[u][j]);
+      rm = fmaxf(rm, rc);
+      key[u][j] = __builtin_amdgcn_exp2f((x[u][j] - fs.M) * LOG2E_F) * rc;
+      km = fmaxf(km, key[u][j]);
+    }
+  km = wave_max(km);
+  const float th = !__any(!(rm <= 0x1p30f)) && km >= 0x1p-60f && km < INFINITY ? km - km * 0x1p-12f : -INFINITY;
 #pragma unroll
   for (int u = 0; u < UNROLL; ++u) {
     const int64_t v0 = (int64_t)c * CH + (int64_t)(threadIdx.x + THREADS * u) * VEC;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      if (v0 + j < V) argmax_merge(bv, bi, fs.of_y(x[u][j]) / e[u][j], (int)(v0 + j));
+      if (v0 + j < V && !(key[u][j] < th)) argmax_merge(bv, bi, fs.of_y(x[u][j]) / er[v0 + j], (int)(v0 + j));
     }
   }
   block_argmax(bv, bi, shf, shi);
@@ -347,23 +423,27 @@ __global__ void __launch_bounds__(THREADS) sample_argmax_kernel(RowSet rs, int64
   }
 }
 
-__global__ void sample_final_kernel(int R, int nch, const float* __restrict__ temps, float t_all, bool greedy_only,
-                                    const Stat* __restrict__ stats, const float* __restrict__ pv,
-                                    const int* __restrict__ pi, int64_t* __restrict__ tok, int32_t* __restrict__ tok32,
-                                    int64_t ld32) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= R) return;
-  int best;
+// one wave per row
+__global__ void __launch_bounds__(64) sample_final_kernel(int nch, const float* __restrict__ temps, float t_all,
+                                                          bool greedy_only, const Stat* __restrict__ stats,
+                                                          const float* __restrict__ pv, const int* __restrict__ pi,
+                                                          int64_t* __restrict__ tok, int32_t* __restrict__ tok32,
+                                                          int64_t ld32) {
+  const int r = blockIdx.x;
   const float T = temps ? temps[r] : t_all;
-  if (greedy_only || T <= 0.f) {
-    best = merge_row(stats + (int64_t)r * nch, nch).ai;
-  } else {
-    float v = pv[(int64_t)r * nch];
-    best = pi[(int64_t)r * nch];
-    for (int c = 1; c < nch; ++c) argmax_merge(v, best, pv[(int64_t)r * nch + c], pi[(int64_t)r * nch + c]);
+  const bool greedy = greedy_only || T <= 0.f;
+  const int64_t r0 = (int64_t)r * nch;
+  float v = -INFINITY;
+  int best = 0x7fffffff;
+  for (int c = threadIdx.x; c < nch; c += 64) {
+    if (greedy) argmax_merge(v, best, stats[r0 + c].av, stats[r0 + c].ai);
+    else argmax_merge(v, best, pv[r0 + c], pi[r0 + c]);
   }
-  tok[r] = best;
-  if (tok32) tok32[(int64_t)r * ld32] = best;
+  wave_argmax(v, best);
+  if (threadIdx.x == 0) {
+    tok[r] = best;
+    if (tok32) tok32[(int64_t)r * ld32] = best;
+  }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -444,46 +524,6 @@ FS_DEVICE void write_outputs(const AcceptArgs& A, int b, int j, int extra, const
     A.n_acc[b] = j;
     if (A.seq_len) A.seq_len[b] = pre.len0 + 1 + j;  // want = cached + 1 + len(accepted) (speculative.py:77)
   }
-}
-
-// The chunk statistics of R rows (one wave, lane c holding chunk c of each) merged as merge_row does:
-// the max over the chunks, Σ s_c 2^(m_c - M) added in chunk order, the first argmax. The rows'
-// reductions are interleaved step by step, so their cross-lane latencies overlap.
-template <int R>
-FS_DEVICE void merge_rows_wave(const Stat (&st)[R], bool in, int nch, Stat (&out)[R]) {
-  float M[R], S[R], term[R], av[R];
-  int ai[R];
-#pragma unroll
-  for (int i = 0; i < R; ++i) {
-    M[i] = in ? st[i].m : -INFINITY;
-    av[i] = in ? st[i].av : -INFINITY;
-    ai[i] = in ? st[i].ai : 0x7fffffff;
-    S[i] = 0.f;
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    float oa[R], om[R];
-    int oi[R];
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-      om[i] = __shfl_xor(M[i], o, 64);
-      oa[i] = __shfl_xor(av[i], o, 64);
-      oi[i] = __shfl_xor(ai[i], o, 64);
-    }
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-      M[i] = fmaxf(M[i], om[i]);
-      argmax_merge(av[i], ai[i], oa[i], oi[i]);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < R; ++i)
-    term[i] = (!in || st[i].m == -INFINITY) ? 0.f : st[i].s * __builtin_amdgcn_exp2f((st[i].m - M[i]) * LOG2E_F);
-  for (int c = 0; c < nch; ++c)
-#pragma unroll
-    for (int i = 0; i < R; ++i) S[i] += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(term[i]), c));
-#pragma unroll
-  for (int i = 0; i < R; ++i) out[i] = Stat{M[i], S[i], av[i], ai[i]};
 }
 
 // The step of sequence b, run by one whole workgroup. Wave 0 tests every proposal at once, one lane
@@ -718,14 +758,11 @@ FS_DEVICE void pair_chunk(const AcceptArgs& A, int b, int c, const PairCtx& pc, 
   }
   const auto* pr = row_ptr<DT>(A.rs, b, j);
   const auto* qr = bonus ? pr : row_ptr<DT>(A.rs, b, A.rs.n0 + j);
-  const bool vec_ok = (A.V % VEC) == 0 &&
-                      (((reinterpret_cast<uintptr_t>(pr) | reinterpret_cast<uintptr_t>(qr)) & 15) == 0);
   const float* er = A.E + (int64_t)b * A.ldE;
-  const bool evec_ok = (A.V % VEC) == 0 && ((reinterpret_cast<uintptr_t>(er) & 15) == 0);
   __builtin_amdgcn_sched_barrier(0);   // j is in hand before the first load below is issued
   float xp[UNROLL_R][8], xq[UNROLL_R][8], e[UNROLL_R][8];   // every load in flight before any arithmetic
   const int64_t vb = (int64_t)c * CHR + (int64_t)threadIdx.x * VEC;
-  if (block_in_range<UNROLL_R>(vb, A.V, vec_ok && evec_ok)) {
+  if (block_in_range<UNROLL_R>(vb, A.V)) {
     Raw8<DT> rp[UNROLL_R], rq[UNROLL_R];
     Raw8<FS_F32> re[UNROLL_R];
 #pragma unroll
@@ -742,9 +779,9 @@ FS_DEVICE void pair_chunk(const AcceptArgs& A, int b, int c, const PairCtx& pc, 
       re[u].to_f32(e[u]);
     }
   } else {
-    load_block<DT, UNROLL_R>(pr, vb, A.V, vec_ok, 0.f, xp);
-    if (!bonus) load_block<DT, UNROLL_R>(qr, vb, A.V, vec_ok, 0.f, xq);
-    load_block<FS_F32, UNROLL_R>(er, vb, A.V, evec_ok, 1.f, e);
+    load_block<DT, UNROLL_R>(pr, vb, A.V, 0.f, xp);
+    if (!bonus) load_block<DT, UNROLL_R>(qr, vb, A.V, 0.f, xq);
+    load_block<FS_F32, UNROLL_R>(er, vb, A.V, 1.f, e);
   }
   if (!PROBS) {   // y = x / T once per element (the ProbFn arithmetic, divided ahead)
     divide_by_t(xp, T);
@@ -958,24 +995,38 @@ __global__ void __launch_bounds__(64) accept_draw_kernel(AcceptArgs A) {
 // ------------------------------------------------------------------------------------------------
 // probs_from_logits
 // ------------------------------------------------------------------------------------------------
+// One workgroup per (row, THREADS * VEC columns), 8 consecutive columns per thread: a row alone fills few CUs, and
+// a thread that walked 32 columns one by one waited for each (one row of 128256: 13.8 us -> 4.1).
 template <int DT>
 __global__ void __launch_bounds__(THREADS) probs_kernel(RowSet rs, int64_t V, int nch, float T,
                                                         const Stat* __restrict__ stats, void* __restrict__ out,
                                                         int64_t ldo) {
-  __shared__ Stat shs;
-  const int c = blockIdx.x, r = blockIdx.y;
-  if (threadIdx.x == 0) shs = merge_row(stats + (int64_t)r * nch, nch);
-  __syncthreads();
-  const Stat st = shs;
-  const auto* row = row_ptr<DT>(rs, r, 0);
-  for (int u = 0; u < UNROLL * VEC; ++u) {
-    const int64_t v = (int64_t)c * CH + (int64_t)u * THREADS + threadIdx.x;
-    if (v >= V) break;
-    if (T > 0.f) {
-      reinterpret_cast<float*>(out)[(int64_t)r * ldo + v] = ProbFn(T, st)(Elem<DT>::load(row, v));
+  typedef typename Elem<DT>::T T_;
+  const int r = blockIdx.y;
+  const int64_t v0 = ((int64_t)blockIdx.x * THREADS + threadIdx.x) * VEC;
+  if (T > 0.f) {
+    const T_* row = row_ptr<DT>(rs, r, 0);
+    float x[1][8];
+    load8<DT>(row, v0, V, -INFINITY, x[0]);
+    const ProbFn f(T, merge_row_wave(stats + (int64_t)r * nch, nch));
+    divide_by_t(x, T);
+    float* o = reinterpret_cast<float*>(out) + (int64_t)r * ldo + v0;
+    if (v0 + 8 <= V && (reinterpret_cast<uintptr_t>(o) & 15) == 0) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        reinterpret_cast<float4_t*>(o)[h] = float4_t{f.of_y(x[0][4 * h]), f.of_y(x[0][4 * h + 1]),
+                                                     f.of_y(x[0][4 * h + 2]), f.of_y(x[0][4 * h + 3])};
     } else {
-      Elem<DT>::store(reinterpret_cast<typename Elem<DT>::T*>(out), (int64_t)r * ldo + v, v == st.ai ? 1.f : 0.f);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (v0 + j < V) o[j] = f.of_y(x[0][j]);
     }
+  } else {
+    const int ai = merge_row_wave(stats + (int64_t)r * nch, nch).ai;
+    T_* o = reinterpret_cast<T_*>(out) + (int64_t)r * ldo;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (v0 + j < V) Elem<DT>::store(o, v0 + j, v0 + j == ai ? 1.f : 0.f);
   }
 }
 
@@ -1124,9 +1175,8 @@ extern "C" int fs_sample_logits(const void* logits, int64_t ld, int64_t R, int64
     default: FS_LAUNCH(FS_F16); break;
   }
 #undef FS_LAUNCH
-  sample_final_kernel<<<dim3((unsigned)((R + 63) / 64)), 64, 0, s>>>((int)R, nch, temperature, temperature_all,
-                                                                     greedy_only, st, pv, pi, tokens_out, tokens_out32,
-                                                                     ld_tok32);
+  sample_final_kernel<<<dim3((unsigned)R), 64, 0, s>>>(nch, temperature, temperature_all, greedy_only, st, pv, pi,
+                                                       tokens_out, tokens_out32, ld_tok32);
   return fs::launch_status("sample_logits");
 }
 
@@ -1146,10 +1196,10 @@ extern "C" int fs_probs_from_logits(const void* logits, int64_t ld, int64_t R, i
   Stat* st = cv.take<Stat>(R * nch);
   RowSet rs{logits, ld, 0, 1, nullptr, 0, 0, 0};
   hipStream_t s = fs::as_stream(stream);
-  dim3 grid((unsigned)nch, (unsigned)R);
+  dim3 grid((unsigned)nch, (unsigned)R), pgrid((unsigned)((V + THREADS * VEC - 1) / (THREADS * VEC)), (unsigned)R);
 #define FS_LAUNCH(DT)                                                                           \
   stats_kernel<DT><<<grid, THREADS, 0, s>>>(rs, V, nch, nullptr, temperature, nullptr, st);  \
-  probs_kernel<DT><<<grid, THREADS, 0, s>>>(rs, V, nch, temperature, st, out, ldo);
+  probs_kernel<DT><<<pgrid, THREADS, 0, s>>>(rs, V, nch, temperature, st, out, ldo);
   switch (dtype) {
     case FS_F32: FS_LAUNCH(FS_F32); break;
     case FS_BF16: FS_LAUNCH(FS_BF16); break;

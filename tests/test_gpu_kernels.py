@@ -1055,6 +1055,43 @@ def test_sample_logits_whole_groups(temperature, dtype):
         assert got == want, v
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("temperature", [0.7, 0.06, 1.5, 2.0 ** 61])
+def test_sample_logits_corners(temperature, dtype):
+    """Draws whose columns leave the bounds that rank them by cheap keys or divide by the temperature's
+    reciprocal, each row against the oracle's draw on the same noise: a ragged vocabulary, masked (-inf)
+    columns, chunks far below the row's maximum, noise of 2^-40, 0 and 2^100, logits whose quotients
+    overflow, ties of equal keys, NaN columns, and the argmax of rows of -inf and of late maxima."""
+    case("sample_logits corners", temperature, dtype)
+    g = torch.Generator().manual_seed(4)
+    for v in (8192 * 2 + 5, 24576):
+        x = (torch.randn(9, v, generator=g) * 3).to(dtype)
+        e = torch.empty(9, v).exponential_(generator=g)
+        x[1, 1::3] = -math.inf
+        x[2, 8192:] -= 200
+        e[3, 77], e[3, 9000] = 2.0 ** -40, 2.0 ** 100
+        x[4, 5:9] = 3e38
+        x[5], e[5] = 1.0, 0.5
+        x[6, 100], x[6, 12000] = 30.0, 30.0
+        e[6, 100], e[6, 12000] = 2.0 ** -20, 2.0 ** -20
+        e[7] = 2.0 ** 70
+        x[8, :] = -40.0
+        x[8, v - 1] = 0.0
+        got = ops.sample_logits(x.to(DEV), temperature, e.to(DEV)).cpu().tolist()
+        for r in range(9):
+            # (a quotient beyond float32 makes the softmax NaN, as torch's is: the draw is nobody's)
+            if torch.isfinite(x[r].float() / temperature).logical_or(x[r].float() == -math.inf).all():
+                assert got[r] == orc.draw(orc.probs_from_logits(x[r].float(), temperature), e[r]), (v, r)
+        x[0] = -math.inf
+        x[1, 3] = math.nan
+        x[2, v - 1] = 100.0
+        want = [0, int(x[1].nan_to_num(-math.inf, neginf=-math.inf).argmax()), v - 1] + [int(x[r].float().argmax()) for r in range(3, 9)]
+        assert ops.sample_logits(x.to(DEV), 0.0, None).cpu().tolist() == want, v
+        row = (torch.randn(2, v + 3, generator=g) * 3).to(dtype)[:, 3:]   # rows that are not 16-byte aligned
+        p = ops.probs_from_logits(row.to(DEV), max(temperature, 0.06)).cpu()
+        torch.testing.assert_close(p, orc.probs_from_logits(row.float(), max(temperature, 0.06)), atol=1e-7, rtol=2e-5)
+
+
 def test_probs_from_logits():
     case("probs_from_logits")
     x = torch.randn(5, 20000) * 4
