@@ -30,8 +30,22 @@ class KVLayout(ctypes.Structure):
     ]
 
 
+class Block(ctypes.Structure):
+    """fs_block: one decoder block of fs_run_blocks."""
+
+    _fields_ = [
+        ("w_qkv", c_p), ("w_o", c_p), ("w_gate_up", c_p), ("w_down", c_p), ("mlp_norm", c_p), ("next_norm", c_p),
+        ("kv", KVLayout), ("tables", c_p), ("table_stride", c_i64), ("slots", c_p), ("visible", c_p),
+        ("mlp_eps", c_f32), ("next_eps", c_f32), ("max_blocks", c_i32), ("reuse_plan", c_i32),
+    ]
+
+
 # name -> (restype, argtypes)
 SIGNATURES = {
+    "fs_run_blocks_workspace": (c_i32, [c_i32, c_i32, c_i32, c_i32, c_i32, c_i64, c_i64, c_i32, c_i32, c_i32,
+                                        ctypes.POINTER(c_i64)]),
+    "fs_run_blocks": (c_i32, [ctypes.POINTER(Block), c_i32, c_i32, c_i32, c_i32, c_i64, c_i64, c_i32, c_p, c_p, c_p, c_i32,
+                              c_f32, c_p, c_p, c_p, c_p, c_p, c_i64, c_p, c_i64, c_p, c_i64, c_p]),
     "fs_last_error": (ctypes.c_char_p, []),
     "fs_abi_version": (c_i32, []),
     "fs_qkv_rope_write": (c_i32, [c_p, c_i64, c_i64, c_i32, c_i32, c_p, c_p, c_p, c_p, c_i32, c_p, c_i64, c_i32,

@@ -28,7 +28,8 @@ FLAGS = [
     "-Wall", "-Wno-unused-function", "-Wno-unused-variable",
 ]
 
-SOURCES = ["abi.hip", "kv.hip", "attention.hip", "norm.hip", "gemm.hip", "gemm_f32.hip", "sample.hip", "rng.hip"]
+SOURCES = ["abi.hip", "kv.hip", "attention.hip", "norm.hip", "gemm.hip", "gemm_f32.hip", "sample.hip", "rng.hip",
+           "blocks.hip"]
 
 
 def _run(cmd):

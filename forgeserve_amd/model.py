@@ -274,6 +274,11 @@ class ForgeModel(nn.Module):
         norm in the same kernel as its last projection's reduction; after block stop-1 by last_norm
         (None: not normalised). x_out: where block stop-1 writes its output (then returned as x)."""
         rope = self._rope()
+        if x_out is None and start < stop:
+            done = self._run_blocks(x, self.layers[start: stop], b, t, pos32, [kv[i] for i in range(start, stop)], rope,
+                                    last_norm)
+            if done is not None:
+                return done
         h = None
         for i in range(start, stop):
             nxt = self.layers[i + 1].attn_norm if i + 1 < stop else last_norm
@@ -282,6 +287,43 @@ class ForgeModel(nn.Module):
         if start >= stop and last_norm is not None:   # no block ran (a draft that is the whole model)
             h = ops.add_rmsnorm(x, last_norm.weight, last_norm.eps)
         return x, h
+
+    @staticmethod
+    def _run_blocks(x, layers, b, t, pos32, kv, rope, last_norm):
+        """_layers' blocks through one native call, which launches what Block.step launches with the choices it
+        makes; None (nothing done) where a block is not a plain one of x's dtype and device, or a view is
+        packed or serves two blocks. The views' tensors are held until the launches are queued."""
+        dt, dev = x.dtype, x.device
+        if (not x.is_contiguous() or b * t == 0 or pos32 is None or pos32.dtype != torch.int32 or pos32.device != dev
+                or not pos32.is_contiguous() or len({id(view) for view in kv}) != len(kv)):
+            return None
+        first = layers[0]
+        d, f, heads = x.shape[1], first.mlp.w_down.weight.shape[1], (first.attn.nh, first.attn.nkv, first.attn.hd)
+        qn, kvn = heads[0] * heads[2], heads[1] * heads[2]
+        norms = [layer.attn_norm for layer in layers[1:]] + [last_norm]
+        weights = []
+        for layer, view, nxt in zip(layers, kv, norms):
+            at, mlp = layer.attn, layer.mlp
+            if (type(layer) is not Block or type(at) is not Attention or type(mlp) is not SwiGLU or at.tp.size != 1
+                    or (at.nh, at.nkv, at.hd) != heads or getattr(view, "packed", False)):
+                return None
+            w = (at.qkv_weight(), at.wo.weight, mlp.gate_up_weight(), mlp.w_down.weight, layer.mlp_norm.weight,
+                 None if nxt is None else nxt.weight)
+            shapes = ((qn + 2 * kvn, d), (d, qn), (2 * f, d), (d, f), (d,), (d,))
+            for p, shape in zip(w, shapes):
+                if p is not None and (p.shape != shape or p.dtype != dt or p.device != dev or not p.is_contiguous()):
+                    return None
+            weights.append(w)
+        h = ops.add_rmsnorm(x, first.attn_norm.weight, first.attn_norm.eps)
+        blocks = []
+        for layer, view, nxt, w in zip(layers, kv, norms, weights):
+            layout, tables, slots, visible = view.prepare(b, t, heads[1], heads[2], dt, dev, pos32)
+            blocks.append((*w[:5], layer.mlp_norm.eps, w[5], 0.0 if nxt is None else nxt.eps,
+                           (layout, tables, slots, visible.contiguous()), getattr(view, "plan_key", None)))
+        out = ops.run_blocks(x, h, b, t, heads, f, pos32, rope[0], rope[1], blocks, last_norm is not None)
+        for view in kv:
+            view.commit(t)
+        return out
 
     def _run_verify_reusing(self, n_shared: int, window: torch.Tensor, pos32: torch.Tensor, kv: List,
                             keff: torch.Tensor, hidden: torch.Tensor, head_stats=None):

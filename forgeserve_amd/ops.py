@@ -5,6 +5,7 @@ allocator, and launches on torch's current stream. Inputs must already be on the
 computes on the CPU.
 """
 
+import math
 from typing import Optional, Tuple
 
 import torch
@@ -425,6 +426,54 @@ def paged_attention_varlen(q: torch.Tensor, layout: KVLayout, tables: torch.Tens
              ptr(cu_seqlens.contiguous()), s, t, h, float(scale), ptr(out), out.stride(0), out.stride(1), ptr(ws),
              ws.numel(), stream_ptr()), "paged_attention_varlen")
     return out
+
+
+# ------------------------------------------------------------------------------------------------
+# decoder blocks
+# ------------------------------------------------------------------------------------------------
+def run_blocks(x: torch.Tensor, h: torch.Tensor, b: int, t: int, heads: tuple, ffn: int, positions: torch.Tensor,
+               rope_cos: torch.Tensor, rope_sin: torch.Tensor, blocks: list, normed: bool):
+    """Decoder blocks launched by one call (fs_run_blocks): x (B*T, d) and h = the first block's attention norm of
+    x, both contiguous; heads: (query heads, KV heads, head_dim). blocks: per block (w_qkv, w_o, w_gate_up, w_down, mlp norm weight, its eps, next norm
+    weight or None, its eps, (layout, tables, slots, visible positions), plan key), tensors of x's dtype and
+    device with contiguous rows (the caller has checked them). Returns (x, next norm of x or None)."""
+    lib = _lib.load()
+    m, d = x.shape
+    n_heads, nkv, hd = heads
+    dt, dev = _dt(x), x.device
+    arr = (_lib.Block * len(blocks))()
+    sizes = set()
+    for e, (wq, wo, wgu, wd, n1, e1, n2, e2, (lay, tab, slots, vis), key) in zip(arr, blocks):
+        if (lay.n_kv_heads, lay.head_dim, lay.dtype) != (nkv, hd, dt):
+            raise ValueError("run_blocks: the cache's heads, head_dim or dtype are not the model's")
+        if (tab.dtype != I32 or vis.dtype != I32 or vis.shape != (b, t) or not vis.is_contiguous()
+                or (slots is not None and (slots.dtype != I32 or slots.numel() != m))):
+            raise ValueError("run_blocks: tables, slots and positions (B, T) must be int32")
+        require_device(tab, vis, slots)
+        e.w_qkv, e.w_o, e.w_gate_up, e.w_down = wq.data_ptr(), wo.data_ptr(), wgu.data_ptr(), wd.data_ptr()
+        e.mlp_norm, e.next_norm = n1.data_ptr(), ptr(n2)
+        e.kv, e.tables, e.table_stride, e.max_blocks = lay, tab.data_ptr(), tab.stride(0), tab.shape[1]
+        e.slots, e.visible, e.mlp_eps, e.next_eps = ptr(slots), vis.data_ptr(), e1, e2
+        e.reuse_plan = _reuse_plan(key, vis)
+        sizes.add((tab.shape[1], lay.block_size))
+    need = (_lib.c_i64 * 3)()
+    attn = 0
+    for nb, bs in sizes:
+        check(lib.fs_run_blocks_workspace(b, t, n_heads, nkv, hd, d, ffn, dt, nb, bs, need), "run_blocks_workspace")
+        attn = max(attn, need[1])
+    gws = _persistent_ws("gemm", need[0], dev) if need[0] > 0 else None
+    aws = _persistent_ws("attention", attn, dev)
+    scratch = _ws(need[2], dev)
+    x_out = torch.empty((m, d), dtype=x.dtype, device=dev)
+    y = torch.empty((m, d), dtype=x.dtype, device=dev) if normed else None
+    rc = lib.fs_run_blocks(arr, len(blocks), b, t, n_heads, d, ffn, dt, positions.data_ptr(), rope_cos.data_ptr(),
+                           rope_sin.data_ptr(), rope_cos.shape[0], 1.0 / math.sqrt(hd), x.data_ptr(), h.data_ptr(),
+                           x_out.data_ptr(), ptr(y), ptr(gws), 0 if gws is None else gws.numel(), aws.data_ptr(),
+                           aws.numel(), scratch.data_ptr(), scratch.numel(), stream_ptr())
+    if rc != 0:
+        _PLAN_KEY[0] = _PLAN_KEY[1] = None   # the attention of some block may not have run
+        check(rc, "run_blocks")
+    return x_out, y
 
 
 # ------------------------------------------------------------------------------------------------

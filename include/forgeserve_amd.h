@@ -259,6 +259,43 @@ int fs_gemm_swiglu(const void* A, int64_t lda, const void* B, int64_t ldb, void*
 int fs_embedding(const int64_t* ids, int64_t M, const void* weight, int64_t d_model, int64_t vocab,
                  void* out, int64_t ldo, int32_t dtype, void* stream);
 
+/* One decoder block of fs_run_blocks: its weights (contiguous rows, the dtype of the run; w_qkv holds wq, wk and
+ * wv one below the other, w_gate_up the gate then the up projection), the norm after the attention, the
+ * norm that the block's output goes through next (NULL: none; the last block only), its cache layer with
+ * the table to write and attend through, the pool slots to write (NULL: through the table) and the
+ * positions up to which each query sees (int32 (B, T)); reuse_plan: as fs_paged_attention_reuse_plan. */
+typedef struct fs_block {
+  const void* w_qkv;
+  const void* w_o;
+  const void* w_gate_up;
+  const void* w_down;
+  const void* mlp_norm;
+  const void* next_norm;
+  fs_kv_layout kv;
+  const int32_t* tables;
+  int64_t table_stride;
+  const int32_t* slots;
+  const int32_t* visible;
+  float mlp_eps, next_eps;
+  int32_t max_blocks, reuse_plan;
+} fs_block;
+
+/* Blocks blocks[0..n_blocks-1] on the residual stream x (B*T rows of d_model, contiguous) whose first norm is h:
+ * x_out the stream behind the last block, y_out its next_norm (unused when that is NULL). Every step is the
+ * entry point that computes it alone, chosen as a caller would (partials into the norm and rotary
+ * kernels where the projection splits K), with the same results (model.py:99-106, 136). All blocks have
+ * blocks[0]'s n_kv_heads and head_dim. The three buffers (256-byte aligned) hold the bytes that
+ * fs_run_blocks_workspace gives for the largest max_blocks: bytes[0] gemm_ws, bytes[1] attn_ws,
+ * bytes[2] scratch. */
+int fs_run_blocks_workspace(int32_t B, int32_t T, int32_t n_heads, int32_t n_kv_heads, int32_t head_dim,
+                            int64_t d_model, int64_t ffn, int32_t dtype, int32_t max_blocks, int32_t block_size,
+                            int64_t* bytes);
+int fs_run_blocks(const fs_block* blocks, int32_t n_blocks, int32_t B, int32_t T, int32_t n_heads, int64_t d_model,
+                  int64_t ffn, int32_t dtype, const int32_t* positions, const float* rope_cos, const float* rope_sin,
+                  int32_t rope_len, float scale, const void* x, const void* h, void* x_out, void* y_out,
+                  void* gemm_ws, int64_t gemm_ws_bytes, void* attn_ws, int64_t attn_ws_bytes, void* scratch,
+                  int64_t scratch_bytes, void* stream);
+
 /* ---------------------------------------------------------------------------------------------- */
 /* Sampling and acceptance                                                                          */
 /* ---------------------------------------------------------------------------------------------- */

@@ -243,6 +243,68 @@ def test_bf16_batch_perfect_draft_accepts_everything(bf_target):
     assert got == [fa.generate(bf_target, torch.tensor([p]), 25)[0].tolist()[len(p):] for p in prompts]
 
 
+@pytest.mark.parametrize("dtype,d,heads,kv_heads,ffn,b,t", [
+    (torch.bfloat16, 2048, 32, 8, 5632, 3, 1), (torch.bfloat16, 256, 4, 2, 704, 2, 5), (torch.bfloat16, 96, 3, 1, 200, 4, 3),
+    (torch.bfloat16, 512, 8, 8, 1376, 1, 300), (torch.float32, 64, 8, 4, 100, 3, 7), (torch.float16, 128, 4, 2, 256, 2, 2)])
+def test_blocks_in_one_call_equal_block_steps_bitwise(dtype, d, heads, kv_heads, ffn, b, t):
+    """The native run of the blocks against Block.step block by block, over both caches: projections that split
+    K and that do not, fused and separate SwiGLU, prefill and decode; logits and caches bit for bit. A block
+    that is not plain, and a view that serves two blocks, go block by block."""
+    case("blocks in one call", dtype, d, heads, kv_heads, ffn, b, t)
+    cfg = fa.ModelConfig(vocab_size=96, d_model=d, n_layers=3, n_heads=heads, n_kv_heads=kv_heads, ffn_dim=ffn,
+                         max_seq_len=1024)
+    torch.manual_seed(d + t)
+    model = fa.ForgeModel(cfg).to("cuda", dtype)
+    native = model._run_blocks
+    runs = []
+
+    def counted(*a):
+        runs.append(native(*a))
+        return runs[-1]
+
+    def both(f):
+        out = []
+        for fn in (counted, lambda *a: None):
+            model._run_blocks = fn
+            out.append(f())
+        model._run_blocks = counted
+        return out
+
+    g = torch.Generator().manual_seed(1)
+    idx, one = torch.randint(0, 96, (b, t), generator=g), torch.randint(0, 96, (b, 2), generator=g)
+
+    def contiguous():
+        kv = fa.new_contiguous_cache(3)
+        return [model(idx, kv=kv), model(one, kv=kv), *(c.k for c in kv), *(c.v for c in kv)]
+
+    def paged():
+        pool = fa.PagedKVPool(cfg, b * 24, 16, dtype=dtype, device="cuda")
+        pool.k_store.zero_(), pool.v_store.zero_()
+        tables = torch.arange(b * 24).reshape(b, 24).flip(0)
+        pos = torch.arange(t).expand(b, t)
+        outs = [model(idx, pos, pool.views(tables, pos))]
+        pos = torch.arange(t, t + 2).expand(b, 2)
+        return outs + [model(one, pos, pool.views(tables, pos)), pool.k_store, pool.v_store]
+
+    for f in (contiguous, paged):
+        for got, want in zip(*both(f)):
+            assert torch.equal(got, want)
+    assert len(runs) == 4 and all(r is not None for r in runs)
+    with torch.no_grad():
+        x = torch.randn(b * t, d, device="cuda").to(dtype)
+        pos = torch.arange(t, dtype=torch.int32, device="cuda").expand(b, t).contiguous()
+        part = both(lambda: model._layers(x, 1, 3, b, t, pos, [None] + fa.new_contiguous_cache(2)))
+        assert torch.equal(part[0][0], part[1][0]) and part[0][1] is None and part[1][1] is None
+        shared = fa.new_contiguous_cache(1) * 3
+        assert native(x, model.layers, b, t, pos, shared, model._rope(), model.norm) is None
+
+    class Other(type(model.layers[1])):
+        pass
+
+    model.layers[1].__class__ = Other
+    assert native(x, model.layers, b, t, pos, fa.new_contiguous_cache(3), model._rope(), model.norm) is None
+
+
 @pytest.mark.parametrize("which", ["bf16", "f32"])
 def test_packed_prefill_equals_per_sequence_prefill(which, bf_target, small):
     """Several prompts prefilled in one packed forward (no padding rows) leave the pool holding exactly
