@@ -933,8 +933,11 @@ attn_unit_part_kernel(AttnParams P) {
 // pair by pair it issued 360. Prompts of 4096, 1228, 1817, 1837 and 817 tokens (32/8 heads, 128 dims):
 // 494 -> 437 us; raising the waves' priority around the products changes it by 1%.
 constexpr int PF_WAVES = 8;      // query tiles (waves) per workgroup
-constexpr int PF_TILES = 4;      // 16-key tiles per ring stage
-constexpr int PF_NS = 4;         // ring stages (two in flight behind the one awaited)
+// 16-key tiles per ring stage, and stages (PF_NS - 2 in flight behind the one awaited). Two long stages rather than four
+// of half their length: half the barriers, each of which puts the eight waves in step again (prompts of 817-4096
+// tokens 395 -> 390 us, four of 2048 246 -> 242; three short stages: 428).
+constexpr int PF_TILES = 8;
+constexpr int PF_NS = 2;
 constexpr int PF_MIN_QTILES = 5; // a call with at least this many query tiles per row takes this kernel
 
 #pragma clang diagnostic push
@@ -981,7 +984,7 @@ attn_prefill_kernel(AttnParams P) {
   constexpr int CPR = D / 8;                        // 16-byte chunks per key row
   constexpr int STAGE = PF_TILES * TB;
   static_assert(PF_WAVES % CPT == 0 && CPW >= 1, "every wave copies the same part of its tiles");
-  static_assert(PF_NS == 4, "the waits below cover two stages in flight behind the awaited one");
+  static_assert(PF_NS >= 2 && PF_NS <= 4, "the waits below cover two stages in flight behind the awaited one");
   __shared__ __attribute__((aligned(1024))) char ring[PF_NS * STAGE];
   __shared__ int tbl[MAX_SPLIT / 16 + 1];           // the chunk's physical blocks (-1: unmapped)
 
@@ -1169,7 +1172,7 @@ attn_prefill_kernel(AttnParams P) {
     // the stage's operand addresses, once per stage: each tile's reads add only its constant offset
     const uint32_t st_lds = ring0 + (uint32_t)((k % PF_NS) * STAGE);
     const uint32_t vad = st_lds + (uint32_t)voff;
-#pragma unroll
+#pragma unroll 2
     for (int u = 0; u < PF_TILES; u += 2) {
       if (k * (PF_TILES / 2) + u / 2 >= npairs) break;
       const int pair = next;
