@@ -218,7 +218,7 @@ FS_DEVICE void merge_rows_wave(const Stat (&st)[R], bool in, int nch, Stat (&out
 // The same for one row whose chunk statistics the calling wave reads itself. (One thread walking the chunks,
 // a load at a time, took as long as the 8192 columns it was for.)
 FS_DEVICE Stat merge_row_wave(const Stat* st, int nch) {
-  if (nch > 64) return merge_row(st, nch);
+  if (nch == 1 || nch > 64) return merge_row(st, nch);   // (one chunk: nothing to reduce across lanes)
   const int lane = threadIdx.x & 63;
   Stat in[1] = {Stat{-INFINITY, 0.f, -INFINITY, 0x7fffffff}}, out[1];
   if (lane < nch) in[0] = st[lane];
