@@ -524,14 +524,15 @@ __device__ __attribute__((always_inline)) inline void attn_wave_tiles(const Attn
   const int BS = BSZ ? BSZ : P.kv.block_size;
   const int64_t v_dim = BSZ ? BSZ : P.kv.v_dim;   // == block_size (dim-major values)
 
-  // lane i: where the tiles of the wave's pair i start in the pool, in 16-byte units from the head's base (an
-  // unmapped block reads block 0 and is masked, a second tile that the chunk lacks reads the first), and
+  // lane i: where the tiles of the wave's pair i start in the pool, in bytes from the head's base (64 bits: the
+  // block stride is the caller's, and a pool that keeps every layer of a block together spans more than 64 GiB;
+  // an unmapped block reads block 0 and is masked, a second tile that the chunk lacks reads the first), and
   // which of them are there
   typedef uint16_t u16;
   const u16* kpool = reinterpret_cast<const u16*>(P.kv.k) + (int64_t)hkv * P.kv.k_head;
   const u16* vpool = reinterpret_cast<const u16*>(P.kv.v) + (int64_t)hkv * P.kv.v_head;
   const int64_t k_slot = P.kv.k_slot;
-  uint32_t k_at[2], v_at[2];
+  uint64_t k_at[2], v_at[2];
   uint64_t mapped[2];
   bool all_mapped = true;
   {
@@ -552,8 +553,8 @@ __device__ __attribute__((always_inline)) inline void attn_wave_tiles(const Attn
       mapped[u] = __ballot(ok);
       all_mapped &= mapped[u] == __ballot(exists[u]);
       const int64_t pb = ok ? phys[u] : 0;
-      k_at[u] = (uint32_t)((pb * P.kv.k_block + slot0[u] * k_slot) >> 3);
-      v_at[u] = (uint32_t)((pb * P.kv.v_block + slot0[u]) >> 3);
+      k_at[u] = (uint64_t)(2 * (pb * P.kv.k_block + slot0[u] * k_slot));
+      v_at[u] = (uint64_t)(2 * (pb * P.kv.v_block + slot0[u]));
     }
     if (!exists[1]) {
       k_at[1] = k_at[0];
@@ -598,9 +599,10 @@ __device__ __attribute__((always_inline)) inline void attn_wave_tiles(const Attn
   for (int ks = 0; ks < KS; ++ks) k_lane[ks] = (uint32_t)(2 * (l16 * k_slot + (g + 4 * ks) * kgs));
   const uint32_t v_lane = (uint32_t)(2 * (l16 * v_dim + 4 * g));
   // where a tile of the wave's pair i starts (a wave without pairs reads block 0 and consumes nothing)
-  auto tile_at = [&](const u16* pool, uint32_t at, int i) {
-    const int a = __builtin_amdgcn_readlane((int)at, max(min(i, np_w - 1), 0));
-    uint64_t t = reinterpret_cast<uint64_t>(pool) + ((uint64_t)(uint32_t)a << 4);
+  auto tile_at = [&](const u16* pool, uint64_t at, int i) {
+    const int l = max(min(i, np_w - 1), 0);
+    const uint32_t lo = __builtin_amdgcn_readlane((int)at, l), hi = __builtin_amdgcn_readlane((int)(at >> 32), l);
+    uint64_t t = reinterpret_cast<uint64_t>(pool) + ((uint64_t)hi << 32 | lo);
     asm("" : "+s"(t));   // a scalar base and 32-bit lane offsets: no 64-bit vector adds per load
     return (__attribute__((address_space(1))) const char*)t;
   };

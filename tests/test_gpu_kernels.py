@@ -669,6 +669,34 @@ def test_attention_tile_pairs(d, t, g, bs, layout):
     assert torch.equal(run(qd, 0.0), run(torch.zeros_like(qd), 1.0 / math.sqrt(d)))
 
 
+@pytest.mark.parametrize("d,bs,layout", [(128, 16, "groups"), (64, 48, "slots")])
+def test_attention_pool_of_more_than_64_gib(d, bs, layout):
+    """A pool whose blocks lie 13 GiB apart, the last one beyond 64 GiB (as a pool that keeps every layer of a block
+    together may): every attention kernel gives the bits that it gives for the same blocks in a compact pool."""
+    case("attention pool of more than 64 GiB", d, bs, layout)
+    gib, nblocks, hkv, g = 1 << 30, 6, 2, 4
+    if torch.cuda.mem_get_info()[0] < 80 * gib:
+        pytest.skip("needs 65 GiB of device memory")
+    gen = torch.Generator().manual_seed(d)
+    k = torch.randn(nblocks, hkv, bs, d, generator=gen).bfloat16()
+    v = torch.randn(nblocks, hkv, bs, d, generator=gen).bfloat16()
+    tables = torch.randint(0, nblocks, (140, 48 * 64 // bs), generator=gen)
+    tables[:, 0] = nblocks - 1
+    _, near = _run_attention(torch.zeros(1, 1, hkv * g, d).bfloat16(), k, v, tables[:1], torch.zeros(1, 1), torch.bfloat16,
+                             bs, layout)
+    store = torch.empty(65 * gib + (1 << 20), dtype=torch.uint8, device=DEV).view(torch.bfloat16)
+    apart = 13 * gib // 2
+    far = lambda t, at: store.as_strided(t.shape, (apart, *t.stride()[1:]), at)
+    kf, vf = far(near.k[0], 0), far(near.v[0], 1 << 18)
+    kf.copy_(near.k[0]), vf.copy_(near.v[0])
+    tab = tables.int().to(DEV)
+    for rows, t in ((140, 1), (64, 5), (8, 1), (8, 5), (2, 300)):   # whole units, in two and four parts, a prompt
+        q = torch.randn(rows, t, hkv * g, d, generator=gen).bfloat16().to(DEV)
+        pos = (torch.randint(t, tables.shape[1] * bs + 1, (rows, 1), generator=gen) - t + torch.arange(t)).int().to(DEV)
+        run = lambda lay: ops.paged_attention(q, lay, tab[:rows], pos, d ** -0.5)
+        assert torch.equal(run(ops.kv_layout(kf, vf)), run(near.layout(0))), (rows, t)
+
+
 def test_attention_prefill_plan_of_many_groups():
     """A prefill plan of more groups of query rows than it has threads (33 rows x 32 groups), most of them
     padding, positions not in order inside a row: each row's bits the same as alone, padding zeros."""
