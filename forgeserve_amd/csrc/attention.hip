@@ -1540,10 +1540,10 @@ __global__ void __launch_bounds__(64 * COMBINE_ROWS) attn_combine_kernel(AttnPar
 #pragma unroll
       for (int jj = 0; jj < 8; ++jj) {
         if (j + jj < n) {
-          const float wj = __builtin_amdgcn_readlane(__float_as_int(w), j + jj);
+          const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j + jj));
           L += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lw), j + jj));
 #pragma unroll
-          for (int c = 0; c < 4; ++c) acc[c] += __int_as_float(wj) * v[jj][c];
+          for (int c = 0; c < 4; ++c) acc[c] += wj * v[jj][c];
         }
       }
     }

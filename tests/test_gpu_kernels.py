@@ -471,6 +471,37 @@ def test_attention_f32_tiles(d, bs, t, g, layout):
         torch.testing.assert_close(got[4, :-1], out[4, :-1], atol=2e-6, rtol=2e-5)
 
 
+@pytest.mark.parametrize("d", [32, 30])   # the matrix-core kernel, the scalar one
+def test_attention_f32_merges_chunks(d):
+    """The merge of a query's two 512-key chunks: one key a chunk has weight (the others' underflow to 0), with scores
+    0 and -x, 0 < x < ln 2, which are exact, and values 1 and -1, so every chunk is exactly (m, 1, its value) and
+    the output is (1 - w) / (1 + w) with w = e^-x. Against float64: w's error is 2^-24 for the exponential, and
+    ln 2 times the rounding of x log2 e < 1 and of log2 e itself (2^-25 + 2^-24), under 1.3e-7 in all, the
+    output's 2 / (1 + w)^2 <= 0.9 times that and three roundings of 2^-24: under 3e-7."""
+    case("attention f32 chunks merge", d)
+    g = torch.Generator().manual_seed(d)
+    b, bs = 256, 16
+    nb = 2 * 512 // bs
+    x = torch.randint(1, 2839, (b,), generator=g) / 4096.0
+    first = torch.randint(0, 2, (b, 1), generator=g)   # which chunk holds the larger score
+    at = torch.randint(0, 512, (b, 2), generator=g) + torch.tensor([0, 512])
+    score = torch.where(torch.arange(2) == first, 0.0, -x[:, None])
+    k, v = torch.zeros(b * nb, 1, bs, d), torch.zeros(b * nb, 1, bs, d)
+    k[..., 0] = -300.0
+    rows = torch.arange(b)[:, None]
+    k.view(b, nb * bs, d)[rows, at, 0] = score
+    v.view(b, nb * bs, d)[rows, at] = torch.where(score == 0, 1.0, -1.0)[:, :, None].expand(b, 2, d)
+    q = torch.zeros(b, 1, 1, d)
+    q[..., 0] = 1.0
+    tables = torch.arange(b * nb).reshape(b, nb)
+    _, pool = _run_attention(q, k, v, tables, torch.zeros(b, 1), torch.float32, bs)
+    pos = torch.full((b, 1), nb * bs - 1, dtype=torch.int32, device=DEV)
+    got = ops.paged_attention(q.to(DEV), pool.layout(0), tables.int().to(DEV), pos, 1.0)[:, 0, 0].cpu()
+    w = torch.exp(-x.double())
+    err = (got.double() - ((1 - w) / (1 + w))[:, None]).abs().max().item()
+    assert err < 3e-7
+
+
 @pytest.mark.parametrize("d,t,g", [(128, 5, 4), (128, 7, 4), (64, 5, 4), (128, 1, 4), (128, 9, 4), (64, 3, 8)])
 def test_attention_mfma_bf16(d, t, g):
     case("attention bf16 mfma", d, t, g)
