@@ -702,27 +702,47 @@ __device__ __attribute__((always_inline)) inline void attn_wave_tiles(const Attn
   }
 }
 
-// Row `rr` of the query rows (token rr / G, head hkv*G + rr % G), dims 16*mt + 4g .. +4, from its
-// folded chunk-s state (M, L, O): a query that sees one chunk only is finished here (a padding query,
+// Row `rr` of the query rows (token rr / G, head hkv*G + rr % G), dims 16*(mt + i) + 4g .. +4 for i < N, from its
+// folded chunk-s state (M, L, o): a query that sees one chunk only is finished here (a padding query,
 // position < 0, gets zeros from chunk 0); any other query gets this chunk's partial for attn_combine
 // if the chunk holds keys it sees.
-template <int D>
+template <int D, int N>
 FS_DEVICE void attn_emit(const AttnParams& P, int b, int s, int kbeg, int hkv, int rr, int rp, int mt, float M,
-                         float L, const float4_t& o) {
+                         float L, const float4_t (&o)[N]) {
   const int lane = threadIdx.x & 63, g = lane >> 4;
   const bool direct = P.direct && (rp < P.split || P.nsplit == 1);
   if (direct ? s != 0 : rp < kbeg) return;
   const int t = rr / P.G, h = hkv * P.G + (rr - t * P.G);
-  if (direct) {   // the same normalisation as attn_combine's
+  if (direct) {
     if (!token_exists(P, b, t)) return;
-    const float inv = L > 0.f ? 1.f / L : 0.f;
-    const float f[4] = {o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv};
+    // o / L, rounded to bf16. o times L's reciprocal, which the row's outputs share, is within 2 ulps of it, and rounds
+    // to the same bf16 unless a tie is that near: then the wave divides (one time in thirty for N = 1, in nine for
+    // 4). Prompts of 817-4096 tokens: every output divided 402 us, products with N = 1 397, with N = 4 362.
+    const float inv = 1.f / L;
+    float f[N][4];
+    uint16_t near = 0xffff;   // the products' smallest distance above four ulps below a tie
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        f[i][c] = o[i][c] * inv;
+        near = min(near, (uint16_t)((uint16_t)__float_as_uint(f[i][c]) - 0x7ffc));
+      }
+    if (__any(near <= 8 || !(L > 0.f))) {
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) f[i][c] = L > 0.f ? o[i][c] / L : 0.f;
+    }
     uint16_t* orow = reinterpret_cast<uint16_t*>(P.out) + o_offset(P, b, t, P.o_sb, P.o_st) + (int64_t)h * P.o_sh;
-    *reinterpret_cast<short4_t*>(orow + 16 * mt + 4 * g) = bf16_rne4(f);
+#pragma unroll
+    for (int i = 0; i < N; ++i) *reinterpret_cast<short4_t*>(orow + 16 * (mt + i) + 4 * g) = bf16_rne4(f[i]);
     return;
   }
   const int64_t R = row_index(P, b, t, h);
-  *reinterpret_cast<float4_t*>(P.ws_acc + (R * P.nsplit + s) * D + 16 * mt + 4 * g) = o;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    *reinterpret_cast<float4_t*>(P.ws_acc + (R * P.nsplit + s) * D + 16 * (mt + i) + 4 * g) = o[i];
   if (mt == 0 && g == 0) {
     float* pm = P.ws_ml + (R * P.nsplit + s) * 2;
     pm[0] = M;
@@ -778,7 +798,7 @@ attn_unit_kernel(AttnParams P) {
       for (int c = 0; c < 4; ++c) o[c] = fold_value(o[c], cM, a[c], cm);
       M = Mn;
     }
-    attn_emit<D>(P, b, s, kbeg, hkv, row0 + r, rpos[nt], mt, M, L, o);
+    attn_emit<D, 1>(P, b, s, kbeg, hkv, row0 + r, rpos[nt], mt, M, L, {o});
   }
 }
 
@@ -913,7 +933,7 @@ attn_unit_part_kernel(AttnParams P) {
       for (int c = 0; c < 4; ++c) o[c] = fold_value(o[c], cM, a[v][c], cm);
       M = Mn;
     }
-    if (r < nrows) attn_emit<D>(P, b, s, kbeg, hkv, row0 + r, nt ? rpos[1] : rpos[0], mt, M, L, o);
+    if (r < nrows) attn_emit<D, 1>(P, b, s, kbeg, hkv, row0 + r, nt ? rpos[1] : rpos[0], mt, M, L, {o});
   }
 }
 
@@ -1216,7 +1236,9 @@ attn_prefill_kernel(AttnParams P) {
     const int r = 16 * nt + l16;
     if (r >= nrows) continue;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) attn_emit<D>(P, b, s, kbeg, hkv, row0 + r, rpos[nt], mt, Ms[nt], Ls[nt], O[mt][nt]);
+    for (int mt = 0; mt < MT; mt += 4)
+      attn_emit<D, 4>(P, b, s, kbeg, hkv, row0 + r, rpos[nt], mt, Ms[nt], Ls[nt],
+                      {O[mt][nt], O[mt + 1][nt], O[mt + 2][nt], O[mt + 3][nt]});
   }
 }
 
@@ -1551,8 +1573,7 @@ __global__ void __launch_bounds__(64 * COMBINE_ROWS) attn_combine_kernel(AttnPar
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     const int d = lane + 64 * c;
-    // (16-bit outputs: one division per row, as attn_emit has it)
-    if (d < D) E::store(orow, d, DT == FS_F32 ? (L > 0.f ? acc[c] / L : 0.f) : acc[c] * (L > 0.f ? 1.f / L : 0.f));
+    if (d < D) E::store(orow, d, L > 0.f ? acc[c] / L : 0.f);
   }
 }
 

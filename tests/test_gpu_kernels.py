@@ -728,6 +728,32 @@ def test_attention_pool_of_more_than_64_gib(d, bs, layout):
         assert torch.equal(run(ops.kv_layout(kf, vf)), run(near.layout(0))), (rows, t)
 
 
+@pytest.mark.parametrize("dtype,d,bs,t,lens", [
+    (torch.bfloat16, 128, 16, 1, range(2, 1200, 8)),   # whole units
+    (torch.bfloat16, 64, 32, 1, range(2, 1200, 200)), (torch.bfloat16, 128, 16, 5, range(1000, 3600, 400)),   # parts
+    (torch.bfloat16, 64, 16, 300, range(302, 700, 90)),   # a prompt
+    (torch.bfloat16, 128, 16, 1, [16386, 20002, 32770]), (torch.float16, 32, 16, 1, range(2, 1400, 50))])   # merged chunks
+def test_attention_outputs_are_quotients_rounded_once(dtype, d, bs, t, lens):
+    """Equal scores, so that the weights are 1 and their sum is the number of keys, and values of which one half is
+    2 - 2u and one half 2 - u in some dims (u the type's last place at 1), 2 - 3u and 2 - 2u in the others: the
+    outputs' sums are exact and their means ties that go to 2 - 2u. A quotient that is off by one float32
+    rounding goes to 2 - u in the former or to 2 - 3u in the latter."""
+    case("attention quotients", dtype, d, bs, t, lens)
+    lens, hkv, g = list(lens), 2, 4
+    u = torch.finfo(dtype).eps
+    nb = -(-max(lens) // bs)
+    v = torch.full((nb, hkv, bs, d), 2 - 2 * u)
+    v[:, :, 1::2, ::2] += u
+    v[:, :, 1::2, 1::2] -= u
+    tables = torch.arange(nb).expand(len(lens), nb)
+    q, k = torch.zeros(len(lens), t, hkv * g, d).to(dtype), torch.ones(nb, hkv, bs, d).to(dtype)
+    last = torch.tensor(lens)[:, None] - 1
+    pos = (last - 2 * torch.arange(t)).clamp_min(1)   # an even number of keys each
+    out, _ = _run_attention(q, k, v.to(dtype), tables, pos, dtype, bs)
+    wrong = (out != 2 - 2 * u).sum().item()
+    assert wrong == 0
+
+
 def test_attention_prefill_plan_of_many_groups():
     """A prefill plan of more groups of query rows than it has threads (33 rows x 32 groups), most of them
     padding, positions not in order inside a row: each row's bits the same as alone, padding zeros."""
