@@ -71,15 +71,17 @@ template <> struct Elem<FS_F16> {
 // ------------------------------------------------------------------------------------------------
 // silu(g) * u as SwiGLU computes it (model.py:93): silu rounded to the dtype, then the product, which the
 // caller rounds when it stores it; g and u are dtype values. Every kernel that forms this product calls
-// this one function, so their results agree bit for bit. For the 16-bit types the exponential and the
-// reciprocal are the hardware's (float32, 5e-6 relative where e^-g is largest, against the dtype's 2^-9 or
-// 2^-12): expf and a correctly rounded division are ~45 instructions an element, 6% of a long gate|up
-// product (8005 x 28672 x 4096: 1.58 -> 1.49 ms).
+// this one function, so their results agree bit for bit. For bf16 the exponential and the reciprocal are the
+// hardware's: expf and a division are ~45 instructions an element, 3% of a long gate|up product (8005 x 28672 x
+// 4096: 1.56 -> 1.51 ms; 7373 x 16384 x 2048: 481 -> 448 us). Each of the 65,280 finite g rounds to the bf16 that expf and the division give: the
+// results differ by at most 58 float32 ulps, and no g with a tie that near falls on its other side. The factor
+// 3/32, exact on g, keeps the reciprocal a normal number up to e^-g = 2^128, and its rounding leaves
+// silu(5.9375), 1.2 ulps from a tie, on the right side (1/16 does not).
 template <int DT>
 FS_DEVICE float silu_times(float g, float u) {
-  if (DT == FS_F32) return g / (1.0f + expf(-g)) * u;
+  if (DT != FS_BF16) return Elem<DT>::round(g / (1.0f + expf(-g))) * u;
   const float e = __builtin_amdgcn_exp2f(g * -1.4426950408889634f);
-  return Elem<DT>::round(g * __builtin_amdgcn_rcpf(1.0f + e)) * u;
+  return Elem<DT>::round((g * 0.09375f) * __builtin_amdgcn_rcpf(fmaf(e, 0.09375f, 0.09375f))) * u;
 }
 
 FS_DEVICE float wave_max(float v) {

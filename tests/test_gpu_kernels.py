@@ -257,6 +257,31 @@ def test_silu_mul(dtype):
         assert ((h.float() - ref.float()).abs() <= ref.float().abs() * 2 ** -7 * 1.01 + 1e-30).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_silu_of_every_16_bit_value(dtype):
+    """silu of each finite g >= -88 of the type (below, e^-g leaves float32), times 1: the float64 value rounded once,
+    give or take 8 float32 roundings, through both elementwise kernels and, in bf16, the gated
+    projections' short and long tiles (one-hot rows, so that g is the weight itself)."""
+    case("silu of every value", dtype)
+    g = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(dtype)
+    g = torch.where(g.isfinite() & (g >= -88), g, torch.zeros_like(g))
+    ref = g.double() * torch.sigmoid(g.double())
+    fi = torch.finfo(dtype)
+    ulp = (2.0 ** torch.floor(torch.log2(ref.abs().clamp_min(fi.tiny)))) * fi.eps
+    bound = ulp * (0.5 + 8 * 2.0 ** -24 / fi.eps)
+    gu = torch.cat([g.view(64, 1024), torch.ones(64, 1024, dtype=dtype)], 1).to(DEV)
+    h = ops.silu_mul(gu)
+    assert ((h.cpu().view(-1).double() - ref).abs() <= bound).all()
+    odd = torch.cat([gu[:, :1023], gu[:, 1024:2047]], 1).contiguous()   # rows of no whole 16 bytes
+    assert torch.equal(ops.silu_mul(odd), h[:, :1023])
+    if dtype == torch.bfloat16:
+        w = torch.ones(6148, 64, dtype=dtype, device=DEV)   # 3074 gate rows, then 3074 up rows
+        w[:1024], w[1024:2048], w[2048:3072] = (gu[:, :1024].T,) * 3
+        for m in (64, 128, 448, 2304):
+            a = torch.eye(64, dtype=dtype, device=DEV).repeat(36, 1)[:m]
+            assert torch.equal(ops.gemm_swiglu(a, w)[:, :3072], h.repeat(36, 3)[:m]), m
+
+
 def test_rmsnorm_and_silu_general_paths_bf16():
     """The row kernels' general paths (rows that are not whole 16-byte groups) against the reference,
     and silu_mul's two paths bit for bit (the same per-element arithmetic)."""
