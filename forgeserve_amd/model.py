@@ -159,6 +159,16 @@ class Block(nn.Module):
         return ops.gemm_add_rmsnorm(g, self.mlp.w_down.weight, x1, next_norm.weight, next_norm.eps, x_out=x_out)
 
 
+_STEP, _ATTEND = Block.step, Attention.attend
+
+
+def _plain_block(layer) -> bool:
+    """Whether layer computes what this module's Block does: not another class, nor one whose step or
+    attend a caller has replaced, on the object or on the class (a timing or tracing wrapper)."""
+    return (type(layer) is Block and type(layer.attn) is Attention and type(layer.mlp) is SwiGLU
+            and getattr(layer.step, "__func__", None) is _STEP and getattr(layer.attn.attend, "__func__", None) is _ATTEND)
+
+
 class ForgeModel(nn.Module):
     """Embedding and head are shared (tied), as in model.py:109-159."""
 
@@ -297,6 +307,8 @@ class ForgeModel(nn.Module):
         if (not x.is_contiguous() or b * t == 0 or pos32 is None or pos32.dtype != torch.int32 or pos32.device != dev
                 or not pos32.is_contiguous() or len({id(view) for view in kv}) != len(kv)):
             return None
+        if not all(_plain_block(layer) for layer in layers):
+            return None
         first = layers[0]
         d, f, heads = x.shape[1], first.mlp.w_down.weight.shape[1], (first.attn.nh, first.attn.nkv, first.attn.hd)
         qn, kvn = heads[0] * heads[2], heads[1] * heads[2]
@@ -304,8 +316,7 @@ class ForgeModel(nn.Module):
         weights = []
         for layer, view, nxt in zip(layers, kv, norms):
             at, mlp = layer.attn, layer.mlp
-            if (type(layer) is not Block or type(at) is not Attention or type(mlp) is not SwiGLU or at.tp.size != 1
-                    or (at.nh, at.nkv, at.hd) != heads or getattr(view, "packed", False)):
+            if at.tp.size != 1 or (at.nh, at.nkv, at.hd) != heads or getattr(view, "packed", False):
                 return None
             w = (at.qkv_weight(), at.wo.weight, mlp.gate_up_weight(), mlp.w_down.weight, layer.mlp_norm.weight,
                  None if nxt is None else nxt.weight)

@@ -138,3 +138,66 @@ def test_captures_run_without_the_garbage_collector():
         assert not gc.isenabled()
     finally:
         gc.enable()
+
+
+def _block_model(n_layers):
+    import torch
+
+    from forgeserve_amd import ForgeModel
+
+    cfg = ModelConfig(vocab_size=8, d_model=32, n_layers=n_layers, n_heads=4, n_kv_heads=2, ffn_dim=64, max_seq_len=16)
+    model = ForgeModel(cfg)
+    return model, torch.zeros(2, 32), torch.zeros(2, 1, dtype=torch.int32)
+
+
+@pytest.mark.parametrize("at", [0, 1])
+def test_blocks_of_another_kind_run_through_their_step(at, monkeypatch):
+    """A block of another class, without the attributes of Block, and a step or attend that a caller has replaced
+    on the object or on the class: every block then runs through its step, in order."""
+    import torch
+
+    from forgeserve_amd.model import Attention, Block, ForgeModel
+
+    class Foreign(torch.nn.Module):
+        def step(self, *a, **kw):
+            return "foreign"
+
+    ran = []
+
+    def run(model, x, pos):
+        views = [object() for _ in model.layers]
+        native = model._run_blocks(x, model.layers, 2, 1, pos, views, model._rope(), model.norm)
+        assert native is None
+        del ran[:]
+        model._layers(x, 0, len(model.layers), 2, 1, pos, views, last_norm=model.norm)
+        return list(ran)
+
+    def step_of(name):
+        def step(x, *a, **kw):
+            ran.append(name)
+            return x, x
+        return step
+
+    model, x, pos = _block_model(3)
+    for i, layer in enumerate(model.layers):
+        object.__setattr__(layer, "step", step_of(i))   # no GPU here: every step is a stand-in
+    assert run(model, x, pos) == [0, 1, 2]
+    foreign = Foreign()
+    foreign.attn_norm = torch.nn.Identity()
+    object.__setattr__(foreign, "step", step_of("foreign"))
+    model.layers[at] = foreign
+    assert run(model, x, pos) == [*range(at), "foreign", *range(at + 1, 3)]
+
+    views = [object(), object()]
+    for owner, name in ((Block, "step"), (Attention, "attend")):
+        model, x, pos = _block_model(2)
+        target = model.layers[at] if owner is Block else model.layers[at].attn
+        old = getattr(target, name)
+        setattr(target, name, lambda *a, **kw: old(*a, **kw))
+        assert ForgeModel._run_blocks(x, model.layers, 2, 1, pos, views, model._rope(), model.norm) is None
+        delattr(target, name)
+        with monkeypatch.context() as m:
+            m.setattr(owner, name, lambda self, *a, **kw: None)
+            assert ForgeModel._run_blocks(x, model.layers, 2, 1, pos, views, model._rope(), model.norm) is None
+        with pytest.raises(RuntimeError):   # plain blocks go to the native call, which needs a GPU
+            ForgeModel._run_blocks(x, model.layers, 2, 1, pos, views, model._rope(), model.norm)
