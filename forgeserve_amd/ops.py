@@ -358,17 +358,21 @@ def paged_gather(layout: KVLayout, tables: torch.Tensor, dtype, device) -> Tuple
     return k_all, v_all
 
 
-# The plan key and positions tensor of the last paged-attention call (held, so that no later object
-# can share their identities).
+# The plan key and positions tensor of the last paged-attention call that went through (held, so that no later
+# object can share their identities).
 _PLAN_KEY = [None, None]
 
 
 def _reuse_plan(plan_key, positions: torch.Tensor) -> bool:
     """True when the previous paged-attention call carried the same plan key and the same positions
     tensor (the layers of one step)."""
-    reuse = plan_key is not None and _PLAN_KEY[0] is plan_key and _PLAN_KEY[1] is positions
-    _PLAN_KEY[0], _PLAN_KEY[1] = plan_key, positions
-    return reuse
+    return plan_key is not None and _PLAN_KEY[0] is plan_key and _PLAN_KEY[1] is positions
+
+
+def _attended(rc: int, what: str, plan_key, positions: torch.Tensor) -> None:
+    """check(rc) of a call that attends, whose plan the next call may reuse only if it went through."""
+    _PLAN_KEY[0], _PLAN_KEY[1] = (plan_key, positions) if rc == 0 else (None, None)
+    check(rc, what)
 
 
 def paged_attention(q: torch.Tensor, layout: KVLayout, tables: torch.Tensor, positions: torch.Tensor,
@@ -392,9 +396,9 @@ def paged_attention(q: torch.Tensor, layout: KVLayout, tables: torch.Tensor, pos
     need = lib.fs_paged_attention_workspace_size(b, t, h, d, nb, layout.block_size)
     ws = _persistent_ws("attention", need, q.device)
     fn = lib.fs_paged_attention_reuse_plan if _reuse_plan(plan_key, positions) else lib.fs_paged_attention
-    check(fn(ptr(q), q.stride(0), q.stride(1), q.stride(2), layout, ptr(tables), tables.stride(0), nb, ptr(positions),
-             b, t, h, float(scale), ptr(out), out.stride(0), out.stride(1), out.stride(2), ptr(ws), ws.numel(),
-             stream_ptr()), "paged_attention")
+    _attended(fn(ptr(q), q.stride(0), q.stride(1), q.stride(2), layout, ptr(tables), tables.stride(0), nb, ptr(positions),
+                 b, t, h, float(scale), ptr(out), out.stride(0), out.stride(1), out.stride(2), ptr(ws), ws.numel(),
+                 stream_ptr()), "paged_attention", plan_key, positions)
     return out
 
 
@@ -422,9 +426,9 @@ def paged_attention_varlen(q: torch.Tensor, layout: KVLayout, tables: torch.Tens
     ws = _persistent_ws("attention", lib.fs_paged_attention_workspace_size(s, t, h, d, nb, layout.block_size), q.device)
     fn = (lib.fs_paged_attention_varlen_reuse_plan if _reuse_plan(plan_key, positions)
           else lib.fs_paged_attention_varlen)
-    check(fn(ptr(q), q.stride(0), q.stride(1), layout, ptr(tables), tables.stride(0), nb, ptr(positions),
-             ptr(cu_seqlens.contiguous()), s, t, h, float(scale), ptr(out), out.stride(0), out.stride(1), ptr(ws),
-             ws.numel(), stream_ptr()), "paged_attention_varlen")
+    _attended(fn(ptr(q), q.stride(0), q.stride(1), layout, ptr(tables), tables.stride(0), nb, ptr(positions),
+                 ptr(cu_seqlens.contiguous()), s, t, h, float(scale), ptr(out), out.stride(0), out.stride(1), ptr(ws),
+                 ws.numel(), stream_ptr()), "paged_attention_varlen", plan_key, positions)
     return out
 
 
@@ -443,7 +447,7 @@ def run_blocks(x: torch.Tensor, h: torch.Tensor, b: int, t: int, heads: tuple, f
     dt, dev = _dt(x), x.device
     arr = (_lib.Block * len(blocks))()
     sizes = set()
-    for e, (wq, wo, wgu, wd, n1, e1, n2, e2, (lay, tab, slots, vis), key) in zip(arr, blocks):
+    for e, (wq, wo, wgu, wd, n1, e1, n2, e2, (lay, tab, slots, vis), _) in zip(arr, blocks):
         if (lay.n_kv_heads, lay.head_dim, lay.dtype) != (nkv, hd, dt):
             raise ValueError("run_blocks: the cache's heads, head_dim or dtype are not the model's")
         if (tab.dtype != I32 or vis.dtype != I32 or vis.shape != (b, t) or not vis.is_contiguous()
@@ -454,7 +458,6 @@ def run_blocks(x: torch.Tensor, h: torch.Tensor, b: int, t: int, heads: tuple, f
         e.mlp_norm, e.next_norm = n1.data_ptr(), ptr(n2)
         e.kv, e.tables, e.table_stride, e.max_blocks = lay, tab.data_ptr(), tab.stride(0), tab.shape[1]
         e.slots, e.visible, e.mlp_eps, e.next_eps = ptr(slots), vis.data_ptr(), e1, e2
-        e.reuse_plan = _reuse_plan(key, vis)
         sizes.add((tab.shape[1], lay.block_size))
     need = (_lib.c_i64 * 3)()
     attn = 0
@@ -466,13 +469,16 @@ def run_blocks(x: torch.Tensor, h: torch.Tensor, b: int, t: int, heads: tuple, f
     scratch = _ws(need[2], dev)
     x_out = torch.empty((m, d), dtype=x.dtype, device=dev)
     y = torch.empty((m, d), dtype=x.dtype, device=dev) if normed else None
+    before = _PLAN_KEY
+    for e, blk in zip(arr, blocks):   # a block reuses the plan of the one before it: same step, same positions
+        key, vis = blk[9], blk[8][3]
+        e.reuse_plan = key is not None and before[0] is key and before[1] is vis
+        before = key, vis
     rc = lib.fs_run_blocks(arr, len(blocks), b, t, n_heads, d, ffn, dt, positions.data_ptr(), rope_cos.data_ptr(),
                            rope_sin.data_ptr(), rope_cos.shape[0], 1.0 / math.sqrt(hd), x.data_ptr(), h.data_ptr(),
                            x_out.data_ptr(), ptr(y), ptr(gws), 0 if gws is None else gws.numel(), aws.data_ptr(),
                            aws.numel(), scratch.data_ptr(), scratch.numel(), stream_ptr())
-    if rc != 0:
-        _PLAN_KEY[0] = _PLAN_KEY[1] = None   # the attention of some block may not have run
-        check(rc, "run_blocks")
+    _attended(rc, "run_blocks", *before)
     return x_out, y
 
 

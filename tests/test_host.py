@@ -201,3 +201,49 @@ def test_blocks_of_another_kind_run_through_their_step(at, monkeypatch):
             assert ForgeModel._run_blocks(x, model.layers, 2, 1, pos, views, model._rope(), model.norm) is None
         with pytest.raises(RuntimeError):   # plain blocks go to the native call, which needs a GPU
             ForgeModel._run_blocks(x, model.layers, 2, 1, pos, views, model._rope(), model.norm)
+
+
+def test_a_failed_attention_call_leaves_no_plan_to_reuse(monkeypatch):
+    """A call that is refused, by its own checks, for want of memory or by the library, never stands as the one
+    whose work plan the next call of the same step reuses; and an earlier one is forgotten only when the
+    library has seen the failed call."""
+    import os
+
+    import torch
+
+    from forgeserve_amd import ops
+    from forgeserve_amd.build import LIB
+
+    if not os.path.exists(LIB):
+        pytest.skip("library not built (python -m forgeserve_amd.build)")
+    monkeypatch.setattr(ops, "require_device", lambda *a: None)
+    monkeypatch.setattr(ops, "stream_ptr", lambda *a: 0)
+    monkeypatch.setattr(ops, "_PERSISTENT", {})
+    monkeypatch.setattr(ops, "_PLAN_KEY", [None, None])
+    key, earlier = object(), object()
+    pos, tables = torch.zeros(2, 1, dtype=torch.int32), torch.zeros(2, 1, dtype=torch.int32)
+    pool = torch.zeros(2, 2, 16, 8)
+    lay = ops.kv_layout(pool, pool)
+
+    def refused(f, error):
+        ops._PLAN_KEY[:] = earlier, pos
+        with pytest.raises(error):
+            f()
+        assert ops._PLAN_KEY[0] is not key
+        return ops._PLAN_KEY[0]
+
+    # three query heads over two KV heads: the library refuses them
+    three = lambda f, q, *a: refused(lambda: f(q, lay, tables, pos, *a, 1.0, plan_key=key), ValueError)
+    assert three(ops.paged_attention, torch.zeros(2, 1, 3, 8)) is None
+    assert three(ops.paged_attention_varlen, torch.zeros(2, 3, 8), torch.tensor([0, 1, 2], dtype=torch.int32)) is None
+
+    x, w = torch.zeros(2, 32), torch.zeros(64, 32)
+    block = lambda tab: (w, w, w, w, x[0], 1e-5, x[0], 1e-5, (lay, tab, None, pos), key)
+    run = lambda blocks: ops.run_blocks(x, x, 2, 1, (4, 2, 8), 32, pos, x, x, blocks, True)
+    assert refused(lambda: run([block(tables), block(tables.long())]), ValueError) is earlier
+
+    def full(*a):
+        raise torch.OutOfMemoryError("none left")
+
+    monkeypatch.setattr(ops, "_ws", full)
+    assert refused(lambda: run([block(tables)]), torch.OutOfMemoryError) is earlier
