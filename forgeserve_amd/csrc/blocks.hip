@@ -104,10 +104,15 @@ extern "C" int fs_run_blocks(const fs_block* blocks, int32_t n_blocks, int32_t B
   Shape s;
   FS_CHECK_ARG(make_shape(s, B, T, n_heads, blocks[0].kv.n_kv_heads, blocks[0].kv.head_dim, d_model, ffn, dtype),
                "run_blocks: shapes");
-  for (int32_t i = 0; i < n_blocks; ++i)
-    FS_CHECK_ARG(blocks[i].kv.n_kv_heads == blocks[0].kv.n_kv_heads && blocks[i].kv.head_dim == s.hd &&
-                     blocks[i].kv.dtype == dtype && (blocks[i].next_norm != nullptr || i == n_blocks - 1),
-                 "run_blocks: block %d", (int)i);
+  FS_CHECK_ARG(positions && rope_cos && rope_sin && attn_ws, "run_blocks: null pointer");
+  for (int32_t i = 0; i < n_blocks; ++i) {   // all of them before the first launch writes to a cache
+    const fs_block& b = blocks[i];
+    FS_CHECK_ARG(b.kv.n_kv_heads == blocks[0].kv.n_kv_heads && b.kv.head_dim == s.hd && b.kv.dtype == dtype,
+                 "run_blocks: block %d: its cache's heads, head_dim or dtype", (int)i);
+    FS_CHECK_ARG(b.w_qkv && b.w_o && b.w_gate_up && b.w_down && b.mlp_norm && b.kv.k && b.kv.v && b.tables && b.visible &&
+                     (b.next_norm || i == n_blocks - 1),
+                 "run_blocks: block %d: null pointer", (int)i);
+  }
   FS_CHECK_ARG(blocks[n_blocks - 1].next_norm == nullptr || y_out, "run_blocks: null y_out");
   const Scratch sc(reinterpret_cast<char*>(scratch), s);
   FS_CHECK_ARG(scratch_bytes >= sc.bytes, "run_blocks: scratch %lld < %lld bytes", (long long)scratch_bytes,

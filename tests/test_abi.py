@@ -84,3 +84,19 @@ def test_workspace_sizes_are_positive(lib):
     assert lib.fs_gemm_serial(32768, 28672, 4096, 1) == 0   # not split
     assert lib.fs_gemm_serial(32768, 4096, 14336, 1) == 0   # 3584-k splits keep their partials
     assert lib.fs_gemm_serial(4096, 4096, 4096, 0) == 0 and lib.fs_gemm_serial(0, 4096, 4096, 1) == 0
+
+
+@pytest.mark.parametrize("field", ["w_qkv", "w_o", "w_gate_up", "w_down", "mlp_norm", "next_norm", "tables", "visible", "k"])
+def test_run_blocks_refuses_a_missing_pointer_before_it_launches(lib, field):
+    """The first of two blocks without one of its tensors (a block's second norm among them: only the last block
+    may lack the norm behind it)."""
+    blocks = (_lib.Block * 2)()
+    for b in blocks:
+        for name in ("w_qkv", "w_o", "w_gate_up", "w_down", "mlp_norm", "next_norm", "tables", "visible"):
+            setattr(b, name, 256)
+        b.kv = _lib.KVLayout(256, 256, 256, 128, 8, 1, 256, 128, 1, 16, 16, 2, 8, 0, 4, 0)
+        b.table_stride = b.max_blocks = 1
+    setattr(blocks[0].kv if field == "k" else blocks[0], field, None)
+    rc = lib.fs_run_blocks(blocks, 2, 1, 1, 4, 32, 64, 0, 256, 256, 256, 16, 1.0, 256, 256, 256, 256, 256, 1 << 20, 256,
+                           1 << 30, 256, 1 << 20, None)
+    assert rc == -1 and b"block 0" in lib.fs_last_error()
