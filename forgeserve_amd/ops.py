@@ -436,11 +436,13 @@ def paged_attention_varlen(q: torch.Tensor, layout: KVLayout, tables: torch.Tens
 # decoder blocks
 # ------------------------------------------------------------------------------------------------
 def run_blocks(x: torch.Tensor, h: torch.Tensor, b: int, t: int, heads: tuple, ffn: int, positions: torch.Tensor,
-               rope_cos: torch.Tensor, rope_sin: torch.Tensor, blocks: list, normed: bool):
+               rope_cos: torch.Tensor, rope_sin: torch.Tensor, blocks: list, normed: bool, buffers: dict):
     """Decoder blocks launched by one call (fs_run_blocks): x (B*T, d) and h = the first block's attention norm of
-    x, both contiguous; heads: (query heads, KV heads, head_dim). blocks: per block (w_qkv, w_o, w_gate_up, w_down, mlp norm weight, its eps, next norm
-    weight or None, its eps, (layout, tables, slots, visible positions), plan key), tensors of x's dtype and
-    device with contiguous rows (the caller has checked them). Returns (x, next norm of x or None)."""
+    x, both contiguous; heads: (query heads, KV heads, head_dim). blocks: per block (w_qkv, w_o, w_gate_up,
+    w_down, mlp norm weight, its eps, next norm weight or None, its eps, (layout, tables, slots, visible
+    positions), plan key), tensors of x's dtype and device with contiguous rows (the caller has checked them).
+    buffers: an empty dict, the same for the calls of one forward, which share their workspaces and scratch
+    through it. Returns (x, next norm of x or None)."""
     lib = _lib.load()
     m, d = x.shape
     n_heads, nkv, hd = heads
@@ -459,14 +461,15 @@ def run_blocks(x: torch.Tensor, h: torch.Tensor, b: int, t: int, heads: tuple, f
         e.kv, e.tables, e.table_stride, e.max_blocks = lay, tab.data_ptr(), tab.stride(0), tab.shape[1]
         e.slots, e.visible, e.mlp_eps, e.next_eps = ptr(slots), vis.data_ptr(), e1, e2
         sizes.add((tab.shape[1], lay.block_size))
-    need = (_lib.c_i64 * 3)()
-    attn = 0
-    for nb, bs in sizes:
-        check(lib.fs_run_blocks_workspace(b, t, n_heads, nkv, hd, d, ffn, dt, nb, bs, need), "run_blocks_workspace")
-        attn = max(attn, need[1])
-    gws = _persistent_ws("gemm", need[0], dev) if need[0] > 0 else None
-    aws = _persistent_ws("attention", attn, dev)
-    scratch = _ws(need[2], dev)
+    shape = (heads, ffn, frozenset(sizes))
+    if shape not in buffers:
+        need, attn = (_lib.c_i64 * 3)(), 0
+        for nb, bs in sizes:
+            check(lib.fs_run_blocks_workspace(b, t, n_heads, nkv, hd, d, ffn, dt, nb, bs, need), "run_blocks_workspace")
+            attn = max(attn, need[1])
+        buffers[shape] = (_persistent_ws("gemm", need[0], dev) if need[0] > 0 else None,
+                          _persistent_ws("attention", attn, dev), _ws(need[2], dev))
+    gws, aws, scratch = buffers[shape]
     x_out = torch.empty((m, d), dtype=x.dtype, device=dev)
     y = torch.empty((m, d), dtype=x.dtype, device=dev) if normed else None
     before = _PLAN_KEY

@@ -305,6 +305,38 @@ def test_blocks_in_one_call_equal_block_steps_bitwise(dtype, d, heads, kv_heads,
     assert native(x, model.layers, b, t, pos, fa.new_contiguous_cache(3), model._rope(), model.norm) is None
 
 
+@pytest.mark.parametrize("dtype,d,b,t", [(torch.bfloat16, 2048, 3, 1), (torch.float32, 64, 2, 5)])
+def test_deep_runs_of_blocks_equal_block_steps_bitwise(dtype, d, b, t):
+    """Ten blocks, which native runs of one, two, four and three take: logits and caches bit for bit those of
+    Block.step block by block, over both caches, also where a caller has wrapped the step of a block in the middle
+    (its step is called, and the blocks around it run natively)."""
+    case("deep runs of blocks", dtype, d, b, t)
+    cfg = fa.ModelConfig(vocab_size=96, d_model=d, n_layers=10, n_heads=8, n_kv_heads=4, ffn_dim=2 * d, max_seq_len=128)
+    torch.manual_seed(d)
+    model = fa.ForgeModel(cfg).to("cuda", dtype)
+    g = torch.Generator().manual_seed(2)
+    idx, one = torch.randint(0, 96, (b, t), generator=g), torch.randint(0, 96, (b, 1), generator=g)
+
+    def outputs():
+        kv = fa.new_contiguous_cache(10)
+        out = [model(idx, kv=kv), model(one, kv=kv), *(c.k for c in kv), *(c.v for c in kv)]
+        pool = fa.PagedKVPool(cfg, b * 4, 16, dtype=dtype, device="cuda")
+        tables = torch.arange(b * 4).reshape(b, 4).flip(0)
+        for toks, pos in ((idx, torch.arange(t).expand(b, t)), (one, torch.full((b, 1), t))):
+            out.append(model(toks, pos, pool.views(tables, pos)))
+        return out + [pool.k_store, pool.v_store]
+
+    native = outputs()
+    seen = []
+    step = model.layers[4].step
+    model.layers[4].step = lambda *a, **kw: seen.append(1) or step(*a, **kw)
+    wrapped = outputs()
+    assert len(seen) == 4
+    model._run_blocks = lambda *a: None
+    for x, y, z in zip(outputs(), native, wrapped):
+        assert torch.equal(x, y) and torch.equal(x, z)
+
+
 @pytest.mark.parametrize("which", ["bf16", "f32"])
 def test_packed_prefill_equals_per_sequence_prefill(which, bf_target, small):
     """Several prompts prefilled in one packed forward (no padding rows) leave the pool holding exactly

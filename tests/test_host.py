@@ -140,67 +140,116 @@ def test_captures_run_without_the_garbage_collector():
         gc.enable()
 
 
-def _block_model(n_layers):
+def _stand_ins(monkeypatch, ran):
+    """Native runs of blocks, norms and the two methods of Block and Attention that note what they were asked for
+    (there is no GPU here)."""
+    from forgeserve_amd import model as mod, ops
+
+    def run_blocks(x, h, b, t, heads, ffn, positions, rope_cos, rope_sin, blocks, normed, buffers):
+        ran.append(("run", len(blocks), normed))
+        return x, x if normed else None
+
+    monkeypatch.setattr(ops, "add_rmsnorm", lambda x, *a, **kw: x)
+    monkeypatch.setattr(ops, "run_blocks", run_blocks)
+
+    def step(self, x, *a, **kw):
+        ran.append(("step",))
+        return x, x
+
+    monkeypatch.setattr(mod.Block, "step", step)
+    monkeypatch.setattr(mod, "_STEP", step)
+
+
+def _block_model(n_layers, log):
     import torch
 
     from forgeserve_amd import ForgeModel
 
+    class View:
+        def __init__(self, i, log):
+            self.i, self.log = i, log
+
+        def prepare(self, b, t, h, d, dtype, device, positions):
+            self.log.append(("prepare", self.i))
+            return None, None, None, positions
+
+        def commit(self, t):
+            self.log.append(("commit", self.i))
+
     cfg = ModelConfig(vocab_size=8, d_model=32, n_layers=n_layers, n_heads=4, n_kv_heads=2, ffn_dim=64, max_seq_len=16)
+    x, pos = torch.zeros(2, 32), torch.zeros(2, 1, dtype=torch.int32)
     model = ForgeModel(cfg)
-    return model, torch.zeros(2, 32), torch.zeros(2, 1, dtype=torch.int32)
+    views = [View(i, log) for i in range(n_layers)]
+    return model, lambda: model._layers(x, 0, n_layers, 2, 1, pos, views, last_norm=model.norm)
 
 
-@pytest.mark.parametrize("at", [0, 1])
+@pytest.mark.parametrize("at", [0, 1, 2])
 def test_blocks_of_another_kind_run_through_their_step(at, monkeypatch):
-    """A block of another class, without the attributes of Block, and a step or attend that a caller has replaced
-    on the object or on the class: every block then runs through its step, in order."""
+    """A layer of another class, without the attributes of Block: every layer runs through its step. A step or attend
+    that a caller has replaced on one object, or on the class, is called."""
     import torch
 
-    from forgeserve_amd.model import Attention, Block, ForgeModel
-
-    class Foreign(torch.nn.Module):
-        def step(self, *a, **kw):
-            return "foreign"
+    from forgeserve_amd import model as mod
 
     ran = []
+    _stand_ins(monkeypatch, ran)
 
-    def run(model, x, pos):
-        views = [object() for _ in model.layers]
-        native = model._run_blocks(x, model.layers, 2, 1, pos, views, model._rope(), model.norm)
-        assert native is None
-        del ran[:]
-        model._layers(x, 0, len(model.layers), 2, 1, pos, views, last_norm=model.norm)
-        return list(ran)
+    class Foreign(torch.nn.Module):
+        attn_norm = torch.nn.Identity()
 
-    def step_of(name):
-        def step(x, *a, **kw):
-            ran.append(name)
+        def step(self, x, *a, **kw):
+            ran.append(("foreign",))
             return x, x
-        return step
 
-    model, x, pos = _block_model(3)
-    for i, layer in enumerate(model.layers):
-        object.__setattr__(layer, "step", step_of(i))   # no GPU here: every step is a stand-in
-    assert run(model, x, pos) == [0, 1, 2]
-    foreign = Foreign()
-    foreign.attn_norm = torch.nn.Identity()
-    object.__setattr__(foreign, "step", step_of("foreign"))
-    model.layers[at] = foreign
-    assert run(model, x, pos) == [*range(at), "foreign", *range(at + 1, 3)]
+    launches = lambda: [e for e in ran if e[0] not in ("prepare", "commit")]
+    model, run = _block_model(3, ran)
+    model.layers[at] = Foreign()
+    run()
+    assert launches() == [("foreign",) if i == at else ("step",) for i in range(3)]
 
-    views = [object(), object()]
-    for owner, name in ((Block, "step"), (Attention, "attend")):
-        model, x, pos = _block_model(2)
-        target = model.layers[at] if owner is Block else model.layers[at].attn
-        old = getattr(target, name)
-        setattr(target, name, lambda *a, **kw: old(*a, **kw))
-        assert ForgeModel._run_blocks(x, model.layers, 2, 1, pos, views, model._rope(), model.norm) is None
-        delattr(target, name)
+    del ran[:]
+    model, run = _block_model(3, ran)   # a step that leaves the norm to the next block
+    model.layers[at].step = lambda x, *a, **kw: ran.append(("wrapped",)) or (x, None)
+    run()
+    assert launches() == [("run", 1, True)] * at + [("wrapped",)] + [("step",)] * (2 - at)
+
+    del ran[:]
+    model, run = _block_model(3, ran)
+    model.layers[at].attn.attend = lambda *a, **kw: None
+    run()
+    assert [e[0] for e in launches()].count("step") == (1 if at else 3)   # (the stand-in step does not attend)
+
+    for owner, name in ((mod.Block, "step"), (mod.Attention, "attend")):
         with monkeypatch.context() as m:
-            m.setattr(owner, name, lambda self, *a, **kw: None)
-            assert ForgeModel._run_blocks(x, model.layers, 2, 1, pos, views, model._rope(), model.norm) is None
-        with pytest.raises(RuntimeError):   # plain blocks go to the native call, which needs a GPU
-            ForgeModel._run_blocks(x, model.layers, 2, 1, pos, views, model._rope(), model.norm)
+            del ran[:]
+            model, run = _block_model(3, ran)
+            m.setattr(owner, name, lambda self, x, *a, **kw: ran.append(("class",)) or (x, x))
+            run()
+            assert launches() == [("class",) if name == "step" else ("step",)] * 3
+
+
+def test_the_first_block_is_launched_before_the_others_are_prepared(monkeypatch):
+    """A native run takes one block, then two, four and so on (a last one of one goes with those before it), each
+    prepared after the run before it is launched, and committed with its run; a block whose weights are of another dtype takes its step in its place."""
+    import torch
+
+    log = []
+    _stand_ins(monkeypatch, log)
+    for n, runs in ((2, (1, 1)), (4, (1, 3)), (16, (1, 2, 4, 9)), (20, (1, 2, 4, 8, 5))):
+        del log[:]
+        _block_model(n, log)[1]()
+        want, i = [], 0
+        for k in runs:
+            ids = range(i, i + k)
+            want += [("prepare", j) for j in ids] + [("run", k, True)] + [("commit", j) for j in ids]
+            i += k
+        assert log == want
+
+    del log[:]
+    model, run = _block_model(4, log)
+    model.layers[2].attn.wo.weight.data = model.layers[2].attn.wo.weight.data.to(torch.bfloat16)
+    run()
+    assert [e for e in log if e[0] in ("run", "step")] == [("run", 1, True), ("run", 1, True), ("step",), ("run", 1, True)]
 
 
 def test_a_failed_attention_call_leaves_no_plan_to_reuse(monkeypatch):
@@ -239,7 +288,7 @@ def test_a_failed_attention_call_leaves_no_plan_to_reuse(monkeypatch):
 
     x, w = torch.zeros(2, 32), torch.zeros(64, 32)
     block = lambda tab: (w, w, w, w, x[0], 1e-5, x[0], 1e-5, (lay, tab, None, pos), key)
-    run = lambda blocks: ops.run_blocks(x, x, 2, 1, (4, 2, 8), 32, pos, x, x, blocks, True)
+    run = lambda blocks: ops.run_blocks(x, x, 2, 1, (4, 2, 8), 32, pos, x, x, blocks, True, {})
     assert refused(lambda: run([block(tables), block(tables.long())]), ValueError) is earlier
 
     def full(*a):
