@@ -1202,6 +1202,31 @@ def test_sample_logits_corners(temperature, dtype):
         torch.testing.assert_close(p, orc.probs_from_logits(row.float(), max(temperature, 0.06)), atol=1e-7, rtol=2e-5)
 
 
+@pytest.mark.parametrize("temperature", [0.7, 0.06, 1.3, 1 / 3, 1.9999999, 2.0 ** -59, 3e17, 2.0 ** 61])
+def test_temperature_quotients_equal_the_division(temperature):
+    """y = x / T through T's reciprocal: the probabilities at T are bit for bit those at T = 1 of the quotients that
+    torch's division gives, for magnitudes from 2^-100 to where the quotients near 2^120 (where the kernel
+    divides), ragged vocabularies, and rows with masked columns."""
+    case("temperature quotients", temperature)
+    g = torch.Generator().manual_seed(6)
+    t = torch.tensor(temperature).item()
+    for v in (24576, 8192 * 2 + 5):
+        x = torch.randn(8, v, generator=g)
+        x[1] *= 12 * t                       # y near a softmax's range
+        x[2] *= 2.0 ** torch.randint(-100, 100, (v,), generator=g)
+        x[3] *= 2.0 ** 110 * min(t, 1.0)
+        x[4] = (x[4] * 4).bfloat16().float()
+        x[5] = t * (torch.randint(-2 ** 20, 2 ** 20, (v,), generator=g) / 2.0 ** 16)   # quotients near short numbers
+        x[6, ::3] = -math.inf
+        x[7] *= 3e-38
+        x = x.to(DEV)
+        got = ops.probs_from_logits(x, temperature)
+        want = ops.probs_from_logits(x / torch.tensor(temperature, dtype=torch.float32, device=DEV), 1.0)
+        for r in range(8):
+            same = (got[r] == want[r]) | (got[r].isnan() & want[r].isnan())
+            assert same.all(), (v, r)
+
+
 def test_probs_from_logits():
     case("probs_from_logits")
     x = torch.randn(5, 20000) * 4
