@@ -5,8 +5,9 @@
 // partials to the kernel that follows). The results are those of the separate calls, bit for bit.
 //
 // A short batch's kernels take 2-17 us each, and a Python caller needs 12 us per launch, so that decode steps waited
-// for the host. Launched from here: one token of 4 blocks (d = 2048, bf16) 440 -> 330 us, which are the kernels';
-// of 4 float32 blocks (d = 256) 520 -> 303; four rows of 160 tokens of those 707 -> 467.
+// for the host. Launched from here: 16 rows of one token through 4 blocks (d = 2048, bf16) 440 -> 330 us, which
+// are the kernels'; one row through 4 float32 blocks (d = 256) 520 -> 303; four rows of 160 tokens through
+// those 707 -> 467.
 #include "common.h"
 
 namespace {

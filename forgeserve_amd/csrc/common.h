@@ -73,10 +73,10 @@ template <> struct Elem<FS_F16> {
 // caller rounds when it stores it; g and u are dtype values. Every kernel that forms this product calls
 // this one function, so their results agree bit for bit. For bf16 the exponential and the reciprocal are the
 // hardware's: expf and a division are ~45 instructions an element, 3% of a long gate|up product (8005 x 28672 x
-// 4096: 1.56 -> 1.51 ms; 7373 x 16384 x 2048: 481 -> 448 us). Each of the 65,280 finite g rounds to the bf16 that expf and the division give: the
-// results differ by at most 58 float32 ulps, and no g with a tie that near falls on its other side. The factor
-// 3/32, exact on g, keeps the reciprocal a normal number up to e^-g = 2^128, and its rounding leaves
-// silu(5.9375), 1.2 ulps from a tie, on the right side (1/16 does not).
+// 4096: 1.56 -> 1.51 ms; 7373 x 16384 x 2048: 481 -> 448 us). Each of the 65,280 finite g rounds to the bf16
+// that expf and the division give: the results differ by at most 58 float32 ulps, and no g with a tie that near
+// falls on its other side. The factor 3/32, exact on g, keeps the reciprocal a normal number up to e^-g = 2^128,
+// and its rounding leaves silu(5.9375), 1.2 ulps from a tie, on the right side (1/16 does not).
 template <int DT>
 FS_DEVICE float silu_times(float g, float u) {
   if (DT != FS_BF16) return Elem<DT>::round(g / (1.0f + expf(-g))) * u;

@@ -288,8 +288,8 @@ class ForgeModel(nn.Module):
         (None: not normalised). x_out: where block stop-1 writes its output (then returned as x)."""
         rope = self._rope()
         if x_out is None and start < stop:
-            done = self._run_blocks(x, list(self.layers)[start: stop], b, t, pos32, [kv[i] for i in range(start, stop)], rope,
-                                    last_norm)
+            done = self._run_blocks(x, list(self.layers)[start: stop], b, t, pos32, [kv[i] for i in range(start, stop)],
+                                    rope, last_norm)
             if done is not None:
                 return done
         h = None

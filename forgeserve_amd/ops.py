@@ -371,8 +371,10 @@ def _reuse_plan(plan_key, positions: torch.Tensor) -> bool:
 
 def _attended(rc: int, what: str, plan_key, positions: torch.Tensor) -> None:
     """check(rc) of a call that attends, whose plan the next call may reuse only if it went through."""
-    _PLAN_KEY[0], _PLAN_KEY[1] = (plan_key, positions) if rc == 0 else (None, None)
-    check(rc, what)
+    if rc != 0:
+        _PLAN_KEY[0] = _PLAN_KEY[1] = None
+        check(rc, what)
+    _PLAN_KEY[0], _PLAN_KEY[1] = plan_key, positions
 
 
 def paged_attention(q: torch.Tensor, layout: KVLayout, tables: torch.Tensor, positions: torch.Tensor,
