@@ -69,6 +69,11 @@ template <> struct Elem<FS_F16> {
 // ------------------------------------------------------------------------------------------------
 // wavefront (64-lane) reductions
 // ------------------------------------------------------------------------------------------------
+// A row's softmax sum takes 2^(y log2 e - M log2 e) in one multiply-add while its maximum M is at most this: the
+// rounding of M log2 e then scales the sum by 1 + 3e-6 at most. Further out (a temperature near 0) that rounding
+// grows with M, to a factor of 2 at 10^7 and past float32's range at 10^9, so y - M is formed first.
+constexpr float STAT_FAR = 64.f;
+
 // silu(g) * u as SwiGLU computes it (model.py:93): silu rounded to the dtype, then the product, which the
 // caller rounds when it stores it; g and u are dtype values. Every kernel that forms this product calls
 // this one function, so their results agree bit for bit. For bf16 the exponential and the reciprocal are the

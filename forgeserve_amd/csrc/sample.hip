@@ -314,12 +314,19 @@ FS_DEVICE Stat chunk_stat(const typename Elem<DT>::T* row, int c, int64_t V, flo
 #pragma unroll
     for (int j = 0; j < 8; ++j) m = fmaxf(m, x[u][j]);
   const float M = block_max(m, shf);
-  const float ML = M * LOG2E_F;
   float sum = 0.f;
+  if (fabsf(M) <= STAT_FAR) {
+    const float ML = M * LOG2E_F;
 #pragma unroll
-  for (int u = 0; u < UNROLL; ++u)
+    for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) sum += __builtin_amdgcn_exp2f(fmaf(x[u][j], LOG2E_F, -ML));  // exp(-inf) = 0
+      for (int j = 0; j < 8; ++j) sum += __builtin_amdgcn_exp2f(fmaf(x[u][j], LOG2E_F, -ML));  // exp(-inf) = 0
+  } else {
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sum += __builtin_amdgcn_exp2f((x[u][j] - M) * LOG2E_F);
+  }
   st.m = M;
   st.s = block_sum(sum, shf);
   st.av = M;

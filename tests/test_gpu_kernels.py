@@ -1343,6 +1343,54 @@ def test_gemm_row_stats(m, n, k):
     assert ((fl[:, 1].double() - want).abs() / want).max() < 2e-6
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("temperature", [1e-2, 1e-3, 1e-5, 1e-6, 1e-8, 1e-20, 1e-30])
+def test_softmax_at_temperatures_near_zero(temperature, dtype):
+    """Quotients x / T of 10^3 to 10^31, many of them within a few units of the row's maximum: the probabilities
+    against float64 on the float32 quotients, and the draws against the oracle's. Tolerance: the
+    exponential, 1 / S, their product and the sum's own rounding, 10 float32 roundings."""
+    case("softmax near T = 0", temperature, dtype)
+    g = torch.Generator().manual_seed(9)
+    for v in (300, 8193, 20000):
+        x = 10 + temperature * torch.randn(6, v, generator=g) * 3
+        x[1] = torch.randn(v, generator=g) * 3
+        x[2] = -0.5                                  # every column ties
+        x[3, ::2] = -math.inf
+        x[4] = (torch.randn(v, generator=g) * 2).round()   # a few values, many ties
+        x = x.to(dtype)
+        y = x.float() / torch.tensor(temperature, dtype=torch.float32)
+        ref = y.double().softmax(-1)
+        got = ops.probs_from_logits(x.to(DEV), temperature).cpu().double()
+        assert ((got - ref).abs() <= ref * 10 * 2.0 ** -24 + 1e-37).all(), v
+        e = torch.empty(6, v).exponential_(generator=g)
+        draws = ops.sample_logits(x.to(DEV), temperature, e.to(DEV)).cpu().tolist()
+        assert draws == [orc.draw(orc.probs_from_logits(x[r].float(), temperature), e[r]) for r in range(6)], v
+
+
+@pytest.mark.parametrize("m", [64, 130])
+def test_gemm_row_stats_at_temperatures_near_zero(m):
+    """The head's statistics where y / T lies far from zero: against float64 on the float32 quotients of the stored
+    logits, with the tolerance of the other temperatures; a row's records do not depend on its neighbours'."""
+    case("gemm row stats near T = 0", m)
+    n, k = 32000, 256
+    g = torch.Generator().manual_seed(m)
+    a = (torch.randn(m, k, generator=g) * 0.5).bfloat16().to(DEV)
+    w = (torch.randn(n, k, generator=g) * 0.5).bfloat16().to(DEV)
+    w[1::2] = w[::2]   # every maximum ties
+    temps = torch.tensor([(1e-3, 0.7, 1e-5, 1e-7, 1.0, 1e-20)[r % 6] for r in range(m)])
+    nparts = ops.row_stats_parts(m, n, k)
+    parts = lambda t: (ops.gemm_row_stats(a, w, t.to(DEV), p := torch.empty((m, nparts, 4), dtype=torch.int32, device=DEV)), p)
+    out, p = parts(temps)
+    fl = ops.row_stats_merge(p, torch.empty((m, 4), dtype=torch.int32, device=DEV)).cpu().view(torch.float32)
+    y = out.cpu().float() / temps[:, None]
+    mx = y.max(-1).values
+    assert torch.equal(fl[:, 0], mx)
+    want = torch.exp((y - mx[:, None]).double()).sum(-1)
+    assert ((fl[:, 1].double() - want).abs() / want).max() < 2e-6
+    near = temps >= 0.7
+    assert torch.equal(parts(torch.where(near, temps, torch.ones(m)))[1][near.to(DEV)], p[near.to(DEV)])
+
+
 @pytest.mark.parametrize("temperature", [1.0, 0.7, 0.0])
 def test_spec_accept_with_row_stats_bit_exact(temperature):
     """fs_spec_accept_stats (statistics given, as the LM head emits them) against the oracle."""
