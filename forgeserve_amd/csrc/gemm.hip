@@ -417,20 +417,19 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_bf16_lds_kernel(const uin
         argmax_merge(av, ai, ov, oi);
       }
       const float ml = ym * L2E;
-      const bool far = !(fabsf(ym) <= STAT_FAR);   // the row's own; the branch is for the wave
-      const bool some_far = __any(far);
+      const bool far = !(fabsf(ym) <= STAT_FAR);   // the row's own; the branch is the wave's
       float se = 0.f;
+      auto sum = [&](auto exponent) {
 #pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int64_t col0 = n0 + wn * WN + 16 * j + 4 * g;
+        for (int j = 0; j < TN; ++j) {
+          const int64_t col0 = n0 + wn * WN + 16 * j + 4 * g;
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (col0 + r < N) {
-            float e = fmaf(acc[i][j][r], L2E, -ml);
-            if (some_far) e = far ? (acc[i][j][r] - ym) * L2E : e;
-            se += __builtin_amdgcn_exp2f(e);
-          }
-      }
+          for (int r = 0; r < 4; ++r)
+            if (col0 + r < N) se += __builtin_amdgcn_exp2f(exponent(acc[i][j][r]));
+        }
+      };
+      if (__any(far)) sum([&](float y) { return far ? (y - ym) * L2E : fmaf(y, L2E, -ml); });
+      else sum([&](float y) { return fmaf(y, L2E, -ml); });
       se += __shfl_xor(se, 16, 64);   // (g0 + g1) + (g2 + g3) in every lane
       se += __shfl_xor(se, 32, 64);
       if (g == 0 && row < M && p < rs.nparts) rs.stats[row * rs.ld + p] = SoftmaxStat{ym, ym == -INFINITY ? 0.f : se, av, ai};
