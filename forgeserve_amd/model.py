@@ -304,8 +304,9 @@ class ForgeModel(nn.Module):
     @staticmethod
     def _run_blocks(x, layers, b, t, pos32, kv, rope, last_norm):
         """_layers' blocks through native calls, which launch what Block.step launches with the choices it makes;
-        None (nothing done) where a layer is of another class, or a view serves two of them. A layer that is
-        not a plain block, or whose weights are not of x's dtype and device, takes its step, as does a packed view.
+        None (nothing done) where a layer is of another class, the first is not a plain block, or a view serves two
+        of them. A later layer that is not plain, or whose weights are not of x's dtype and device, takes its
+        step, as does a packed view.
         A call takes one block, then two, four and so on: the blocks of the next are prepared (10-20 us each) while
         the last one's compute, where preparing all of them first kept the GPU waiting (one decode step waited
         for, 8 rows and 32 blocks of the 8B shape: 5.05 -> 4.55 ms, block by block 4.52; 16 rows and 16 blocks
