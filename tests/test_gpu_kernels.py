@@ -259,9 +259,10 @@ def test_silu_mul(dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_silu_of_every_16_bit_value(dtype):
-    """silu of each finite g >= -88 of the type (below, e^-g leaves float32), times 1: the float64 value rounded once,
-    give or take 8 float32 roundings, through both elementwise kernels and, in bf16, the gated
-    projections' short and long tiles (one-hot rows, so that g is the weight itself)."""
+    """silu of each finite g of the type, times 1: the bits that the float32 kernel's result rounds to, and, from -88
+    on (below, e^-g leaves float32), the float64 value rounded once, give or take 8 float32 roundings; through
+    both elementwise kernels and, in bf16, the gated projections' short and long tiles (one-hot rows, so that g
+    is the weight itself)."""
     case("silu of every value", dtype)
     g = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(dtype)
     g = torch.where(g.isfinite() & (g >= -88), g, torch.zeros_like(g))
@@ -272,6 +273,10 @@ def test_silu_of_every_16_bit_value(dtype):
     gu = torch.cat([g.view(64, 1024), torch.ones(64, 1024, dtype=dtype)], 1).to(DEV)
     h = ops.silu_mul(gu)
     assert ((h.cpu().view(-1).double() - ref).abs() <= bound).all()
+    full = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(dtype).view(64, 1024)
+    full = torch.cat([torch.where(full.isfinite(), full, torch.zeros_like(full)), torch.ones_like(full)], 1).to(DEV)
+    got, f32 = ops.silu_mul(full), ops.silu_mul(full.float()).to(dtype)   # (float32: expf and a division)
+    assert torch.equal(got.view(torch.int16), f32.view(torch.int16))
     odd = torch.cat([gu[:, :1023], gu[:, 1024:2047]], 1).contiguous()   # rows of no whole 16 bytes
     assert torch.equal(ops.silu_mul(odd), h[:, :1023])
     if dtype == torch.bfloat16:
